@@ -21,7 +21,11 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "liblbfast_hip.so")
-SOURCES = ["lbf_fused.hip", "lbf_stages.hip", "lbf_api.cpp"]
+# translation units: (source, preprocessor switches).  The fused kernels are
+# compiled one storage precision to a unit (lbf_common.h Prec, | 8 with the
+# default 16-bit scales compiled in), so that the units build in parallel.
+SOURCES = [("lbf_fused.hip", [f"-DLBF_FUSED_PREC={p}"]) for p in (0, 1, 2, 3, 4, 11, 12)]
+SOURCES += [(s, []) for s in ("lbf_stages.hip", "lbf_fused.hip", "lbf_api.cpp")]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLANG = os.environ.get("FLANG", "/opt/rocm/bin/amdflang")
 FDIR = os.path.join(HERE, "fortran")
@@ -46,9 +50,10 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
          "-munsafe-fp-atomics", "-Wno-unused-result"]
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", "-x", "hip", os.path.join(CSRC, src), "-o", obj]
+def _compile(unit) -> str:
+    src, defs = unit
+    obj = os.path.join(BUILD, os.path.splitext(src)[0] + "".join(d.replace("-DLBF_FUSED_PREC=", "_p") for d in defs) + ".o")
+    cmd = [HIPCC, *FLAGS, *defs, "-c", "-x", "hip", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr[-6000:]}")

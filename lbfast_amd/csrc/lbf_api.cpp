@@ -40,6 +40,7 @@ struct lbf_ctx {
   void* pre = nullptr;  // 5-field set (fast path phase-field prep)
   void* sopen = nullptr;  // open faces: post-moments state of the fast path (10-field set)
   int8_t* isfh = nullptr;
+  uint32_t* words = nullptr;  // obstacles: the fused kernel's word per haloed node
   void* rep = nullptr;         // REPULSIVE_FLUX: locaux 3..8 (6-field set)
   int8_t* rep_mask = nullptr;  // REPULSIVE_FLUX
   float* raw = nullptr;  // 10-field FP32 staging of 16-bit storage uploads
@@ -83,7 +84,8 @@ static int fail(lbf_ctx* c, int code, const char* fmt, ...) {
 
 static void* dalloc(lbf_ctx* c, size_t bytes, hipError_t* e) {
   void* p = nullptr;
-  *e = hipMalloc(&p, bytes);
+  // the kernels' 16-byte row transfers may read past a set's last row
+  *e = hipMalloc(&p, bytes + 1024);
   if (*e == hipSuccess) c->allocs.push_back(p);
   return p;
 }
@@ -355,6 +357,7 @@ int lbf_create(const lbf_params* pin, lbf_ctx** out) {
     c->rep_mask = (int8_t*)A(c->N);
   }
   c->isfh = (int8_t*)A((size_t)(p.nx + 2) * (p.ny + 2) * (p.nz + 2));
+  if (p.internal_obstacles) c->words = (uint32_t*)A((size_t)(p.nx + 2) * (p.ny + 2) * (p.nz + 2) * sizeof(uint32_t));
   c->staging = A(c->N * 8);
   c->nred = REDUCE_SCRATCH_BLOCKS;  // the no-alloc variant's partials match this launch
   c->partial = (double*)A((size_t)c->nred * 8 * sizeof(double));
@@ -373,6 +376,10 @@ int lbf_create(const lbf_params* pin, lbf_ctx** out) {
   // all-fluid isfluid until the host uploads one (halo = 1 everywhere)
   std::vector<int8_t> ones((size_t)(p.nx + 2) * (p.ny + 2) * (p.nz + 2), 1);
   if (hipMemcpy(c->isfh, ones.data(), ones.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    lbf_destroy(c);
+    return fail(nullptr, LBF_EHIP, "isfluid init failed");
+  }
+  if (c->words && launch_node_words(c->isfh, c->words, c->dp, c->stream) != hipSuccess) {
     lbf_destroy(c);
     return fail(nullptr, LBF_EHIP, "isfluid init failed");
   }
@@ -548,6 +555,10 @@ int lbf_upload_isfluid(lbf_ctx* c, const int8_t* host) {
             one ? 1 : host[(size_t)c3[0] + (size_t)nx * ((size_t)c3[1] + (size_t)ny * c3[2])];
       }
   HIPCHK(c, hipMemcpy(c->isfh, h.data(), h.size(), hipMemcpyHostToDevice));
+  if (c->words) {
+    HIPCHK(c, launch_node_words(c->isfh, c->words, c->dp, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
   c->isf_set = true;
   return LBF_OK;
 }
@@ -592,7 +603,7 @@ static FusedArgs fused_args(lbf_ctx* c) {
   a.phiout = c->phi[1 - c->cur];
   a.pre = c->pre;
   a.frc = c->frc;
-  a.isfh = c->isfh;
+  a.words = c->words;
   a.dp = c->dp;
   a.ty = c->ty;
   a.tz = c->tz;
@@ -871,7 +882,10 @@ struct lbf_batch {
   std::vector<int> order;
   FusedBatchEntry* ftab[2] = {};
   PrepBatchEntry* ptab[2] = {};
-  int ftotal[2] = {}, ptotal[2] = {};
+  // the fused table holds the domains of std_switches() first (nstd of them,
+  // ftotal[.][0] tiles), then the others (ftotal[.][1]): a launch each
+  int nstd = 0;
+  int ftotal[2][2] = {}, ptotal[2] = {};
   int par = 0;  // 0: tables built from the contexts' current buffers
   std::vector<int> tcur, tucur, tstep;  // each context's (cur, ucur, step) that table 0 describes
   uint32_t* ctr = nullptr;  // per-domain step counters: the 16-bit codecs' rounding seeds
@@ -911,12 +925,20 @@ static void batch_drop_graph(lbf_batch* b) {
 // Device tables for both buffer parities (parity 1 = after one step).
 static int batch_tables(lbf_batch* b) {
   const int nd = (int)b->ctx.size();
+  std::vector<int> order = b->order;
+  b->nstd = (int)(std::stable_partition(order.begin(), order.end(),
+                                        [&](int d) { return std_switches(b->ctx[d]->dp); }) - order.begin());
   for (int par = 0; par < 2; ++par) {
     std::vector<FusedBatchEntry> f(nd);
     std::vector<PrepBatchEntry> q(nd);
     int ft = 0, pt = 0;
+    b->ftotal[par][0] = 0;
     for (int i = 0; i < nd; ++i) {
-      const int d = b->order[i];
+      if (i == b->nstd) {
+        b->ftotal[par][0] = ft;
+        ft = 0;
+      }
+      const int d = order[i];
       lbf_ctx* c = b->ctx[d];
       const int cur0 = c->cur, ucur0 = c->ucur;
       c->cur ^= par;
@@ -942,7 +964,7 @@ static int batch_tables(lbf_batch* b) {
     if (!b->ptab[par]) BHIPCHK(b, hipMalloc(&b->ptab[par], nd * sizeof(PrepBatchEntry)));
     BHIPCHK(b, hipMemcpy(b->ftab[par], f.data(), nd * sizeof(FusedBatchEntry), hipMemcpyHostToDevice));
     BHIPCHK(b, hipMemcpy(b->ptab[par], q.data(), nd * sizeof(PrepBatchEntry), hipMemcpyHostToDevice));
-    b->ftotal[par] = ft;
+    b->ftotal[par][b->nstd < nd ? 1 : 0] = ft;
     b->ptotal[par] = pt;
   }
   b->tcur.resize(nd);
@@ -983,7 +1005,12 @@ static int batch_enqueue(lbf_batch* b, int par) {
     for (lbf_ctx* c : b->ctx) ds = ds && default_scales(c->dp);
     if (ds) kprec |= PREC_DEFSCALE;
   }
-  BHIPCHK(b, launch_fused_batch(b->ftab[par], nd, b->ftotal[par], kprec, b->lattice, b->ho, b->two, b->ty, b->stream));
+  if (b->nstd > 0)
+    BHIPCHK(b, launch_fused_batch(b->ftab[par], b->nstd, b->ftotal[par][0], kprec, b->lattice, b->ho, b->two, true,
+                                  b->ty, b->stream));
+  if (b->nstd < nd)
+    BHIPCHK(b, launch_fused_batch(b->ftab[par] + b->nstd, nd - b->nstd, b->ftotal[par][1], kprec, b->lattice, b->ho,
+                                  b->two, false, b->ty, b->stream));
   if (b->prec == LBF_PREC_FP16S || b->prec == LBF_PREC_BF16S) BHIPCHK(b, launch_tick(b->ctr, nd, b->stream));
   return LBF_OK;
 }
@@ -1120,8 +1147,8 @@ int lbf_batch_step(lbf_batch* b, int32_t nsteps) {
   if (b->par) {
     FusedBatchEntry* f = b->ftab[0]; b->ftab[0] = b->ftab[1]; b->ftab[1] = f;
     PrepBatchEntry* q = b->ptab[0]; b->ptab[0] = b->ptab[1]; b->ptab[1] = q;
-    int t = b->ftotal[0]; b->ftotal[0] = b->ftotal[1]; b->ftotal[1] = t;
-    t = b->ptotal[0]; b->ptotal[0] = b->ptotal[1]; b->ptotal[1] = t;
+    for (int k = 0; k < 2; ++k) std::swap(b->ftotal[0][k], b->ftotal[1][k]);
+    int t = b->ptotal[0]; b->ptotal[0] = b->ptotal[1]; b->ptotal[1] = t;
     b->par = 0;
     batch_drop_graph(b);  // a captured graph refers to the old parity's tables
   }

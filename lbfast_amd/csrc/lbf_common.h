@@ -4,6 +4,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_bf16.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace lbf {
 
@@ -56,6 +57,13 @@ __host__ __device__ inline size_t set_elems(int F, int nx, int ny, int nz) {
   return (size_t)F * set_sx(nx) * ny * nz;
 }
 
+// z plane z of a buffer whose planes are pbytes long
+template <class T>
+__device__ __forceinline__ T* plane_at(T* base, uint32_t pbytes, int z) {
+  typedef typename std::conditional<std::is_const<T>::value, const char, char>::type B;
+  return (T*)((B*)base + (uint64_t)pbytes * (uint32_t)z);
+}
+
 // Load through a wave-uniform base pointer and a 32-bit byte offset (selects
 // the scalar-base + vector-offset global addressing mode).
 template <class T>
@@ -104,6 +112,21 @@ __device__ __forceinline__ void bst(Rsrc r, uint32_t boff, __half v) {
 __device__ __forceinline__ void bst(Rsrc r, uint32_t boff, __hip_bfloat16 v) {
   __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, 0, 0);
 }
+// ... with a wave-uniform byte offset added to every lane's (a scalar operand:
+// the fields of a set share one resource)
+__device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, float v) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, boff, soff, 0);
+}
+__device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, double v) {
+  typedef decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0)) V2;
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, boff, soff, 0);
+}
+__device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, __half v) {
+  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, 0);
+}
+__device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, __hip_bfloat16 v) {
+  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, 0);
+}
 // field f of a field set at one z plane
 template <class T>
 __device__ __forceinline__ T fld(const T* plane0, size_t fs, int f, uint32_t pbytes, uint32_t boff) {
@@ -111,7 +134,7 @@ __device__ __forceinline__ T fld(const T* plane0, size_t fs, int f, uint32_t pby
 }
 template <class T>
 __device__ __forceinline__ void fst(T* plane0, size_t fs, int f, uint32_t pbytes, uint32_t boff, T v) {
-  bst(mkrsrc(plane0 + (size_t)f * fs, pbytes), boff, v);
+  bsts(mkrsrc(plane0, pbytes), boff, (uint32_t)f * (uint32_t)(fs * sizeof(T)), v);
 }
 
 // LDS DMA.  buffer_load_dword with the lds modifier writes each lane's dword
@@ -122,27 +145,46 @@ __device__ __forceinline__ void fst(T* plane0, size_t fs, int f, uint32_t pbytes
 // does not see it; the consumer waits with dma_wait_all() before reading.
 // M0 (= lds + OFF, OFF a compile-time byte offset) is saved and restored
 // around the load, and s_nop 4 covers the M0-write and SGPR-write hazards
-// ahead of the memory instruction.
+// ahead of the memory instruction.  soff is added to
+// every lane's offset (a field of a set whose resource starts at field 0).
 typedef __attribute__((address_space(3))) float lds_float;
 __device__ __forceinline__ uint32_t lds_addr(float* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_float*)p);
 }
 template <uint32_t OFF = 0>
-__device__ __forceinline__ void dma_dword(Rsrc r, uint32_t voff, uint32_t lds) {
+__device__ __forceinline__ void dma_dword(Rsrc r, uint32_t voff, uint32_t lds, uint32_t soff = 0) {
   uint32_t save;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_add_u32 m0, %3, %4\n\t"
       "s_nop 4\n\t"
-      "buffer_load_dword %1, %2, 0 offen lds\n\t"
+      "buffer_load_dword %1, %2, %5 offen lds\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(save)
-      : "v"(voff), "s"(r), "s"(lds), "n"(OFF)
+      : "v"(voff), "s"(r), "s"(lds), "n"(OFF), "s"(__builtin_amdgcn_readfirstlane(soff))
+      : "memory", "scc");
+}
+// The 16-byte form: each lane's four dwords go to M0 + 16*lane, so one transfer
+// moves four 64-value rows of 32-bit fields (eight of 16-bit ones).
+template <uint32_t OFF = 0>
+__device__ __forceinline__ void dma_quad(Rsrc r, uint32_t voff, uint32_t soff, uint32_t lds) {
+  uint32_t save;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_add_u32 m0, %3, %4\n\t"
+      "s_nop 4\n\t"
+      "buffer_load_dwordx4 %1, %2, %5 offen lds\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(save)
+      : "v"(voff), "s"(r), "s"(lds), "n"(OFF), "s"(__builtin_amdgcn_readfirstlane(soff))
       : "memory", "scc");
 }
 // Wait for every outstanding vector-memory operation of this wave (the
 // counter also covers stores, so issue a plane's stores before its DMA).
 __device__ __forceinline__ void dma_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// ... for all but the newest N of them (they retire in issue order)
+template <int N>
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Separable D3Q27 stencils.  The isotropic weights of the gradient and
@@ -470,18 +512,24 @@ __host__ __device__ constexpr double weight(int p, int q, int r) {
 // One-axis Hermite reconstruction of the tensor-product D3Q27 basis:
 // f(c) = sum_a g_a(c) A_a with g_0 = w1d(c), g_1 = 3 w1d c,
 // g_2 = 4.5 w1d (c^2 - 1/3), w1d = (1/6, 2/3, 1/6).  (Minv_mrt of
-// vars_module.f90:359-521 is the product of three of these.)
+// vars_module.f90:359-521 is the product of three of these.)  A1 and A2 are
+// given halved.
 // The centre value is formed as A0 - (fm + fp), which equals 2/3 A0 - A2:
 // in FP32, fl(1/6) + fl(2/3) + fl(1/6) = 1 + 3.0e-8, so weighting A0 by the
 // rounded 2/3 would scale the zeroth moment (the density deviation P) by
 // 1 + 9e-8 per step over the three passes -- a mass drift eleven times that
 // of the rounded weights of the reference's own table.  Formed this way the
 // three values sum to A0 up to unbiased rounding.
+// h1, h2: A1 and A2 are present (constants after unrolling).
 template <class R>
-__device__ __forceinline__ void recon3(R A0, R A1, R A2, R& fm, R& f0, R& fp) {
-  const R t = A0 * (R)(1.0 / 6.0) + A2 * (R)0.5;
-  fp = t + A1 * (R)0.5;
-  fm = t - A1 * (R)0.5;
+__device__ __forceinline__ R recon_side(R A0, R A2, bool h2) {
+  return h2 ? A0 * (R)(1.0 / 6.0) + A2 : A0 * (R)(1.0 / 6.0);
+}
+template <class R>
+__device__ __forceinline__ void recon3(R A0, R A1, R A2, R& fm, R& f0, R& fp, bool h1 = true, bool h2 = true) {
+  const R t = recon_side(A0, A2, h2);
+  fp = h1 ? t + A1 : t;
+  fm = h1 ? t - A1 : t;
   f0 = A0 - (R)2 * t;
 }
 

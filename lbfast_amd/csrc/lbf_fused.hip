@@ -18,21 +18,24 @@
 //   A_0 = P, A_i = u_i + a_i/2, A_ij = u_i u_j + (1-omega) Pn_ij + (u_i a_j + u_j a_i)/2,
 //   A_k = E_k + (1-omega) N_k (k >= 10)
 // (a = force/rho_phi; Guo forcing of fused:705-706 is exactly the order-1/2
-// Hermite part).  The 27 populations then cost three 1-D passes (135 ops)
-// instead of the dense 27x27 sum.  D3Q19 is not a tensor product; its 19
-// populations are built directly from the order <= 2 coefficients.
+// Hermite part).  D3Q19 is not a tensor product; its 19 populations are built
+// directly from the order <= 2 coefficients.
 //
 // Streaming + moments.  out_m(x) = sum_l M_ml f*_l(x - c_l) separates by
-// axis too.  A block owns a 64-wide x segment (one wave per y row, lanes =
-// x) of TY output rows plus one halo row on each side, and marches z.  For
-// each source plane it:
-//   x: shifts the p = +-1 populations one lane (DPP) and contracts
-//      over p with (1, c, c^2-1/3); the two x-halo nodes of every row are
-//      computed by one extra wave and handed over through LDS;
-//   y: exchanges the q = +-1 partial sums with the neighbouring rows through
-//      LDS and contracts over q;
-//   z: adds the r = -1/0/+1 partial sums into three per-lane accumulator
-//      planes; the lowest is complete and is stored.
+// axis too, and the axes' operators (reconstruct over a, shift, contract with
+// 1, c, c^2 - 1/3) commute, so they run axis by axis on the coefficients and
+// the populations as a whole are never formed.  A block owns a 64-wide x
+// segment (one wave per y row, lanes = x) of TY output rows plus one halo row
+// on each side, and marches z.  For each source plane it:
+//   x: reconstructs the 9 lines (b, c), shifts the p = +-1 values one lane
+//      (DPP) and contracts over p; the two x-halo nodes of every row are
+//      computed by one extra wave, which forms only the side it hands over
+//      (through LDS);
+//   y: reconstructs the 9 lines (d, c), exchanges the q = +-1 values with the
+//      neighbouring rows through LDS (halo rows form one side only) and
+//      contracts over q;
+//   z: reconstructs the 6 lines (d, e) that are left and adds r = -1/0/+1 into
+//      15 per-lane sums in flight; the lowest plane is complete and is stored.
 // Every node of the block's (x,y) footprint is collided once per plane; the
 // recomputation is only the two y-halo rows, the x-halo wave and the two
 // z-halo planes of the march.
@@ -46,14 +49,39 @@
 // rewrites phi on solid nodes after compute_norm and before the moments
 // stage, so the gradients come from the prep's output instead.
 //
+// What bounds it: arithmetic and scalar issue, and HBM where the domain is
+// large.  Measured at 512^3 before and after the axis-by-axis order (27% fewer
+// vector instructions a launch), the 16-byte row transfers, the compiled-in
+// switches (std_switches) and one buffer resource per set (scalar instructions
+// of the plane loop 661 -> 367): two components FP32 3.81 -> 3.25 ms (15.0 GB of
+// compulsory state at 4.6 TB/s, the rate of a plain copy on the same card),
+// FP16S 3.15 -> 2.57 ms, one component FP32 2.76 -> 2.34 ms.  Registers decide
+// the variants: a spill inside the plane loop makes the compiler wait for every
+// transfer in flight (FP16S 2.57 -> 3.70 ms with 32 bytes of spills).
+//
 // Periodicity: indices wrap in-kernel (the reference's intpbc halo copies,
-// mpi_module.f90:2820-2918).  isfluid is read from a copy with the
-// reference's 1-node halo (periodic image or 1, LBFAST.f90:258-328).
+// mpi_module.f90:2820-2918).  isfluid and the solid neighbours of near-wall
+// nodes come as one word per node of a copy with the reference's 1-node halo
+// (periodic image or 1, LBFAST.f90:258-328).
 #include "lbf_common.h"
 #include "lbf_kernels.h"
 #include "lbf_physics.h"
 
 namespace lbf {
+
+// The kernels of one storage precision; each is compiled in a translation
+// unit of its own (LBF_FUSED_PREC), the dispatch in one without it.
+template <int PREC>
+hipError_t fused_prec(const FusedArgs& a, bool inline_moments, hipStream_t s);
+template <int PREC>
+hipError_t fused_batch_prec(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool two, bool std, int ty,
+                            hipStream_t s);
+template <int TY>
+__host__ __device__ inline int fused_tiles(const FusedArgs& a) {
+  return ((a.dp.nx + 63) / 64) * ((a.dp.ny + TY - 1) / TY) * ((a.dp.nz + a.tz - 1) / a.tz);
+}
+
+#ifdef LBF_FUSED_PREC
 
 // Whole-wave lane shifts through DPP (wave_shr:1 / wave_shl:1, a VALU
 // operand modifier, no LDS round trip).  With bound_ctrl off, the lane whose
@@ -105,19 +133,40 @@ struct Slots<true, true, true> {
 struct FOff {
   uint32_t m, u, g, p;
   uint32_t pm, pu, pg, pp;
-  // 16-bit storage, full 64-node row segments (pair != 0, wave-uniform;
-  // lane l holds node x0 + l): one transfer moves two fields' rows, lanes
-  // 0-31 the dwords of field f (nodes x0 .. x0+63) and lanes 32-63 those of
-  // field f+1 (pair_delta)
-  int pair;
+  // where the transfers of dma_raw start in the moment, u_old and g sets.  Row
+  // waves (rows != 0, wave-uniform) fetch whole field rows, 16 bytes a lane
+  // (the lane's node + row_off); the x-halo wave the aligned dword of its node.
+  int rows;
+  uint32_t lm, lu, lg;
 };
 
-// byte offset from a lane's own 16-bit element to its dword of a paired
-// transfer: lane l < 32 fetches elements x0+2l, x0+2l+1 of field f, lane
-// l >= 32 elements x0+2(l-32), +1 of field f+1 (sx elements further)
-__device__ __forceinline__ uint32_t pair_delta(int sx) {
+// A wave's 64-node row segments of a set move four (32-bit values) or eight
+// (16-bit) fields to a transfer: lane l fetches 16 bytes of field l / G at
+// element E (l % G), G lanes to a 64-value row.  Lanes past a short row read
+// on into the row's end and the next field; those nodes are never used, and
+// every buffer is padded past its last plane.  The transfers were bound by
+// their number, not their bytes: with a dword a lane the row waves of a block
+// issued 14 a plane (one per field), with 16 bytes 5.
+template <class V>
+__device__ __forceinline__ uint32_t row_off(int sx) {
+  constexpr uint32_t E = 16 / sizeof(V), G = 64 / E;
   const uint32_t l = threadIdx.x & 63;
-  return 2u * (l < 32 ? l : l - 64u + (uint32_t)sx);
+  return ((l / G) * (uint32_t)sx + (l % G) * E - l) * (uint32_t)sizeof(V);
+}
+// the NF fields of a set at one plane into the wave's LDS from byte OFF on
+template <class V, uint32_t OFF, int NF>
+__device__ __forceinline__ void dma_rows(const V* plane0, uint32_t voff, int sx, uint32_t lds0) {
+  constexpr int G = 64 * sizeof(V) / 16, PER = 64 / G;  // lanes per row, rows per transfer
+  const Rsrc r = mkrsrc(plane0, 0xFFFFFFFFu);
+  const uint32_t step = (uint32_t)(PER * sizeof(V)) * (uint32_t)sx;
+  const int l = threadIdx.x & 63;
+  if constexpr (NF >= PER) dma_quad<OFF>(r, voff, 0u, lds0);
+  if constexpr (NF >= 2 * PER) dma_quad<OFF + 1024u>(r, voff, step, lds0);
+  constexpr int W = NF / PER, REM = NF % PER;
+  static_assert(W <= 2, "at most two full transfers");
+  if constexpr (REM != 0) {
+    if (l < REM * G) dma_quad<OFF + 1024u * W>(r, voff, (uint32_t)W * step, lds0);
+  }
 }
 
 // Direct loads of one plane's inputs (used when the inputs are not prefetched).
@@ -155,97 +204,78 @@ __device__ __forceinline__ void load_raw(RawNode<PREC>& r, const FusedArgs& a, i
 // byte (o.m & 2) of the slot; sx is even, so every 16-bit field row starts on
 // a dword and the u_old offsets share that parity).
 template <int PREC, bool TWO, bool INLINE, bool GI>
-__device__ __forceinline__ void dma_raw(const FusedArgs& a, int zw, size_t fs, const FOff& o, uint32_t lds0) {
+__device__ __forceinline__ void dma_raw(const FusedArgs& a, int zw, const FOff& o, bool dens, uint32_t lds0) {
   typedef Slots<TWO, INLINE, GI> SL;
   typedef typename Codec<PREC>::T T;
   static_assert(sizeof(typename Aux<PREC>::T) == 4, "float phase-field storage");
-  constexpr int GF = INLINE ? 5 : 3;
-  const DevParams& dp = a.dp;
-  const size_t rows = (size_t)zw * dp.ny;
-  const uint32_t vM = o.m & ~3u, vU = o.u & ~3u;
-  const T* S = (const T*)a.min + rows * 10 * fs;
+  const int sx = a.dp.sx;
+  const T* S = plane_at((const T*)a.min, o.pm, zw);
+  const float* g = plane_at((const float*)(INLINE ? a.pre : a.frc), o.pg, zw);
+  const T* uo = plane_at((const T*)a.uin, o.pu, zw);
   // slot offsets are immediates: only the wave's LDS base stays live
-  constexpr bool P16 = sizeof(T) == 2 && INLINE;
-  if (P16 && o.pair) {
-    // field pairs (0,1) .. (8,9) into slots 0-4
-    const uint32_t vP = o.m + pair_delta(dp.sx);
-    dma_dword<256u * 0>(mkrsrc(S + 0 * fs, o.pm), vP, lds0);
-    dma_dword<256u * 1>(mkrsrc(S + 2 * fs, o.pm), vP, lds0);
-    dma_dword<256u * 2>(mkrsrc(S + 4 * fs, o.pm), vP, lds0);
-    dma_dword<256u * 3>(mkrsrc(S + 6 * fs, o.pm), vP, lds0);
-    dma_dword<256u * 4>(mkrsrc(S + 8 * fs, o.pm), vP, lds0);
-  } else {
-    dma_dword<256u * 0>(mkrsrc(S + 0 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 1>(mkrsrc(S + 1 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 2>(mkrsrc(S + 2 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 3>(mkrsrc(S + 3 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 4>(mkrsrc(S + 4 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 5>(mkrsrc(S + 5 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 6>(mkrsrc(S + 6 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 7>(mkrsrc(S + 7 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 8>(mkrsrc(S + 8 * fs, o.pm), vM, lds0);
-    dma_dword<256u * 9>(mkrsrc(S + 9 * fs, o.pm), vM, lds0);
-  }
-  if constexpr (TWO && !GI) dma_dword<256u * SL::PHI>(mkrsrc((const float*)a.phin + rows * dp.nx, o.pp), o.p, lds0);
-  if constexpr (!INLINE) {
-    const float* fr = (const float*)a.frc + rows * GF * fs;
-    dma_dword<256u * (SL::G + 0)>(mkrsrc(fr + 0 * fs, o.pg), o.g, lds0);
-    dma_dword<256u * (SL::G + 1)>(mkrsrc(fr + 1 * fs, o.pg), o.g, lds0);
-    dma_dword<256u * (SL::G + 2)>(mkrsrc(fr + 2 * fs, o.pg), o.g, lds0);
-  } else if constexpr (TWO) {
-    const float* pr = (const float*)a.pre + rows * GF * fs;
-    if constexpr (GI) {
-      dma_dword<256u * SL::G>(mkrsrc(pr + 4 * fs, o.pg), o.g, lds0);
-    } else {
-      dma_dword<256u * (SL::G + 0)>(mkrsrc(pr + 0 * fs, o.pg), o.g, lds0);
-      dma_dword<256u * (SL::G + 1)>(mkrsrc(pr + 1 * fs, o.pg), o.g, lds0);
-      dma_dword<256u * (SL::G + 2)>(mkrsrc(pr + 2 * fs, o.pg), o.g, lds0);
-      dma_dword<256u * (SL::G + 3)>(mkrsrc(pr + 3 * fs, o.pg), o.g, lds0);
-      dma_dword<256u * (SL::G + 4)>(mkrsrc(pr + 4 * fs, o.pg), o.g, lds0);
+  if constexpr (TWO && !GI)
+    dma_dword<256u * SL::PHI>(mkrsrc(plane_at((const float*)a.phin, o.pp, zw), o.pp), o.p, lds0);
+  if constexpr (GI) dma_dword<256u * SL::G>(mkrsrc(g, o.pg), o.g, lds0, 16u * (uint32_t)sx);
+  if (o.rows) {
+    dma_rows<T, 0u, 10>(S, o.lm, sx, lds0);
+    if constexpr (!INLINE) dma_rows<float, 256u * SL::G, 3>(g, o.lg, sx, lds0);
+    else if constexpr (TWO && !GI) dma_rows<float, 256u * SL::G, 5>(g, o.lg, sx, lds0);
+    if constexpr (INLINE && TWO) {
+      if (dens) dma_rows<T, 256u * SL::UO, 3>(uo, o.lu, sx, lds0);
     }
-    if (dp.dens) {
-      const T* uo = (const T*)a.uin + rows * 3 * fs;
-      if (P16 && o.pair) {
-        // (u, v) into slot UO, w into the lower half of slot UO+1
-        const uint32_t vP = o.u + pair_delta(dp.sx);
-        dma_dword<256u * (SL::UO + 0)>(mkrsrc(uo + 0 * fs, o.pu), vP, lds0);
-        if ((threadIdx.x & 63) < 32) dma_dword<256u * (SL::UO + 1)>(mkrsrc(uo + 2 * fs, o.pu), vP, lds0);
-      } else {
-        dma_dword<256u * (SL::UO + 0)>(mkrsrc(uo + 0 * fs, o.pu), vU, lds0);
-        dma_dword<256u * (SL::UO + 1)>(mkrsrc(uo + 1 * fs, o.pu), vU, lds0);
-        dma_dword<256u * (SL::UO + 2)>(mkrsrc(uo + 2 * fs, o.pu), vU, lds0);
+    return;
+  }
+  // x-halo wave: at most 32 nodes, a dword each.  A 16-bit field's slot is then
+  // 128 B long as in the row waves
+  const uint32_t fb = (uint32_t)sx * (uint32_t)sizeof(T), gb = (uint32_t)sx * 4u;
+  constexpr uint32_t SB = 64u * (uint32_t)sizeof(T);  // bytes of a field's slot
+  if ((threadIdx.x & 63) < 32) {
+    const Rsrc rm = mkrsrc(S, o.pm);
+    dma_dword<SB * 0>(rm, o.lm, lds0);
+    dma_dword<SB * 1>(rm, o.lm, lds0, 1 * fb);
+    dma_dword<SB * 2>(rm, o.lm, lds0, 2 * fb);
+    dma_dword<SB * 3>(rm, o.lm, lds0, 3 * fb);
+    dma_dword<SB * 4>(rm, o.lm, lds0, 4 * fb);
+    dma_dword<SB * 5>(rm, o.lm, lds0, 5 * fb);
+    dma_dword<SB * 6>(rm, o.lm, lds0, 6 * fb);
+    dma_dword<SB * 7>(rm, o.lm, lds0, 7 * fb);
+    dma_dword<SB * 8>(rm, o.lm, lds0, 8 * fb);
+    dma_dword<SB * 9>(rm, o.lm, lds0, 9 * fb);
+    if constexpr (INLINE && TWO) {
+      if (dens) {
+        const Rsrc ru = mkrsrc(uo, o.pu);
+        dma_dword<256u * SL::UO + SB * 0>(ru, o.lu, lds0);
+        dma_dword<256u * SL::UO + SB * 1>(ru, o.lu, lds0, 1 * fb);
+        dma_dword<256u * SL::UO + SB * 2>(ru, o.lu, lds0, 2 * fb);
       }
+    }
+  }
+  if constexpr (!INLINE || (TWO && !GI)) {
+    const Rsrc rg = mkrsrc(g, o.pg);
+    dma_dword<256u * (SL::G + 0)>(rg, o.lg, lds0);
+    dma_dword<256u * (SL::G + 1)>(rg, o.lg, lds0, 1 * gb);
+    dma_dword<256u * (SL::G + 2)>(rg, o.lg, lds0, 2 * gb);
+    if constexpr (INLINE) {
+      dma_dword<256u * (SL::G + 3)>(rg, o.lg, lds0, 3 * gb);
+      dma_dword<256u * (SL::G + 4)>(rg, o.lg, lds0, 4 * gb);
     }
   }
 }
 
 template <int PREC, bool TWO, bool INLINE, bool GI>
 __device__ __forceinline__ void lds_raw(RawNode<PREC>& r, const float (*slot)[64], int lane, bool dens, uint32_t bT,
-                                        bool pair) {
+                                        bool rows) {
   typedef Slots<TWO, INLINE, GI> SL;
   typedef typename Codec<PREC>::T T;
-  constexpr bool P16 = sizeof(T) == 2 && INLINE;
-  // a 16-bit element sits at byte (bT & 2) of its lane's dword; in a paired
-  // slot (s0 + f/2) field f's 64 elements are the slot's lower or upper 128 B
-  const uint32_t hs = sizeof(T) == 2 ? (bT & 2u) : 0u;
-  auto one = [&](int f) { return *(const T*)((const char*)&slot[f][lane] + hs); };
-  auto two = [&](int s0, int f) { return *(const T*)((const char*)&slot[s0 + (f >> 1)][0] + (f & 1) * 128 + lane * 2); };
-  const bool pr = P16 && pair;
-  constexpr bool UO = INLINE && TWO;
-  if (pr) {
+  // field f's slot holds 64 values (64 sizeof(T) bytes); a 16-bit element of the
+  // x-halo wave is half (bT & 2) of its lane's dword
+  const char* at = (const char*)&slot[0][0] +
+                   (sizeof(T) == 2 && !rows ? (uint32_t)lane * 4u + (bT & 2u) : (uint32_t)lane * (uint32_t)sizeof(T));
 #pragma unroll
-    for (int f = 0; f < 10; ++f) r.m[f] = two(0, f);
-    if (UO && dens) {
+  for (int f = 0; f < 10; ++f) r.m[f] = *(const T*)(at + f * 64 * sizeof(T));
+  if (INLINE && TWO && dens) {
 #pragma unroll
-      for (int f = 0; f < 3; ++f) r.uo[f] = two(SL::UO, f);
-    }
-  } else {
-#pragma unroll
-    for (int f = 0; f < 10; ++f) r.m[f] = one(f);
-    if (UO && dens) {
-#pragma unroll
-      for (int f = 0; f < 3; ++f) r.uo[f] = one(SL::UO + f);
-    }
+    for (int f = 0; f < 3; ++f) r.uo[f] = *(const T*)(at + SL::UO * 256 + f * 64 * sizeof(T));
   }
   if constexpr (TWO && !GI) r.phi = slot[SL::PHI][lane];
   if constexpr (!INLINE) {
@@ -266,13 +296,8 @@ __device__ __forceinline__ void lds_raw(RawNode<PREC>& r, const float (*slot)[64
 // shared load/store counter makes a wait for everything) finds the older
 // stores long done.  The completed output plane is therefore stored at the
 // top of the following iteration.
-template <int TY>
-__host__ __device__ inline int fused_tiles(const FusedArgs& a) {
-  return ((a.dp.nx + 63) / 64) * ((a.dp.ny + TY - 1) / TY) * ((a.dp.nz + a.tz - 1) / a.tz);
-}
-
 // One block: tile `tile` (x fastest, then y, then z chunks) of the domain `a`.
-// OB: the domain has internal obstacles (isfluid loads, solid nodes, the
+// OB: the domain has internal obstacles (node words, solid nodes, the
 // near-wall closures); without them that code is compiled out.
 // A node next to the wall of a non-periodic axis (coordinate 1 or n-2): a
 // superset of the first fluid layers of the open faces.
@@ -281,9 +306,54 @@ __device__ __forceinline__ bool open_layer(const DevParams& dp, int x, int y, in
          (!dp.pbc[2] && (z == 1 || z == dp.nz - 2));
 }
 
+// One population f of velocity (p, q, r) added to the ten closure moments.
+template <class R>
+__device__ __forceinline__ void add_closure(R (&l)[10], int p, int q, int r, R f) {
+  const R cssq = (R)(1.0 / 3.0);
+  l[0] += f;
+  l[1] += f * (R)p; l[2] += f * (R)q; l[3] += f * (R)r;
+  l[4] += f * ((R)(p * p) - cssq); l[5] += f * ((R)(q * q) - cssq); l[6] += f * ((R)(r * r) - cssq);
+  l[7] += f * (R)(p * q); l[8] += f * (R)(p * r); l[9] += f * (R)(q * r);
+}
+// The closure moments of a node of the source plane, put into the z sums of
+// its own plane: line k of zn (which becomes za, or part of zb) takes what
+// enters that line's difference or only sum, lbs[0..2] what its r = 0 value
+// still needs, and lbs[3] the rest of Pi_zz.
+template <class R>
+__device__ __forceinline__ void closure_to_z(const R (&l)[10], R (&zn)[6], R (&lbs)[4]) {
+  zn[0] += l[3]; lbs[0] = l[0] - l[3];
+  zn[1] += l[9]; lbs[1] = l[2] - l[9];
+  zn[2] += l[8]; lbs[2] = l[1] - l[8];
+  zn[3] += (R)3 * l[4]; zn[4] += (R)3 * l[5]; zn[5] += l[7];
+  lbs[3] = l[6] - ((R)(2.0 / 3.0) * l[3] - (R)(1.0 / 3.0) * lbs[0]);
+}
+// One of the three values of recon3, side p = -1, 0 or +1 (uniform over the
+// wave), with the same roundings.
+template <class R>
+__device__ __forceinline__ R recon_one(R A0, R A1, R A2, int p, bool h1, bool h2) {
+  const R t = recon_side(A0, A2, h2);
+  return p == 0 ? A0 - (R)2 * t : (h1 ? t + (R)p * A1 : t);
+}
+// Population (p, q, r) from the Hermite coefficients of hermite27.
+template <bool HO, class R>
+__device__ __forceinline__ R population27(const R (&A)[27], int p, int q, int r) {
+  R C[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    R B[3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+      B[b] = HO || b + c <= 2 ? recon_one(A[3 * b + 9 * c], A[1 + 3 * b + 9 * c], A[2 + 3 * b + 9 * c], p,
+                                          HO || b + c <= 1, HO || b + c == 0)
+                              : (R)0;
+    C[c] = recon_one(B[0], B[1], B[2], q, HO || c <= 1, HO || c == 0);
+  }
+  return recon_one(C[0], C[1], C[2], r, true, true);
+}
+
 // OPEN: open faces (with OB and the inline moments stage only): the kernel
 // also hands over the post-moments state of the wall-adjacent nodes
-template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY, bool OB, bool OPEN = false>
+template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY, bool OB, bool STD, bool OPEN = false>
 __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   typedef Codec<PREC> C;
   typedef typename C::R R;
@@ -308,9 +378,10 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
 
   const DevParams& dp = a.dp;
   const Phys<R>& ph = dp.ph<R>();
+  const bool dens = STD ? TWO : dp.dens != 0;
   const int nx = dp.nx, ny = dp.ny, nz = dp.nz;
   const size_t nxny = (size_t)nx * ny;
-  const bool obst = OB && dp.obst != 0, bb = OB && dp.bb != 0;
+  const bool bb = OB && dp.bb != 0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int ntx = (nx + 63) / 64, nty = (ny + TY - 1) / TY;
   const int tx = tile % ntx, ty = (tile / ntx) % nty, tzi = tile / (ntx * nty);
@@ -337,7 +408,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   // row waves: w == wave (wave-uniform); the halo wave's lanes map to (row, side)
   const bool out_row = !halo_wave && wave >= 1 && wave <= TY && y0 - 1 + wave < ny;
   const bool out_node = out_row && lane < XW;
-  const int xw = ((xs % nx) + nx) % nx;  // lanes past a short row wrap more than once
+  // row waves: lanes past a short row stay unwrapped (never stored)
+  const int xw = PF && !halo_wave ? xs : ((xs % nx) + nx) % nx;
   const int yw = ((ys % ny) + ny) % ny;  // ys may exceed 2ny when ny < TY
   constexpr int GF = INLINE ? 5 : 3;     // fields of the g set: prep output or forces
   const int sx = dp.sx;
@@ -345,26 +417,25 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   FOff off;
   off.m = ((uint32_t)xw + 10u * srow) * (uint32_t)sizeof(T);
   off.u = ((uint32_t)xw + 3u * srow) * (uint32_t)sizeof(T);
-  // paired 16-bit transfers for row waves over a full 64-node segment
-  // (x0 + 63 < nx: no wrap inside the segment)
-  off.pair = (!halo_wave && XW == 64) ? 1 : 0;
+  off.rows = halo_wave ? 0 : 1;
   off.g = ((uint32_t)xw + (uint32_t)GF * srow) * (uint32_t)sizeof(TA);
+  off.lm = off.rows ? off.m + row_off<T>(sx) : off.m & ~3u;
+  off.lu = off.rows ? off.u + row_off<T>(sx) : off.u & ~3u;
+  off.lg = off.rows ? off.g + row_off<float>(sx) : off.g;
   off.p = ((uint32_t)xw + (uint32_t)nx * (uint32_t)yw) * (uint32_t)sizeof(TA);
   const uint32_t splane = (uint32_t)sx * (uint32_t)ny;
   off.pm = ((10u * splane * (uint32_t)sizeof(T)) + 3u) & ~3u;
   off.pu = ((3u * splane * (uint32_t)sizeof(T)) + 3u) & ~3u;
   off.pg = (uint32_t)GF * splane * (uint32_t)sizeof(TA);
   off.pp = (uint32_t)(nxny * sizeof(TA));
-  // isfluid with halo: per-lane in-plane offset, per-plane uniform base
-  const uint32_t bI = (uint32_t)(clampi(xs, -1, nx) + 1) + (uint32_t)(nx + 2) * (uint32_t)(clampi(ys, -1, ny) + 1);
-  const size_t hplane = (size_t)(nx + 2) * (ny + 2);
-  const uint32_t pbI = (uint32_t)hplane;
-  auto isf_load = [&](int z) -> int {
-    return (int)bld<int8_t>(mkrsrc(a.isfh + (size_t)(clampi(z, -1, nz) + 1) * hplane, pbI), bI);
+  // node words with halo: per-lane in-plane offset, per-plane uniform base
+  const uint32_t bI = 4u * ((uint32_t)(clampi(xs, -1, nx) + 1) + (uint32_t)(nx + 2) * (uint32_t)(clampi(ys, -1, ny) + 1));
+  const uint32_t pbI = 4u * (uint32_t)(nx + 2) * (uint32_t)(ny + 2);
+  auto word_load = [&](int z) -> uint32_t {
+    return __builtin_amdgcn_raw_buffer_load_b32(mkrsrc(plane_at(a.words, pbI, clampi(z, -1, nz) + 1), pbI), bI, 0, 0);
   };
 
   T* Sout = (T*)a.mout;
-  const size_t plM = (size_t)10 * sx * ny;  // elements of one z plane of the moment set
   // 16-bit codecs: per-node seed of the stochastic rounding
   // and of the step: without a step term a node whose sibling field is
   // constant (e.g. exactly 0 in a planar flow) would draw the same threshold
@@ -375,24 +446,33 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
     nseed = mix32((uint32_t)xw * 0x9E3779B9u ^ (uint32_t)(yw + 1) * 0x85EBCA6Bu ^ mix32(step * 0x632BE5ABu + 0x1B873593u));
   }
 
-  R lo[10], mid[10], hi[10];
+  // z sums in flight.  The six lines (d, e) that outlive the x and y
+  // contractions -- 0: (0,0), 1: (0,1), 2: (1,0), 3: (2,0), 4: (0,2), 5: (1,1) --
+  // each give a source plane s the values r = -1, 0, +1.  zn: r = +1 of the last
+  // source plane (it streams to the plane above); za, zb: r = +1 from below and
+  // r = 0 of the plane that the next source plane completes, added up where
+  // only their sum is needed (lines 3..5).  15 values instead of three planes of
+  // ten accumulators, and no moves of whole accumulator planes.
+  R zn[6], za[3], zb[6], oc[10];
 #pragma unroll
-  for (int m = 0; m < 10; ++m) { lo[m] = 0; mid[m] = 0; hi[m] = 0; }
-  auto store_lo = [&](int zo, size_t fs) {
+  for (int k = 0; k < 6; ++k) { zn[k] = 0; zb[k] = 0; }
+  za[0] = za[1] = za[2] = 0;
+  R zbz = 0;  // the closure's share of the pending plane's Pi_zz (OB)
+  auto store_oc = [&](int zo) {
     Mom<R> o;
-    o.P = lo[0]; o.u = lo[1]; o.v = lo[2]; o.w = lo[3];
-    o.xx = lo[4]; o.yy = lo[5]; o.zz = lo[6]; o.xy = lo[7]; o.xz = lo[8]; o.yz = lo[9];
-    store_mom_b<PREC>(Sout + (size_t)zo * plM, fs, off.pm, off.m, o, dp, nseed ^ (uint32_t)zo * 0xC2B2AE35u);
+    o.P = oc[0]; o.u = oc[1]; o.v = oc[2]; o.w = oc[3];
+    o.xx = oc[4]; o.yy = oc[5]; o.zz = oc[6]; o.xy = oc[7]; o.xz = oc[8]; o.yz = oc[9];
+    store_mom_b<PREC>(plane_at(Sout, off.pm, zo), (size_t)sx, off.pm, off.m, o, dp, nseed ^ (uint32_t)zo * 0xC2B2AE35u);
   };
 
-  const R third = (R)(1.0 / 3.0), twothird = (R)(2.0 / 3.0);
+  const R third = (R)(1.0 / 3.0);
 
   uint32_t lds0 = 0;
-  int isf_next = 1;
+  uint32_t word_next = NODE_FLUID;
   if constexpr (PF) {
     lds0 = lds_addr(&sPF[wave][0][0]);
-    dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(z0 - 1, nz), (size_t)sx, off, lds0);
-    if (obst) isf_next = isf_load(z0 - 1);
+    dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(z0 - 1, nz), off, dens, lds0);
+    if constexpr (OB) word_next = word_load(z0 - 1);
   }
 
   // ---- GI: phi tile stream and the per-node partial sums ------------------------
@@ -403,32 +483,43 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   // published by that iteration's barriers) and streams plane zsrc+3 into the
   // slot of plane zsrc-1, which every wave finished reading in iteration
   // zsrc-2.
-  uint32_t ph_row1 = 0, ph_row2 = 0, ph_xm = 0, ph_xl = 0, ph_xr = 0;
+  uint32_t ph_row1 = 0, ph_row2 = 0, ph_xm = 0, ph_xh = 0;
   const uint32_t lds_ph = GI ? lds_addr(&sPH[0][0][0]) : 0u;
   auto modn = [](int i, int n) { return ((i % n) + n) % n; };
   if constexpr (GI) {
     ph_row1 = __builtin_amdgcn_readfirstlane((uint32_t)modn(y0 - 2 + wave, ny) * (uint32_t)nx * 4u);
     ph_row2 = __builtin_amdgcn_readfirstlane((uint32_t)modn(y0 - 2 + GR - 1, ny) * (uint32_t)nx * 4u);
     ph_xm = (uint32_t)modn(x0 + lane, nx) * 4u;
-    ph_xl = (uint32_t)modn(x0 - 2 + (lane & 1), nx) * 4u;
-    ph_xr = (uint32_t)modn(x0 + 64 + (lane & 1), nx) * 4u;
+    // halo columns: lanes 0-1 the left pair, lanes 2-3 the right
+    ph_xh = (uint32_t)modn((lane & 2) ? x0 + 62 + (lane & 3) : x0 - 2 + (lane & 1), nx) * 4u;
+  }
+  // Away from the x faces (no wrap inside the tile's columns) the tile is one
+  // run of 17 GR 16-byte pieces, a lane each.
+  const bool ph_quad = GI && x0 >= 2 && x0 + 66 <= nx;
+  if (ph_quad) {
+    const int L = min((int)threadIdx.x, GR * (GC / 4) - 1);
+    ph_xm = ((uint32_t)modn(y0 - 2 + L / (GC / 4), ny) * (uint32_t)nx + (uint32_t)(x0 - 2 + 4 * (L % (GC / 4)))) * 4u;
   }
   auto dma_phi = [&](int z) {
-    const Rsrc rs = mkrsrc((const float*)a.phin + (size_t)modn(z, nz) * nxny, (uint32_t)(nxny * 4u));
+    if (ph_quad) {
+      if ((int)threadIdx.x < GR * (GC / 4)) {
+        const Rsrc rq = mkrsrc(plane_at((const float*)a.phin, off.pp, modn(z, nz)), off.pp);
+        dma_quad<0u>(rq, ph_xm, 0u,
+                     lds_ph + (uint32_t)(z & 3) * (uint32_t)(GR * GC * 4) + (uint32_t)wave * 1024u);
+      }
+      return;
+    }
+    const Rsrc rs = mkrsrc(plane_at((const float*)a.phin, off.pp, modn(z, nz)), off.pp);
     const uint32_t base = lds_ph + (uint32_t)(z & 3) * (uint32_t)(GR * GC * 4);
     const uint32_t r1 = base + (uint32_t)wave * (uint32_t)(GC * 4);
     dma_dword<8u>(rs, ph_row1 + ph_xm, r1);
-    if (lane < 2) {
-      dma_dword<0u>(rs, ph_row1 + ph_xl, r1);
-      dma_dword<66u * 4u>(rs, ph_row1 + ph_xr, r1);
-    }
+    if (lane < 2) dma_dword<0u>(rs, ph_row1 + ph_xh, r1);
+    if ((lane & ~1) == 2) dma_dword<64u * 4u>(rs, ph_row1 + ph_xh, r1);
     if (wave == 0) {
       const uint32_t r2 = base + (uint32_t)(GR - 1) * (uint32_t)(GC * 4);
       dma_dword<8u>(rs, ph_row2 + ph_xm, r2);
-      if (lane < 2) {
-        dma_dword<0u>(rs, ph_row2 + ph_xl, r2);
-        dma_dword<66u * 4u>(rs, ph_row2 + ph_xr, r2);
-      }
+      if (lane < 2) dma_dword<0u>(rs, ph_row2 + ph_xh, r2);
+      if ((lane & ~1) == 2) dma_dword<64u * 4u>(rs, ph_row2 + ph_xh, r2);
     }
   };
   // this lane's node sits at tile row w + 1, column pc
@@ -458,14 +549,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   for (int zsrc = z0 - 1; zsrc <= zend; ++zsrc) {
     const int zw = wrapg(zsrc, nz);
     const bool own_plane = zsrc >= z0 && zsrc < zend;
-    // the field stride, opaque to the optimiser inside the loop: the ~30
-    // per-field plane offsets are then rebuilt by scalar ALU each iteration
-    // instead of being hoisted and spilled to vector-register lanes
-    size_t fs = (size_t)sx;
-    asm volatile("" : "+s"(fs));
-
     RawNode<PREC> cur;
-    int8_t isf = 1;
+    uint32_t word = NODE_FLUID;
     if constexpr (PF) {
       dma_wait_all();
       // 16-bit storage: waves between this wait and the next plane's DMA
@@ -473,14 +558,13 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
       // waves in the collision, so the transfers start sooner (fused kernel
       // 3.92 -> 3.43 ms FP16S at 512^3; no gain for FP32)
       if constexpr (sizeof(T) == 2) __builtin_amdgcn_s_setprio(2);
-      int t = isf_next;
-      asm volatile("" : "+v"(t));  // consume the prefetched isfluid before this iteration's stores
-      isf = (int8_t)t;
+      if constexpr (OB) {
+        word = word_next;
+        asm volatile("" : "+v"(word));  // consume the prefetched word before this iteration's stores
+      }
       // the plane completed by the previous iteration
-      if (out_row && lane < XW && zsrc - 2 >= z0) store_lo(zsrc - 2, fs);
-#pragma unroll
-      for (int m = 0; m < 10; ++m) { lo[m] = mid[m]; mid[m] = hi[m]; }
-      lds_raw<PREC, TWO, INLINE, GI>(cur, sPF[wave], lane, dp.dens, off.m, off.pair != 0);
+      if (out_row && lane < XW && zsrc - 2 >= z0) store_oc(zsrc - 2);
+      lds_raw<PREC, TWO, INLINE, GI>(cur, sPF[wave], lane, dens, off.m, off.rows != 0);
       if constexpr (GI) {
         // the prep's fields 0-3 (prep_body_z, stored at storage precision)
         const Part3<R> gpp = phi_part(zsrc + 1);
@@ -498,14 +582,15 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
         gp0 = gpp;
       }
     } else {
-      if (obst) isf = (int8_t)isf_load(zsrc);
-      load_raw<PREC, TWO, INLINE>(cur, a, zw, fs, off);
+      if constexpr (OB) word = word_load(zsrc);
+      load_raw<PREC, TWO, INLINE>(cur, a, zw, (size_t)sx, off);
     }
 
     // ---- 1. decode + (inline) moments stage + collision ---------------------
+    // f: D3Q27 the Hermite coefficients A[a + 3b + 9c] (hermite27), D3Q19 the
+    // populations
     R f[27];
-    R lbc[10];
-    bool has_lbc = false;
+    R lbs[4] = {0, 0, 0, 0};  // near-wall closure: what zn cannot take (below)
     {
       NodeIn<R> in;
       Mom<R> m;
@@ -524,9 +609,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
         m.yz = C::decpi(cur.m[9], iscl<PREC>(dp, 9), m.v * m.w);
       }
       R phl = 0, Fx, Fy, Fz;
-      const bool solid = obst && isf == 0;
+      const bool solid = OB && !(word & NODE_FLUID), wall = OB && (word & NODE_WALL);
       if constexpr (TWO) phl = (R)cur.phi;
-      const NodeRates<R> nr = node_rates<TWO, R>(dp, phl);
+      const NodeRates<R> nr = node_rates<TWO, R, STD>(dp, phl);
       const R rinv = nr.irho;
       if constexpr (!INLINE) {
         Fx = (R)cur.g[0] * rinv;
@@ -540,14 +625,14 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
           gfz = (R)cur.g[2];
           lap = (R)cur.g[3];
           dvt = (R)cur.g[4];
-          if (dp.dens) {
+          if (dens) {
             uox = C::dec(cur.uo[0], iscl<PREC>(dp, 1));
             uoy = C::dec(cur.uo[1], iscl<PREC>(dp, 2));
             uoz = C::dec(cur.uo[2], iscl<PREC>(dp, 3));
           }
         }
         R tFx, tFy, tFz;
-        moments_stage<TWO, R>(dp, nr, phl, gfx, gfy, gfz, lap, dvt, uox, uoy, uoz, m, tFx, tFy, tFz);
+        moments_stage<TWO, R, STD>(dp, nr, phl, gfx, gfy, gfz, lap, dvt, uox, uoy, uoz, m, tFx, tFy, tFz);
         // the reference stores S and the forces at storage precision between
         // the moments and fused kernels
         m.u = C::round(m.u); m.v = C::round(m.v); m.w = C::round(m.w);
@@ -557,16 +642,16 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
         Fx = tFx * rinv; Fy = tFy * rinv; Fz = tFz * rinv;
         if (out_node && own_plane && !solid) {
           if constexpr (OPEN) {
-            if (isf == -1 && open_layer(dp, xs, ys, zsrc)) {
+            if (wall && open_layer(dp, xs, ys, zsrc)) {
               // open faces: the post-moments state of a first-layer node,
               // which the open-face correction reads after this launch (the
               // stage sequence reads it from S)
-              store_mom_b<PREC>((T*)a.sopen + (size_t)zw * plM, fs, off.pm, off.m, m, dp, 0u);
+              store_mom_b<PREC>(plane_at((T*)a.sopen, off.pm, zw), (size_t)sx, off.pm, off.m, m, dp, 0u);
             }
           }
           if constexpr (TWO) {
-            if (dp.dens) {
-              T* uo = (T*)a.uout + (size_t)zw * ny * 3 * fs;
+            if (dens) {
+              T* uo = plane_at((T*)a.uout, off.pu, zw);
               T eu = C::enc(m.u, scl<PREC>(dp, 1)), ev = C::enc(m.v, scl<PREC>(dp, 2)), ew = C::enc(m.w, scl<PREC>(dp, 3));
               if constexpr (C::dev) {
                 const uint32_t st = (nseed ^ (uint32_t)zw * 0x27D4EB2Fu) & C::RBITS;
@@ -575,40 +660,38 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
                 ev = C::srx(xv, (__float_as_uint(xw_) & C::RBITS) ^ st);
                 ew = C::srx(xw_, (__float_as_uint(xu) & C::RBITS) ^ st);
               }
-              fst(uo, fs, 0, off.pu, off.u, eu);
-              fst(uo, fs, 1, off.pu, off.u, ev);
-              fst(uo, fs, 2, off.pu, off.u, ew);
+              fst(uo, (size_t)sx, 0, off.pu, off.u, eu);
+              fst(uo, (size_t)sx, 1, off.pu, off.u, ev);
+              fst(uo, (size_t)sx, 2, off.pu, off.u, ew);
             }
             // update_phi (update_phi:88-93), u after the moments stage
             const R t = -ph.sharp_c * dvt;
             const R po = phl - m.u * (R)0.5 * (gfx) - m.v * (R)0.5 * (gfy) - m.w * (R)0.5 * (gfz) +
                          ph.tau_diff * lap + t;
-            fst((TA*)a.phiout + (size_t)zw * nxny, fs, 0, off.pp, off.p, (TA)po);
+            fst(plane_at((TA*)a.phiout, off.pp, zw), (size_t)sx, 0, off.pp, off.p, (TA)po);
           }
-          if (obst && !bb && isf == -1) {
-            // LB_int_boundary (boundary:117-212) on the post-moments state
-            has_lbc = true;
+          if (OB && !bb && wall) {
+            // LB_int_boundary (boundary:117-212) on the post-moments state: the
+            // directions that some lane of the wave needs, one at a time
+            R lbc[10];
             const R cssq = (R)(1.0 / 3.0);
             const R pxx = m.xx - m.u * m.u, pyy = m.yy - m.v * m.v, pzz = m.zz - m.w * m.w;
             const R pxy = m.xy - m.u * m.v, pxz = m.xz - m.u * m.w, pyz = m.yz - m.v * m.w;
-            const R om = relax_rate<TWO, R>(dp, nr, pxx, pyy, pzz, pxy, pxz, pyz);
+            const R om1 = (R)4.5 * ((R)1 - relax_rate<TWO, R, STD>(dp, nr, pxx, pyy, pzz, pxy, pxz, pyz));
 #pragma unroll
             for (int q = 0; q < 10; ++q) lbc[q] = 0;
 #pragma unroll
             for (int c = 0; c < 27; ++c) {
               const int p = c % 3 - 1, q = (c / 3) % 3 - 1, r = c / 9 - 1;
               if (c == 13 || !present<LAT>(p, q, r)) continue;
-              if (isf_at(a.isfh, xs - p, ys - q, zsrc - r, nx, ny, nz) != 0) continue;
-              const R wl = (R)weight<LAT>(p, q, r);
-              const R fneq = wl * (R)4.5 *
-                             (((R)(p * p) - cssq) * pxx + ((R)(q * q) - cssq) * pyy + ((R)(r * r) - cssq) * pzz +
-                              (R)(2 * p * q) * pxy + (R)(2 * p * r) * pxz + (R)(2 * q * r) * pyz);
-              const R fp = wl * m.P + ((R)1 - om) * fneq;
-              lbc[0] += fp;
-              lbc[1] += fp * (R)p; lbc[2] += fp * (R)q; lbc[3] += fp * (R)r;
-              lbc[4] += fp * ((R)(p * p) - cssq); lbc[5] += fp * ((R)(q * q) - cssq); lbc[6] += fp * ((R)(r * r) - cssq);
-              lbc[7] += fp * (R)(p * q); lbc[8] += fp * (R)(p * r); lbc[9] += fp * (R)(q * r);
+              const bool hit = word & (1u << c);
+              if (__ballot(hit) == 0) continue;
+              const R qn = ((R)(p * p) - cssq) * pxx + ((R)(q * q) - cssq) * pyy + ((R)(r * r) - cssq) * pzz +
+                           (R)(2 * p * q) * pxy + (R)(2 * p * r) * pxz + (R)(2 * q * r) * pyz;
+              const R fp = (R)weight<LAT>(p, q, r) * (m.P + om1 * qn);
+              add_closure<R>(lbc, p, q, r, hit ? fp : (R)0);
             }
+            closure_to_z<R>(lbc, zn, lbs);
           }
         }
       }
@@ -620,58 +703,92 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
       in.xx = m.xx - m.u * m.u; in.yy = m.yy - m.v * m.v; in.zz = m.zz - m.w * m.w;
       in.xy = m.xy - m.u * m.v; in.xz = m.xz - m.u * m.w; in.yz = m.yz - m.v * m.w;
       in.ax = Fx; in.ay = Fy; in.az = Fz;
-      in.om = relax_rate<TWO, R>(dp, nr, in.xx, in.yy, in.zz, in.xy, in.xz, in.yz);
+      in.om = relax_rate<TWO, R, STD>(dp, nr, in.xx, in.yy, in.zz, in.xy, in.xz, in.yz);
       if constexpr (PF) {
         // every store of this iteration is issued: stream the next plane in
         lds_wait_all();
         if (zsrc < zend) {
-          if (!halo_wave) dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(zsrc + 1, nz), fs, off, lds0);
-          if (obst) isf_next = isf_load(zsrc + 1);
+          if (!halo_wave) dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(zsrc + 1, nz), off, dens, lds0);
+          if constexpr (OB) word_next = word_load(zsrc + 1);
         }
         if (GI && zsrc + 3 <= zend + 1) dma_phi(zsrc + 3);
         if constexpr (sizeof(T) == 2) __builtin_amdgcn_s_setprio(0);
       }
-      collide<LAT, HO, R>(in, f);
-      if (bb && isf == -1 && out_node && own_plane) {
+      if constexpr (LAT == 27) hermite27<HO, R>(in, f);
+      else collide<LAT, HO, R>(in, f);
+      if (bb && wall && out_node && own_plane) {
         // BOUNCE_BACK (fused_LB_kernel_bb, fused:364-382): a population whose
         // upstream node is solid is replaced by this node's own opposite
         // post-collision population.  The solid node's pushed population is
         // exactly zero (its moments and force are zeroed), so the pull below
-        // adds zero and the replacement is this correction.
-        has_lbc = true;
-        const R cssq = (R)(1.0 / 3.0);
+        // adds zero and the replacement is this correction.  D3Q27 forms the
+        // opposite population from the coefficients, one direction at a time
+        // (a loop, not 26 copies: the populations all at once would not fit
+        // the registers beside the coefficients).
+        R lbc[10];
 #pragma unroll
         for (int q = 0; q < 10; ++q) lbc[q] = 0;
+        if constexpr (LAT == 27) {
+#pragma unroll 1
+          for (int c = 0; c < 27; ++c) {
+            const bool hit = word & (1u << c);
+            if (c == 13 || __ballot(hit) == 0) continue;
+            const int p = c % 3 - 1, q = (c / 3) % 3 - 1, r = c / 9 - 1;
+            add_closure<R>(lbc, p, q, r, hit ? population27<HO, R>(f, -p, -q, -r) : (R)0);
+          }
+        } else {
 #pragma unroll
-        for (int c = 0; c < 27; ++c) {
-          const int p = c % 3 - 1, q = (c / 3) % 3 - 1, r = c / 9 - 1;
-          if (c == 13 || !present<LAT>(p, q, r)) continue;
-          if (isf_at(a.isfh, xs - p, ys - q, zsrc - r, nx, ny, nz) != 0) continue;
-          const R fo = f[cidx(-p, -q, -r)];
-          lbc[0] += fo;
-          lbc[1] += fo * (R)p; lbc[2] += fo * (R)q; lbc[3] += fo * (R)r;
-          lbc[4] += fo * ((R)(p * p) - cssq); lbc[5] += fo * ((R)(q * q) - cssq); lbc[6] += fo * ((R)(r * r) - cssq);
-          lbc[7] += fo * (R)(p * q); lbc[8] += fo * (R)(p * r); lbc[9] += fo * (R)(q * r);
+          for (int c = 0; c < 27; ++c) {
+            const int p = c % 3 - 1, q = (c / 3) % 3 - 1, r = c / 9 - 1;
+            if (c == 13 || !present<LAT>(p, q, r)) continue;
+            add_closure<R>(lbc, p, q, r, word & (1u << c) ? f[cidx(-p, -q, -r)] : (R)0);
+          }
         }
+        closure_to_z<R>(lbc, zn, lbs);
       }
     }
 
-    // ---- 2. x-halo slices through LDS -------------------------------------------
-    if (halo_wave && active) {
-      // left halo streams +x into lane 0, right -x into lane XW-1.  The two
-      // sides are separate branches with constant register indices: a
-      // select between the sides' values is turned by the compiler into a
-      // lane-variable index and expanded into a 27-way compare chain.
-      if (side == 0) {
+    // ---- 2. x: reconstruct over a (D3Q27); the halo's slices through LDS ------------
+    // Axis by axis: a line (b, c) of Hermite coefficients (D3Q19: (q, r) of
+    // populations) becomes its three x populations, which shift one lane and
+    // contract to the moment index d before the next axis is reconstructed.
+    // The axes' operators commute, so this is the full reconstruction followed
+    // by the full contraction with fewer lines left on the later axes (6
+    // instead of 9 in z), and a halo node stops at the one slice that it hands
+    // over: the x-halo wave forms 9 of its 27 populations, the halo rows 9
+    // partial sums.
+    if (halo_wave) {
+      // the left halo (side 0) streams +x into lane 0, the right -x into lane XW-1
+      if constexpr (LAT == 27) {
+        const R sg = side ? (R)-1 : (R)1;
 #pragma unroll
-        for (int r = -1; r <= 1; ++r)
+        for (int j = 0; j < 9; ++j) {
+          const int b = j % 3, c = j / 3;
+          R t = 0;
+          if (HO || b + c <= 2) t = recon_side(f[3 * j], f[3 * j + 2], HO || b + c == 0);
+          if (HO || b + c <= 1) t = t + sg * f[3 * j + 1];
+          if (active) sHX[w][side][j] = t;
+        }
+      } else if (active) {
+        // the two sides are separate branches with constant register indices:
+        // a select between the sides' values is turned by the compiler into a
+        // lane-variable index and expanded into a 27-way compare chain
+        if (side == 0) {
 #pragma unroll
-          for (int q = -1; q <= 1; ++q) sHX[w][0][(q + 1) + 3 * (r + 1)] = f[cidx(1, q, r)];
-      } else {
+          for (int j = 0; j < 9; ++j) sHX[w][0][j] = f[3 * j + 2];
+        } else {
 #pragma unroll
-        for (int r = -1; r <= 1; ++r)
+          for (int j = 0; j < 9; ++j) sHX[w][1][j] = f[3 * j];
+        }
+      }
+    } else if constexpr (LAT == 27) {
 #pragma unroll
-          for (int q = -1; q <= 1; ++q) sHX[w][1][(q + 1) + 3 * (r + 1)] = f[cidx(-1, q, r)];
+      for (int j = 0; j < 9; ++j) {
+        const int b = j % 3, c = j / 3;
+        if (!HO && b + c > 2) continue;
+        R fm, f0, fp;
+        recon3(f[3 * j], f[3 * j + 1], f[3 * j + 2], fm, f0, fp, HO || b + c <= 1, HO || b + c == 0);
+        f[3 * j] = fm; f[3 * j + 1] = f0; f[3 * j + 2] = fp;
       }
     }
     if constexpr (PF) {
@@ -682,113 +799,144 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
       // FP16S at 512^3).  Its slots were read at the top of the iteration.
       if (halo_wave && zsrc < zend) {
         lds_wait_all();
-        dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(zsrc + 1, nz), (size_t)sx, off, lds0);
+        dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(zsrc + 1, nz), off, dens, lds0);
       }
     }
     __syncthreads();
 
-    R G0[9];  // q = 0 partial sums kept in registers: [d][r]
+    R G0[9];  // q = 0 partial sums kept in registers: [d][c]
     if (!halo_wave) {
       // ---- 3. x: shift by one lane, contract over p ---------------------------
       // the x-halo values enter as DPP fill operands, read by every lane
-      // from one LDS address (a broadcast)
-      const bool short_row = XW < 64;  // the right halo enters below lane 63
-      R G[3][3][3];  // [d][q][r]
+      // from one LDS address (a broadcast).  d = 2 is carried as 3 (c^2 - 1/3)
+      // = 2, -1, 2 (one multiply-add, one rounding); the factor 1/3 follows
+      // when the plane is complete.
+      if (XW < 64 && lane == XW) {
+        // a short row's right halo enters below lane 63: put it where lane
+        // XW - 1 fetches from
 #pragma unroll
-      for (int r = -1; r <= 1; ++r)
+        for (int j = 0; j < 9; ++j) f[3 * j] = sHX[wave][1][j];
+      }
+      R G[3][9];  // [d][line]
 #pragma unroll
-        for (int q = -1; q <= 1; ++q) {
-          const int qr = (q + 1) + 3 * (r + 1);
-          R fm_in = 0, fp_in = 0;
-          if (present<LAT>(1, q, r)) fp_in = shift_from_lower(f[cidx(1, q, r)], sHX[wave][0][qr]);
-          if (present<LAT>(-1, q, r)) {
-            const R hr = sHX[wave][1][qr];
-            fm_in = shift_from_upper(f[cidx(-1, q, r)], hr);
-            if (short_row) fm_in = lane == XW - 1 ? hr : fm_in;
-          }
-          const R f0 = present<LAT>(0, q, r) ? f[cidx(0, q, r)] : (R)0;
-          const R s = fm_in + f0 + fp_in;
-          G[0][q + 1][r + 1] = s;
-          G[1][q + 1][r + 1] = fp_in - fm_in;
-          G[2][q + 1][r + 1] = twothird * (fp_in + fm_in) - third * f0;
+      for (int j = 0; j < 9; ++j) {
+        const int b = j % 3, c = j / 3;  // D3Q19: q + 1, r + 1
+        const bool any = LAT == 27 ? (HO || b + c <= 2) : true;
+        const bool sides = LAT == 27 ? any : present<LAT>(1, b - 1, c - 1);
+        R fm_in = 0, fp_in = 0;
+        if (sides) {
+          fp_in = shift_from_lower(f[3 * j + 2], sHX[wave][0][j]);
+          fm_in = shift_from_upper(f[3 * j], sHX[wave][1][j]);
         }
+        if (!any) {
+          G[0][j] = G[1][j] = G[2][j] = 0;
+        } else if (!sides) {
+          G[0][j] = f[3 * j + 1]; G[1][j] = 0; G[2][j] = -f[3 * j + 1];
+        } else {
+          const R sp = fp_in + fm_in;
+          G[0][j] = f[3 * j + 1] + sp;
+          G[1][j] = fp_in - fm_in;
+          G[2][j] = (R)2 * sp - f[3 * j + 1];
+        }
+      }
       // ---- 4a. y: hand the q = +-1 partial sums to the neighbouring rows ------
+      R T0[9], T1[9];
 #pragma unroll
       for (int d = 0; d < 3; ++d)
 #pragma unroll
-        for (int r = 0; r < 3; ++r) {
-          if (wave < NW - 1) sUP[wave][d * 3 + r][lane] = G[d][2][r];
-          if (wave > 0) sDN[wave][d * 3 + r][lane] = G[d][0][r];
-          G0[d * 3 + r] = G[d][1][r];
+        for (int c = 0; c < 3; ++c) {
+          const int k = d * 3 + c, j = 3 * c;
+          if constexpr (LAT == 27) {
+            T0[k] = recon_side(G[d][j], G[d][j + 2], HO || c == 0);
+            T1[k] = HO || c <= 1 ? G[d][j + 1] : (R)0;
+            G0[k] = G[d][j] - (R)2 * T0[k];
+          } else {
+            T0[k] = G[d][j + 2]; T1[k] = G[d][j];
+            G0[k] = G[d][j + 1];
+          }
         }
+      if (wave < NW - 1) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) sUP[wave][k][lane] = LAT == 27 ? T0[k] + T1[k] : T0[k];
+      }
+      if (wave > 0) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) sDN[wave][k][lane] = LAT == 27 ? T0[k] - T1[k] : T1[k];
+      }
     }
     __syncthreads();
 
     if (out_row) {
       // ---- 4b. y: contract over q ------------------------------------------------
-      // H[d][e][r] for (d,e) in {00, 01, 02, 10, 11, 20}
-      R H00[3], H01[3], H02[3], H10[3], H11[3], H20[3];
+      // H[k][c] of the six lines (d, e); e = 2 tripled as d = 2 above
+      R H[6][3];
 #pragma unroll
-      for (int r = 0; r < 3; ++r) {
+      for (int c = 0; c < 3; ++c) {
         {
-          const R gp = sUP[wave - 1][0 * 3 + r][lane], gm = sDN[wave + 1][0 * 3 + r][lane], g0 = G0[0 * 3 + r];
-          H00[r] = gm + g0 + gp;
-          H01[r] = gp - gm;
-          H02[r] = twothird * (gp + gm) - third * g0;
+          const R gp = sUP[wave - 1][c][lane], gm = sDN[wave + 1][c][lane], sp = gp + gm;
+          H[0][c] = G0[c] + sp;
+          H[1][c] = gp - gm;
+          H[4][c] = (R)2 * sp - G0[c];
         }
         {
-          const R gp = sUP[wave - 1][1 * 3 + r][lane], gm = sDN[wave + 1][1 * 3 + r][lane], g0 = G0[1 * 3 + r];
-          H10[r] = gm + g0 + gp;
-          H11[r] = gp - gm;
+          const R gp = sUP[wave - 1][3 + c][lane], gm = sDN[wave + 1][3 + c][lane];
+          H[2][c] = G0[3 + c] + (gp + gm);
+          H[5][c] = gp - gm;
         }
-        {
-          const R gp = sUP[wave - 1][2 * 3 + r][lane], gm = sDN[wave + 1][2 * 3 + r][lane], g0 = G0[2 * 3 + r];
-          H20[r] = gm + g0 + gp;
-        }
+        H[3][c] = G0[6 + c] + (sUP[wave - 1][6 + c][lane] + sDN[wave + 1][6 + c][lane]);
       }
-      // ---- 5. z: r = +1 -> plane zsrc+1 (hi), 0 -> zsrc (mid), -1 -> zsrc-1 (lo)
+      // ---- 5. z: r = -1 completes plane zsrc-1, r = 0 and +1 stay in flight --------
       // outputs: 0 P(000) 1 u(100) 2 v(010) 3 w(001) 4 xx(200) 5 yy(020) 6 zz(002)
-      //          7 xy(110) 8 xz(101) 9 yz(011); index [0]=r-1 [1]=r0 [2]=r+1
-      // plane zsrc+1 receives its first term here: assign rather than add to
-      // a zero (0 + x cannot be folded for signed zeros)
-      hi[0] = H00[2]; mid[0] += H00[1]; lo[0] += H00[0];
-      hi[3] = H00[2]; lo[3] -= H00[0];
-      hi[6] = twothird * H00[2]; mid[6] -= third * H00[1]; lo[6] += twothird * H00[0];
-      hi[2] = H01[2]; mid[2] += H01[1]; lo[2] += H01[0];
-      hi[9] = H01[2]; lo[9] -= H01[0];
-      hi[1] = H10[2]; mid[1] += H10[1]; lo[1] += H10[0];
-      hi[8] = H10[2]; lo[8] -= H10[0];
-      hi[5] = H02[2]; mid[5] += H02[1]; lo[5] += H02[0];
-      hi[4] = H20[2]; mid[4] += H20[1]; lo[4] += H20[0];
-      hi[7] = H11[2]; mid[7] += H11[1]; lo[7] += H11[0];
-      if (has_lbc) {
+      //          7 xy(110) 8 xz(101) 9 yz(011)
+      R hm[6], h0[6], hp[6];
 #pragma unroll
-        for (int q = 0; q < 10; ++q) mid[q] += lbc[q];
+      for (int k = 0; k < 6; ++k) {
+        if constexpr (LAT == 27) recon3(H[k][0], H[k][1], H[k][2], hm[k], h0[k], hp[k]);
+        else { hm[k] = H[k][0]; h0[k] = H[k][1]; hp[k] = H[k][2]; }
       }
+      {
+        const R sp = za[0] + hm[0];
+        oc[0] = zb[0] + sp; oc[3] = za[0] - hm[0]; oc[6] = ((R)2 * sp - zb[0]) * third;
+        oc[2] = zb[1] + (za[1] + hm[1]); oc[9] = za[1] - hm[1];
+        oc[1] = zb[2] + (za[2] + hm[2]); oc[8] = za[2] - hm[2];
+        oc[4] = (zb[3] + hm[3]) * third; oc[5] = (zb[4] + hm[4]) * third; oc[7] = zb[5] + hm[5];
+      }
+      if constexpr (OB) {
+        oc[6] += zbz;
+        zbz = lbs[3];
+      }
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        za[k] = zn[k];
+        zb[k] = h0[k];
+        if constexpr (OB) zb[k] += lbs[k];
+      }
+#pragma unroll
+      for (int k = 3; k < 6; ++k) zb[k] = zn[k] + h0[k];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) zn[k] = hp[k];
       // ---- 6. plane zsrc-1 is complete (stored here, or by the next iteration) --
       if constexpr (!PF) {
         const int zo = zsrc - 1;
-        if (lane < XW && zo >= z0 && zo < zend) store_lo(zo, fs);
-#pragma unroll
-        for (int m = 0; m < 10; ++m) { lo[m] = mid[m]; mid[m] = hi[m]; }
+        if (lane < XW && zo >= z0 && zo < zend) store_oc(zo);
       }
     }
   }
   if constexpr (PF) {
-    if (out_row && lane < XW) store_lo(zend - 1, (size_t)sx);
+    if (out_row && lane < XW) store_oc(zend - 1);
   }
 }
 
 // One domain per launch: 1-D grid, XCD-aware tile order.
-template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY, bool OB, bool OPEN>
+template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY, bool OB, bool STD, bool OPEN>
 __global__ void __launch_bounds__((TY + 3) * 64) fused_kernel(FusedArgs a) {
-  fused_body<LAT, HO, PREC, TWO, INLINE, TY, OB, OPEN>(a, xcd_tile(blockIdx.x, fused_tiles<TY>(a)));
+  fused_body<LAT, HO, PREC, TWO, INLINE, TY, OB, STD, OPEN>(a, xcd_tile(blockIdx.x, fused_tiles<TY>(a)));
 }
 
 // Many domains per launch: the grid covers every domain's tiles in table
 // order (domain-major); a block finds its domain by binary search over the
 // tile offsets, then runs the same body on that domain's arguments.
-template <int LAT, bool HO, int PREC, bool TWO, int TY>
+template <int LAT, bool HO, int PREC, bool TWO, int TY, bool STD>
 __global__ void __launch_bounds__((TY + 3) * 64)
     fused_kernel_batch(const FusedBatchEntry* __restrict__ tab, int ndom, int total) {
   const int g = xcd_tile(blockIdx.x, total);
@@ -797,12 +945,12 @@ __global__ void __launch_bounds__((TY + 3) * 64)
     const int mid = (lo + hi + 1) >> 1;
     if (tab[mid].tile0 <= g) lo = mid; else hi = mid - 1;
   }
-  fused_body<LAT, HO, PREC, TWO, true, TY, false>(tab[lo].a, g - tab[lo].tile0);  // batches hold no obstacles
+  fused_body<LAT, HO, PREC, TWO, true, TY, false, STD>(tab[lo].a, g - tab[lo].tile0);  // batches hold no obstacles
 }
 
 // ---------------------------------------------------------------------------
-template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY>
-static hipError_t launch_t(const FusedArgs& a, hipStream_t s) {
+template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY, bool STD>
+static hipError_t launch_std(const FusedArgs& a, hipStream_t s) {
   dim3 grid(fused_tiles<TY>(a));
   dim3 block((TY + 3) * 64);
   // open faces reach the fast path with obstacles and 32/64-bit storage only
@@ -810,15 +958,24 @@ static hipError_t launch_t(const FusedArgs& a, hipStream_t s) {
   if (a.dp.obst) {
     if constexpr (open_ok) {
       if (a.sopen) {
-        hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, true, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, true, STD, true>), grid, block, 0, s, a);
         return hipGetLastError();
       }
     }
-    hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, true, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, true, STD, false>), grid, block, 0, s, a);
   } else {
-    hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((fused_kernel<LAT, HO, PREC, TWO, INLINE, TY, false, STD, false>), grid, block, 0, s, a);
   }
   return hipGetLastError();
+}
+
+template <int LAT, bool HO, int PREC, bool TWO, bool INLINE, int TY>
+static hipError_t launch_t(const FusedArgs& a, hipStream_t s) {
+  // the stage path's kernel has few switches left in it
+  if constexpr (INLINE) {
+    if (std_switches(a.dp)) return launch_std<LAT, HO, PREC, TWO, INLINE, TY, true>(a, s);
+  }
+  return launch_std<LAT, HO, PREC, TWO, INLINE, TY, false>(a, s);
 }
 
 template <int PREC, bool TWO, bool INLINE, int TY>
@@ -843,6 +1000,43 @@ static hipError_t launch_ty(const FusedArgs& a, hipStream_t s) {
   }
 }
 
+template <int PREC, bool TWO, int TY, bool STD>
+static hipError_t batch_lat(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, hipStream_t s) {
+  dim3 grid(total), block((TY + 3) * 64);
+  if (lat == 19) hipLaunchKernelGGL((fused_kernel_batch<19, false, PREC, TWO, TY, STD>), grid, block, 0, s, tab, ndom, total);
+  else if (ho) hipLaunchKernelGGL((fused_kernel_batch<27, true, PREC, TWO, TY, STD>), grid, block, 0, s, tab, ndom, total);
+  else hipLaunchKernelGGL((fused_kernel_batch<27, false, PREC, TWO, TY, STD>), grid, block, 0, s, tab, ndom, total);
+  return hipGetLastError();
+}
+
+template <int PREC, bool TWO, int TY>
+static hipError_t batch_std(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool std, hipStream_t s) {
+  return std ? batch_lat<PREC, TWO, TY, true>(tab, ndom, total, lat, ho, s)
+             : batch_lat<PREC, TWO, TY, false>(tab, ndom, total, lat, ho, s);
+}
+
+template <int PREC>
+hipError_t fused_batch_prec(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool two, bool std, int ty,
+                            hipStream_t s) {
+  if (ty == 8) return two ? batch_std<PREC, true, 8>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 8>(tab, ndom, total, lat, ho, std, s);
+  if (ty == 13) return two ? batch_std<PREC, true, 13>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 13>(tab, ndom, total, lat, ho, std, s);
+  return hipErrorInvalidValue;
+}
+
+template <int PREC>
+hipError_t fused_prec(const FusedArgs& a, bool inline_moments, hipStream_t s) {
+  if (inline_moments) return launch_ty<PREC, true>(a, s);
+  // the stage path stores 32 or 64 bits
+  if constexpr (PREC <= PREC_MIXED) return launch_ty<PREC, false>(a, s);
+  else return hipErrorInvalidValue;
+}
+
+template hipError_t fused_prec<LBF_FUSED_PREC>(const FusedArgs&, bool, hipStream_t);
+template hipError_t fused_batch_prec<LBF_FUSED_PREC>(const FusedBatchEntry*, int, int, int, bool, bool, bool, int,
+                                                         hipStream_t);
+
+#else  // the dispatch
+
 int fused_tile_count(const FusedArgs& a) {
   switch (a.ty) {
     case 8: return fused_tiles<8>(a);
@@ -851,35 +1045,18 @@ int fused_tile_count(const FusedArgs& a) {
   return -1;
 }
 
-template <int PREC, bool TWO, int TY>
-static hipError_t batch_lat(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, hipStream_t s) {
-  dim3 grid(total), block((TY + 3) * 64);
-  if (lat == 19) hipLaunchKernelGGL((fused_kernel_batch<19, false, PREC, TWO, TY>), grid, block, 0, s, tab, ndom, total);
-  else if (ho) hipLaunchKernelGGL((fused_kernel_batch<27, true, PREC, TWO, TY>), grid, block, 0, s, tab, ndom, total);
-  else hipLaunchKernelGGL((fused_kernel_batch<27, false, PREC, TWO, TY>), grid, block, 0, s, tab, ndom, total);
-  return hipGetLastError();
-}
-
-template <int PREC>
-static hipError_t batch_prec(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool two, int ty,
-                             hipStream_t s) {
-  if (ty == 8) return two ? batch_lat<PREC, true, 8>(tab, ndom, total, lat, ho, s) : batch_lat<PREC, false, 8>(tab, ndom, total, lat, ho, s);
-  if (ty == 13) return two ? batch_lat<PREC, true, 13>(tab, ndom, total, lat, ho, s) : batch_lat<PREC, false, 13>(tab, ndom, total, lat, ho, s);
-  return hipErrorInvalidValue;
-}
-
 hipError_t launch_fused_batch(const FusedBatchEntry* dev_tab, int ndom, int total_tiles, int prec, int lattice,
-                              bool highorder, bool two, int ty, hipStream_t s) {
+                              bool highorder, bool two, bool std, int ty, hipStream_t s) {
   switch (prec) {
     case PREC_FP16S | PREC_DEFSCALE:
-      return batch_prec<PREC_FP16S | PREC_DEFSCALE>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
+      return fused_batch_prec<PREC_FP16S | PREC_DEFSCALE>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
     case PREC_BF16S | PREC_DEFSCALE:
-      return batch_prec<PREC_BF16S | PREC_DEFSCALE>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
-    case PREC_FP64: return batch_prec<PREC_FP64>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
-    case PREC_FP32: return batch_prec<PREC_FP32>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
-    case PREC_MIXED: return batch_prec<PREC_MIXED>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
-    case PREC_FP16S: return batch_prec<PREC_FP16S>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
-    case PREC_BF16S: return batch_prec<PREC_BF16S>(dev_tab, ndom, total_tiles, lattice, highorder, two, ty, s);
+      return fused_batch_prec<PREC_BF16S | PREC_DEFSCALE>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
+    case PREC_FP64: return fused_batch_prec<PREC_FP64>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
+    case PREC_FP32: return fused_batch_prec<PREC_FP32>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
+    case PREC_MIXED: return fused_batch_prec<PREC_MIXED>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
+    case PREC_FP16S: return fused_batch_prec<PREC_FP16S>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
+    case PREC_BF16S: return fused_batch_prec<PREC_BF16S>(dev_tab, ndom, total_tiles, lattice, highorder, two, std, ty, s);
   }
   return hipErrorInvalidValue;
 }
@@ -891,25 +1068,19 @@ bool default_scales(const DevParams& dp) {
 }
 
 hipError_t launch_fused(const FusedArgs& a, int prec, bool inline_moments, hipStream_t s) {
-  if (inline_moments) {
-    const bool ds = default_scales(a.dp);
-    switch (prec) {
-      case PREC_FP64: return launch_ty<PREC_FP64, true>(a, s);
-      case PREC_FP32: return launch_ty<PREC_FP32, true>(a, s);
-      case PREC_MIXED: return launch_ty<PREC_MIXED, true>(a, s);
-      case PREC_FP16S:
-        return ds ? launch_ty<PREC_FP16S | PREC_DEFSCALE, true>(a, s) : launch_ty<PREC_FP16S, true>(a, s);
-      case PREC_BF16S:
-        return ds ? launch_ty<PREC_BF16S | PREC_DEFSCALE, true>(a, s) : launch_ty<PREC_BF16S, true>(a, s);
-    }
-  } else {
-    switch (prec) {
-      case PREC_FP64: return launch_ty<PREC_FP64, false>(a, s);
-      case PREC_FP32: return launch_ty<PREC_FP32, false>(a, s);
-      case PREC_MIXED: return launch_ty<PREC_MIXED, false>(a, s);
-    }
+  if ((prec == PREC_FP16S || prec == PREC_BF16S) && default_scales(a.dp)) prec |= PREC_DEFSCALE;
+  switch (prec) {
+    case PREC_FP64: return fused_prec<PREC_FP64>(a, inline_moments, s);
+    case PREC_FP32: return fused_prec<PREC_FP32>(a, inline_moments, s);
+    case PREC_MIXED: return fused_prec<PREC_MIXED>(a, inline_moments, s);
+    case PREC_FP16S: return fused_prec<PREC_FP16S>(a, inline_moments, s);
+    case PREC_BF16S: return fused_prec<PREC_BF16S>(a, inline_moments, s);
+    case PREC_FP16S | PREC_DEFSCALE: return fused_prec<PREC_FP16S | PREC_DEFSCALE>(a, inline_moments, s);
+    case PREC_BF16S | PREC_DEFSCALE: return fused_prec<PREC_BF16S | PREC_DEFSCALE>(a, inline_moments, s);
   }
   return hipErrorInvalidValue;
 }
+
+#endif
 
 }  // namespace lbf

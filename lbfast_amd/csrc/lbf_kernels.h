@@ -15,7 +15,7 @@ struct FusedArgs {
   void* phiout;      // phase field O
   const void* pre;   // 5-field set: grad phi (3, as n*|g|), lap phi, div(theta n) (inline)
   const void* frc;   // forces: 3-field set (stage path)
-  const int8_t* isfh;  // isfluid with 1-node halo
+  const uint32_t* words;  // obstacles: a word per node of the haloed isfluid (NODE_FLUID, lbf_physics.h)
   DevParams dp;
   int ty, tz;        // tile rows, z-chunk length
   // 16-bit storage: the step's stochastic-rounding seed is seed (+ *seedp
@@ -64,6 +64,15 @@ inline bool fused_grad_inline(int prec, const DevParams& dp) {
   return (prec == PREC_FP32 || prec == PREC_FP16S || prec == PREC_BF16S) && dp.twocomp && !dp.obst;
 }
 
+// The switches of every two-component configuration as the reference's
+// defines.h sets them (INTERFACE_INCOMP follows DENSRATIO), or of a plain
+// one-component run: the fast path's kernels have them compiled in, which
+// takes their branches and scalar state out of the plane loop; other settings
+// take the kernels that read the switches.
+inline bool std_switches(const DevParams& dp) {
+  return !dp.smag && (!dp.twocomp || (dp.dens && dp.incomp && !dp.buoy));
+}
+
 // Batched launches: one grid over many domains (same lattice, precision,
 // component count and row tile; any sizes and physical parameters).
 struct FusedBatchEntry {
@@ -81,10 +90,13 @@ hipError_t launch_fused(const FusedArgs& a, int prec, bool inline_moments, hipSt
 bool default_scales(const DevParams& dp);
 int fused_tile_count(const FusedArgs& a);
 // prec may carry PREC_DEFSCALE (every domain with the default 16-bit scales)
+// std: std_switches() holds for every domain
 hipError_t launch_fused_batch(const FusedBatchEntry* dev_tab, int ndom, int total_tiles, int prec, int lattice,
-                              bool highorder, bool two, int ty, hipStream_t s);
+                              bool highorder, bool two, bool std, int ty, hipStream_t s);
 int prep_tile_count(const StageArgs& a, int prec, int tz);
 hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int total_tiles, int prec, hipStream_t s);
+// the fused kernel's words from the haloed isfluid
+hipError_t launch_node_words(const int8_t* isfh, uint32_t* words, const DevParams& dp, hipStream_t s);
 hipError_t launch_stage(int stage, const StageArgs& a, int prec, hipStream_t s);
 
 // storage conversion: host-order double/float array -> field (codec-aware)

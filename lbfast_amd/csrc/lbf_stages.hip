@@ -547,6 +547,30 @@ __global__ void __launch_bounds__(QNT)
 }
 
 // ---------------------------------------------------------------------------
+// The fused kernel's word of each haloed node (lbf_physics.h), once per
+// uploaded isfluid.
+__global__ void __launch_bounds__(BS) k_node_words(const int8_t* isfh, uint32_t* words, DevParams dp) {
+  const size_t t = (size_t)blockIdx.x * BS + threadIdx.x;
+  if (t >= halo_nodes(dp)) return;
+  const int hx = dp.nx + 2, hy = dp.ny + 2;
+  const int x = (int)(t % hx) - 1, y = (int)(t / hx % hy) - 1, z = (int)(t / hx / hy) - 1;
+  const int8_t isf = isfh[t];
+  uint32_t w = isf == 0 ? 0u : isf == -1 ? NODE_FLUID | NODE_WALL : NODE_FLUID;
+  if (isf == -1) {
+    for (int c = 0; c < 27; ++c) {
+      const int p = c % 3 - 1, q = (c / 3) % 3 - 1, r = c / 9 - 1;
+      if (c != 13 && isf_at(isfh, x - p, y - q, z - r, dp.nx, dp.ny, dp.nz) == 0) w |= 1u << c;
+    }
+  }
+  words[t] = w;
+}
+
+hipError_t launch_node_words(const int8_t* isfh, uint32_t* words, const DevParams& dp, hipStream_t s) {
+  hipLaunchKernelGGL(k_node_words, dim3((unsigned)((halo_nodes(dp) + BS - 1) / BS)), dim3(BS), 0, s, isfh, words, dp);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 template <int PREC>
 __global__ void __launch_bounds__(BS) k_phi_bnd(StageArgs a) {
   typedef typename Codec<PREC>::R R;
