@@ -293,8 +293,9 @@ int lbf_batch_set_tile(lbf_batch* b, int32_t tile_y, int32_t tile_z, int32_t til
  * permutation of 0..ndomains-1.  Results do not depend on it. */
 int lbf_batch_set_order(lbf_batch* b, const int32_t* order);
 /* Time trial_steps (even) steps of each candidate on the batch itself, keep
- * the fastest and restore every domain's state.  Searched in turn: the row
- * tile with one z chunk for all domains (reported in tile_y, tile_z); the z
+ * the fastest and restore every domain's state.  Searched in turn: the tiles
+ * as they are and the row tiles with one z chunk for all domains (tile_y: the row
+ * tile kept, tile_z: the fastest of the common chunks); the z
  * chunk of each size class (domains of one nz); the table order (as given,
  * largest first, largest and smallest alternating). */
 int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* tile_y, int32_t* tile_z);

@@ -26,6 +26,7 @@ struct lbf_ctx {
   int prec = 0;
   hipStream_t stream = nullptr;
   int device = 0;
+  int ncu = 256;  // compute units
   size_t N = 0;
   size_t NS = 0;   // values per field of a field set: sx*ny*nz (row-interleaved sets)
   size_t tsz = 0;  // bytes of one moment value
@@ -232,36 +233,65 @@ void lbf_destroy(lbf_ctx* c) {
   delete c;
 }
 
+// z chunk of a z-marching grid of `tiles` x-y tiles: the one with the least
+// makespan, counted in planes.  A block of tz planes marches tz + extra (halo
+// planes of the march and the prologue); t[k - 1] is a plane's time with k
+// blocks on every CU (nt at most), in units of t[0].  Chunks of ceil(nz / c)
+// planes; of equals the longest, which repeats fewest halo planes.
+static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t, int nt, int* tz_out) {
+  double best = 1e300;
+  int last = 0;
+  for (int c = 1; c <= nz; ++c) {
+    const int tz = (nz + c - 1) / c;
+    if (tz == last) continue;
+    last = tz;
+    const long n = tiles * ((nz + tz - 1) / tz), slots = (long)ncu * nt;
+    const long rest = n % slots;
+    const double rounds = (double)(n / slots) * t[nt - 1] + (rest ? t[(rest + ncu - 1) / ncu - 1] : 0.0);
+    const double cost = rounds * (tz + extra);
+    if (cost < best * 0.999) {
+      best = cost;
+      *tz_out = tz;
+    }
+  }
+  return best;
+}
+
+// One block of the fused kernel fits a CU.  A plane of an 8-row block takes
+// 0.72 of a 13-row block's time (measured 0.66 at 512^3, where HBM counts, to
+// 0.81 at 64^3); with 64-bit arithmetic the 13-row block's 128 registers a lane
+// spill and 8 rows are always the faster (160^3: FP64 311 against 560 us,
+// MIXED 219 against 404).
+static const double T_FUSED[1] = {1.0};
+constexpr int FUSED_EXTRA = 3;
+constexpr double T8 = 0.72;
+static long fused_xy(const lbf_params& p, int ty) { return (long)((p.nx + 63) / 64) * ((p.ny + ty - 1) / ty); }
+static bool rows8_only(int prec) { return prec == LBF_PREC_FP64 || prec == LBF_PREC_MIXED; }
+// Three blocks of the 16/32-bit phase prep fit a CU (measured plane times 1.65,
+// 2.2, 2.9 us with one to three), two of the FP64 prep.
+static const double T_PREP[3] = {1.0, 1.34, 1.75};
+static const double T_PREP64[2] = {1.0, 1.5};
+
+// Chunks that fill the CUs in whole rounds.  The rule before aimed at 1024
+// blocks and at least 8 planes a chunk, which left small domains a serial march
+// (32^3: 12 blocks of 10 planes) and others a last round that is nearly empty
+// (256^3: 1040 blocks, 4.06 rounds).  Fused kernel, old and new chunks:
+// 32^3 36.8 -> 17.9 us, 64^3 46.8 -> 22.2, 128^3 92.5 -> 62.2, 201x130x117
+// 149 -> 113, 256^3 FP16S 435 -> 353, 160^3 FP64 678 -> 311.
 static void default_tiles(lbf_ctx* c) {
-  // rows per block: 8 or 13, whichever needs fewer waves for the y extent
-  // (a block of ty rows runs ty + 3 waves: two halo rows and the x-halo wave)
-  const long w8 = (long)((c->p.ny + 7) / 8) * 11, w13 = (long)((c->p.ny + 12) / 13) * 16;
-  c->ty = w13 < w8 ? 13 : 8;
-  // z-chunks so the grid holds ~1024 blocks (4 per CU, one resident at a time)
-  const long bxy = (long)((c->p.nx + 63) / 64) * ((c->p.ny + c->ty - 1) / c->ty);
-  long nchunks = (1024 + bxy - 1) / bxy;
-  if (nchunks < 1) nchunks = 1;
-  long tz = (c->p.nz + nchunks - 1) / nchunks;
-  if (tz < 8) tz = 8;
-  if (tz > c->p.nz) tz = c->p.nz;
-  c->tz = (int)tz;
-  // phase prep: z-chunks so the grid holds at least ~2048 blocks. The 64 x 12
-  // tiles of the 16/32-bit prep take chunks of 16..32 planes (measured at
-  // 512^3: 1.27 ms with 32 planes against 1.38 ms with 128; each chunk re-reads
-  // 4 planes of phi and recomputes 2 planes of theta); the FP64 prep's 64 x 8
-  // tiles take chunks of at least 8
+  int tz8 = 1, tz13 = 1;
+  const double c8 = T8 * pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
+  const double c13 = pick_chunk(fused_xy(c->p, 13), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz13);
+  const bool r8 = rows8_only(c->prec) || c8 < c13;
+  c->ty = r8 ? 8 : 13;
+  c->tz = r8 ? tz8 : tz13;
+  // prep blocks: 64 x 12 tiles that march 5 planes beyond their chunk (theta and
+  // phi halo planes, one step of store lag); the FP64 prep's 64 x 8 tiles 2
   StageArgs one{};
   one.dp = c->dp;
   const long pt = prep_tile_count(one, c->prec, c->p.nz);
-  const bool tiles_z = pt > 0;
-  const long pxy = tiles_z ? pt : (long)((c->p.nx + 63) / 64) * ((c->p.ny + 7) / 8);
-  long pch = (2048 + pxy - 1) / pxy;
-  if (pch < 1) pch = 1;
-  long tzp = (c->p.nz + pch - 1) / pch;
-  if (tiles_z && tzp > 32) tzp = 32;
-  if (tzp < (tiles_z ? 16 : 8)) tzp = tiles_z ? 16 : 8;
-  if (tzp > c->p.nz) tzp = c->p.nz;
-  c->tz_prep = (int)tzp;
+  if (pt > 0) pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP, 3, &c->tz_prep);
+  else pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, 2, T_PREP64, 2, &c->tz_prep);
 }
 
 int lbf_create(const lbf_params* pin, lbf_ctx** out) {
@@ -323,6 +353,7 @@ int lbf_create(const lbf_params* pin, lbf_ctx** out) {
   c->p = p;
   c->prec = p.precision;
   c->device = dev;
+  c->ncu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
   fill_devparams(c);
   c->N = (size_t)p.nx * p.ny * p.nz;
   c->NS = (size_t)set_sx(p.nx) * p.ny * p.nz;
@@ -1025,6 +1056,39 @@ static void batch_advance(lbf_batch* b, int nsteps) {
   }
 }
 
+// The chunk length T (clipped to each domain) and row tile with the least
+// estimated makespan: all planes marched over the CUs, plus half a longest block
+// for the uneven end of the grid.
+static void batch_default_tiles(lbf_batch* b) {
+  const int ncu = b->ctx[0]->ncu;
+  auto chunk = [](int nz, int T) { return (nz + (nz + T - 1) / T - 1) / ((nz + T - 1) / T); };
+  auto search = [&](int rows, int extra, double slots, int* Tbest) {
+    double best = 1e300;
+    for (int T = 1; T <= 128; ++T) {
+      double work = 0, longest = 0;
+      for (lbf_ctx* c : b->ctx) {
+        const int tz = chunk(c->p.nz, T);
+        work += (double)fused_xy(c->p, rows) * ((c->p.nz + tz - 1) / tz) * (tz + extra);
+        longest = std::max(longest, (double)(tz + extra));
+      }
+      const double est = std::max(work / (ncu * slots) + 0.5 * longest, longest);
+      if (est < best * 0.999) { best = est; *Tbest = T; }
+    }
+    return best;
+  };
+  int T8b = 1, T13b = 1, Tp = 1;
+  const double c8 = T8 * search(8, FUSED_EXTRA, 1, &T8b), c13 = search(13, FUSED_EXTRA, 1, &T13b);
+  const bool r8 = rows8_only(b->prec) || c8 < c13;
+  b->ty = r8 ? 8 : 13;
+  search(12, 5, 3, &Tp);
+  b->tz.clear();
+  b->tz_prep.clear();
+  for (lbf_ctx* c : b->ctx) {
+    b->tz.push_back(chunk(c->p.nz, r8 ? T8b : T13b));
+    b->tz_prep.push_back(chunk(c->p.nz, Tp));
+  }
+}
+
 int lbf_batch_create(lbf_ctx* const* ctxs, int32_t ndomains, lbf_batch** out) {
   if (!ctxs || !out || ndomains < 1) return bfail(nullptr, LBF_EINVAL, "bad arguments");
   *out = nullptr;
@@ -1049,11 +1113,7 @@ int lbf_batch_create(lbf_ctx* const* ctxs, int32_t ndomains, lbf_batch** out) {
   b->lattice = c0->p.lattice;
   b->ho = c0->dp.highorder != 0;
   b->two = c0->p.twocomponent != 0;
-  b->ty = 13;
-  for (lbf_ctx* c : b->ctx) {
-    b->tz.push_back(c->p.nz < 32 ? c->p.nz : 32);
-    b->tz_prep.push_back(c->p.nz < 32 ? c->p.nz : 32);
-  }
+  batch_default_tiles(b);
   for (int d = 0; d < ndomains; ++d) b->order.push_back(d);
   bool ok = hipStreamCreate(&b->stream) == hipSuccess && hipEventCreate(&b->t0) == hipSuccess &&
             hipEventCreate(&b->t1) == hipSuccess && hipMalloc(&b->ctr, ndomains * sizeof(uint32_t)) == hipSuccess;
@@ -1207,8 +1267,8 @@ int lbf_batch_timing(lbf_batch* b, double* ms) {
 
 // The project's autotuner: times `trial_steps` (even) steps of each candidate
 // on the batch itself, keeps the fastest, and restores every domain's state
-// afterwards.  Candidates, searched in turn: the row tile (8 or 13) with one z
-// chunk (16..128) for every domain; then the z chunk of each size class
+// afterwards.  Candidates, searched in turn: the tiles as they are, or a row tile
+// (8 or 13) with one z chunk (16..128) for every domain; then the z chunk of each size class
 // (domains of one nz) with the others held; then the table order (as given,
 // largest first, or largest and smallest alternating).
 int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int32_t* best_tz) {
@@ -1261,10 +1321,15 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
     }
   };
   batch_drop_graph(b);
-  // 1. row tile and one z chunk for every domain
+  // 1. the current tiles, or a row tile and one z chunk for every domain
   const int tys[2] = {8, 13}, tzs[4] = {16, 32, 64, 128};
-  double best = 1e300;
-  int bty = b->ty, btz = b->tz.empty() ? 32 : b->tz[0];
+  const std::vector<int> tz0 = b->tz, tzp0 = b->tz_prep;
+  double best = 1e300, ubest = 1e300;
+  int bty = b->ty, btz = 0, utz = tzs[0];  // utz: the fastest uniform chunk, reported
+  {
+    int rc = trial(&best);
+    if (rc) { release(); return rc; }
+  }
   for (int ty : tys)
     for (int tz : tzs) {
       b->ty = ty;
@@ -1272,10 +1337,16 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
       double m = 0;
       int rc = trial(&m);
       if (rc) { release(); return rc; }
+      if (m < ubest) { ubest = m; utz = tz; }
       if (m < best) { best = m; bty = ty; btz = tz; }
     }
   b->ty = bty;
-  set_uniform(btz);
+  if (btz) {
+    set_uniform(btz);
+  } else {
+    b->tz = tz0;
+    b->tz_prep = tzp0;
+  }
   // 2. the z chunk of each size class (domains of one nz), the others held:
   // short domains lose least to the chunks' two halo planes with one chunk,
   // tall ones may balance better with more
@@ -1288,7 +1359,7 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
       int keep = -1;
       for (int tz : cand) {
         if (tz > nz) continue;
-        std::vector<int> save = b->tz;
+        const std::vector<int> save = b->tz, save_p = b->tz_prep;
         for (int d = 0; d < nd; ++d)
           if (b->ctx[d]->p.nz == nz) b->tz[d] = b->tz_prep[d] = tz;
         double m = 0;
@@ -1296,7 +1367,7 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
         if (rc) { release(); return rc; }
         if (m < best * 0.995) { best = m; keep = tz; }
         b->tz = save;
-        b->tz_prep = save;
+        b->tz_prep = save_p;
       }
       if (keep > 0)
         for (int d = 0; d < nd; ++d)
@@ -1339,7 +1410,7 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
   int rc = batch_tables(b);
   if (rc) return rc;
   if (best_ty) *best_ty = b->ty;
-  if (best_tz) *best_tz = btz;
+  if (best_tz) *best_tz = utz;
   b->timing_valid = false;
   return LBF_OK;
 }
