@@ -41,6 +41,9 @@ struct lbf_ctx {
   void* pre = nullptr;  // 5-field set (fast path phase-field prep)
   void* sopen = nullptr;  // open faces: post-moments state of the fast path (10-field set)
   int8_t* isfh = nullptr;
+  void* wet = nullptr;         // WetNode list (obstacles, two components)
+  uint32_t nwet = 0;
+  uint32_t* wet_count = nullptr;
   uint32_t* words = nullptr;  // obstacles: the fused kernel's word per haloed node
   void* rep = nullptr;         // REPULSIVE_FLUX: locaux 3..8 (6-field set)
   int8_t* rep_mask = nullptr;  // REPULSIVE_FLUX
@@ -226,6 +229,7 @@ void lbf_destroy(lbf_ctx* c) {
   if (!c) return;
   if (c->stream) hipStreamSynchronize(c->stream);
   for (void* p : c->allocs) hipFree(p);
+  if (c->wet) hipFree(c->wet);
   for (hipEvent_t e : c->evs) hipEventDestroy(e);
   if (c->t0) hipEventDestroy(c->t0);
   if (c->t1) hipEventDestroy(c->t1);
@@ -389,6 +393,7 @@ int lbf_create(const lbf_params* pin, lbf_ctx** out) {
   }
   c->isfh = (int8_t*)A((size_t)(p.nx + 2) * (p.ny + 2) * (p.nz + 2));
   if (p.internal_obstacles) c->words = (uint32_t*)A((size_t)(p.nx + 2) * (p.ny + 2) * (p.nz + 2) * sizeof(uint32_t));
+  if (p.internal_obstacles && p.twocomponent) c->wet_count = (uint32_t*)A(sizeof(uint32_t));
   c->staging = A(c->N * 8);
   c->nred = REDUCE_SCRATCH_BLOCKS;  // the no-alloc variant's partials match this launch
   c->partial = (double*)A((size_t)c->nred * 8 * sizeof(double));
@@ -586,10 +591,27 @@ int lbf_upload_isfluid(lbf_ctx* c, const int8_t* host) {
             one ? 1 : host[(size_t)c3[0] + (size_t)nx * ((size_t)c3[1] + (size_t)ny * c3[2])];
       }
   HIPCHK(c, hipMemcpy(c->isfh, h.data(), h.size(), hipMemcpyHostToDevice));
-  if (c->words) {
-    HIPCHK(c, launch_node_words(c->isfh, c->words, c->dp, c->stream));
+  if (c->words) HIPCHK(c, launch_node_words(c->isfh, c->words, c->dp, c->stream));
+  if (c->wet_count) {
+    // the wetting list: count, allocate, write (an empty one for no solid node)
+    c->nwet = 0;
+    uint32_t n = 0;
+    if (any_solid) {
+      HIPCHK(c, launch_fill_zero(c->wet_count, sizeof n, c->stream));
+      HIPCHK(c, launch_wet_list(c->isfh, nullptr, c->wet_count, c->dp, c->prec, c->stream));
+      HIPCHK(c, hipMemcpyAsync(&n, c->wet_count, sizeof n, hipMemcpyDeviceToHost, c->stream));
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (c->wet) HIPCHK(c, hipFree(c->wet));
+    c->wet = nullptr;
+    if (n) {
+      HIPCHK(c, hipMalloc(&c->wet, (size_t)n * wet_node_size(c->prec)));
+      HIPCHK(c, launch_fill_zero(c->wet_count, sizeof n, c->stream));
+      HIPCHK(c, launch_wet_list(c->isfh, c->wet, c->wet_count, c->dp, c->prec, c->stream));
+    }
+    c->nwet = n;
   }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->isf_set = true;
   return LBF_OK;
 }
@@ -612,6 +634,8 @@ static StageArgs stage_args(lbf_ctx* c) {
   a.rep = c->rep;
   a.rep_mask = c->rep_mask;
   a.isfh = c->isfh;
+  a.wet = c->wet;
+  a.nwet = c->nwet;
   a.dp = c->dp;
   a.obc = c->p.openbc != 0 && c->p.internal_obstacles != 0;
   for (int f = 0; f < 6; ++f) {

@@ -28,6 +28,16 @@ struct FusedArgs {
   void* sopen;
 };
 
+// A solid node whose phi the wetting update sets (PHI_int_boundary): all of it
+// that isfluid alone decides.
+template <class R>
+struct WetNode {
+  R wx, wy, wz;           // wall normal
+  uint32_t n, d;          // the node and its donor (x-fastest indices)
+  int8_t sx, sy, sz;      // donor to node
+  int8_t zero;            // the donor lies where the reference reads zeros: the ghost is 0
+};
+
 // Stage-path buffers (the reference's per-kernel arguments), as field sets.
 struct StageArgs {
   void* S;           // 10-field set
@@ -46,6 +56,8 @@ struct StageArgs {
   void* rep;         // REPULSIVE_FLUX: 6-field set, locaux 3..8 (partner index, flux)
   int8_t* rep_mask;  // REPULSIVE_FLUX: nx*ny*nz
   const int8_t* isfh;
+  const void* wet;   // WetNode<R> list of PHI_int_boundary
+  uint32_t nwet;
   DevParams dp;
   // open boundaries (openbc = 1): faces x(1) x(2) y(1) y(2) z(1) z(2), each
   // with its type (0 velocity, 1 pressure, 2 the node's own values) and its
@@ -95,6 +107,12 @@ hipError_t launch_fused_batch(const FusedBatchEntry* dev_tab, int ndom, int tota
                               bool highorder, bool two, bool std, int ty, hipStream_t s);
 int prep_tile_count(const StageArgs& a, int prec, int tz);
 hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int total_tiles, int prec, hipStream_t s);
+// the WetNode list from the haloed isfluid: counts the nodes into *count (list
+// null) or writes them
+hipError_t launch_wet_list(const int8_t* isfh, void* list, uint32_t* count, const DevParams& dp, int prec, hipStream_t s);
+inline size_t wet_node_size(int prec) {
+  return prec == PREC_FP64 || prec == PREC_MIXED ? sizeof(WetNode<double>) : sizeof(WetNode<float>);
+}
 // the fused kernel's words from the haloed isfluid
 hipError_t launch_node_words(const int8_t* isfh, uint32_t* words, const DevParams& dp, hipStream_t s);
 hipError_t launch_stage(int stage, const StageArgs& a, int prec, hipStream_t s);

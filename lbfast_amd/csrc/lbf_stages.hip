@@ -1,10 +1,11 @@
 // lbf_stages.hip -- the reference's per-stage kernels for gfx950 (one thread
-// per node, row-interleaved field sets, in-kernel periodic wrap), the tiled phase-field
+// per node they work on, row-interleaved field sets, in-kernel periodic wrap), the tiled phase-field
 // prep kernel of the fast path, and the encode/decode/reduction helpers.
 //
 //   k_norm        compute_norm_interface_kernel (lb_cuda_auxfields_module.f90:19-139)
 //   k_div         compute_div_theta_n_kernel    (lb_cuda_auxfields_module.f90:1085-1164)
-//   k_phi_bnd     PHI_int_boundary_kernel       (lb_cuda_boundary_module.f90:218-459)
+//   k_phi_bnd     PHI_int_boundary_kernel       (lb_cuda_boundary_module.f90:218-459),
+//                 over the list that k_wet_list lays out
 //   k_moments     moments_LB_kernel             (lb_cuda_moments_module.f90:19-341)
 //   k_update_phi  update_phifields_kernel       (lb_cuda_update_phi_module.f90:19-104)
 //   k_lb_int_bnd  LB_int_boundary_kernel        (lb_cuda_boundary_module.f90:19-216)
@@ -571,89 +572,119 @@ hipError_t launch_node_words(const int8_t* isfh, uint32_t* words, const DevParam
 }
 
 // ---------------------------------------------------------------------------
-template <int PREC>
-__global__ void __launch_bounds__(BS) k_phi_bnd(StageArgs a) {
-  typedef typename Codec<PREC>::R R;
-  typedef typename Aux<PREC>::T TA;
-  const DevParams& dp = a.dp;
-  int x, y, z;
-  if (!node_of((size_t)blockIdx.x * BS + threadIdx.x, dp, x, y, z)) return;
+// Wetting (PHI_int_boundary, boundary:218-459).  The wall normal of a solid
+// node and its donor depend on isfluid alone, and few nodes have any: the list
+// of them is laid out once per uploaded isfluid, and the update runs a thread
+// per listed node.  A thread per node of the domain that gathered up to 52
+// neighbours in most waves took 207 us at 256x128x128 (25% spheres) and 662 us
+// at 384x192x192; from the list it takes 16 and 47 us (1.3 million nodes).
+template <class R>
+__device__ __forceinline__ bool wet_node(const int8_t* isfh, const DevParams& dp, int x, int y, int z, WetNode<R>& o) {
   const int nx = dp.nx, ny = dp.ny, nz = dp.nz;
-  if (isf_at(a.isfh, x, y, z, nx, ny, nz) != 0) return;
+  if (isf_at(isfh, x, y, z, nx, ny, nz) != 0) return false;
   const int nl = dp.lattice == 27 ? 27 : 19;
-  const R eps_norm = (R)1.0e-14, huge_cot = (R)1.0e14;
+  const R eps_norm = (R)1.0e-14;
   const R inv_sqrt2 = (R)0.70710678118654752440, inv_sqrt3 = (R)0.57735026918962576450;
   const R half_val = (R)0.5, third_val = (R)(1.0 / 3.0);
-  const R pi = (R)3.1415926535897932384626433832795028841971;
-  const int sx = dp.sx;
-  TA* ph = (TA*)a.phiS;
-  const size_t n = nidx(x, y, z, nx, ny);
-  R ghost = (R)ph[n];
   R wnx = 0, wny = 0, wnz = 0;
   for (int l = 1; l < nl; ++l) {
     const int d2 = cEX[l] * cEX[l] + cEY[l] * cEY[l] + cEZ[l] * cEZ[l];
-    if (isf_at(a.isfh, x + cEX[l], y + cEY[l], z + cEZ[l], nx, ny, nz) == 0) continue;
+    if (isf_at(isfh, x + cEX[l], y + cEY[l], z + cEZ[l], nx, ny, nz) == 0) continue;
     const R s = d2 == 1 ? (R)1 : (d2 == 2 ? half_val : third_val);
     wnx = wnx + s * (-(R)cEX[l]);
     wny = wny + s * (-(R)cEY[l]);
     wnz = wnz + s * (-(R)cEZ[l]);
   }
   const R wn = sqrt(wnx * wnx + wny * wny + wnz * wnz);
-  if (wn < eps_norm) return;
+  if (wn < eps_norm) return false;
   wnx = wnx / wn; wny = wny / wn; wnz = wnz / wn;
   R best = (R)-1.0e30;
-  int dx = 0, dy = 0, dz = 0;
-  bool have = false;
-  R bsx = 0, bsy = 0, bsz = 0;
+  int dx = 0, dy = 0, dz = 0, bl = 0;
   for (int l = 1; l < nl; ++l) {
     const int d2 = cEX[l] * cEX[l] + cEY[l] * cEY[l] + cEZ[l] * cEZ[l];
     const int xi = x + cEX[l], yj = y + cEY[l], zk = z + cEZ[l];
-    const int8_t v = isf_at(a.isfh, xi, yj, zk, nx, ny, nz);
+    const int8_t v = isf_at(isfh, xi, yj, zk, nx, ny, nz);
     if (v != 1 && v != -1) continue;
     const R s = d2 == 1 ? (R)1 : (d2 == 2 ? inv_sqrt2 : inv_sqrt3);
     const R sx = -(R)cEX[l], sy = -(R)cEY[l], sz = -(R)cEZ[l];
     const R score = (sx * wnx + sy * wny + sz * wnz) * s;
-    if (score > best) {
-      best = score; dx = xi; dy = yj; dz = zk; bsx = sx; bsy = sy; bsz = sz; have = true;
-    }
+    if (score > best) { best = score; dx = xi; dy = yj; dz = zk; bl = l; }
   }
   // the reference skips a donor with a zero (1-based) coordinate, i.e. one in
   // the lower halo (boundary:395); 0-based that is -1
-  if (!have || dx == -1 || dy == -1 || dz == -1) return;
+  if (bl == 0 || dx == -1 || dy == -1 || dz == -1) return false;
+  o.wx = wnx; o.wy = wny; o.wz = wnz;
+  o.n = (uint32_t)nidx(x, y, z, nx, ny);
+  o.d = (uint32_t)nidx(wrapg(dx, nx), wrapg(dy, ny), wrapg(dz, nz), nx, ny);
+  o.sx = (int8_t)-cEX[bl]; o.sy = (int8_t)-cEY[bl]; o.sz = (int8_t)-cEZ[bl];
   // a donor past an upper non-periodic face (isfluid 1 there) lies in the
   // reference's halo, which nothing writes on such an axis: phi and its
   // gradient read zero, so the ghost is 0 + 0 (the donor search picks such a
   // node only where two walls meet: on a plane wall the halo's and the
   // fluid's pulls on the wall normal cancel)
-  if ((!dp.pbc[0] && dx == nx) || (!dp.pbc[1] && dy == ny) || (!dp.pbc[2] && dz == nz)) {
-    ph[n] = (TA)0;
+  o.zero = (!dp.pbc[0] && dx == nx) || (!dp.pbc[1] && dy == ny) || (!dp.pbc[2] && dz == nz);
+  return true;
+}
+
+template <class R>
+__global__ void __launch_bounds__(BS) k_wet_list(const int8_t* isfh, WetNode<R>* list, uint32_t* count, DevParams dp) {
+  int x, y, z;
+  WetNode<R> w;
+  const bool have = node_of((size_t)blockIdx.x * BS + threadIdx.x, dp, x, y, z) && wet_node(isfh, dp, x, y, z, w);
+  const uint64_t m = __ballot(have);
+  if (m == 0) return;
+  const int lane = threadIdx.x & 63;
+  uint32_t base = 0;
+  if (lane == 0) base = atomicAdd(count, (uint32_t)__popcll(m));
+  base = __shfl(base, 0);
+  if (have && list) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = w;
+}
+
+hipError_t launch_wet_list(const int8_t* isfh, void* list, uint32_t* count, const DevParams& dp, int prec, hipStream_t s) {
+  const dim3 grid((unsigned)((dp.nn + BS - 1) / BS)), block(BS);
+  if (prec == PREC_FP64 || prec == PREC_MIXED)
+    hipLaunchKernelGGL(k_wet_list<double>, grid, block, 0, s, isfh, (WetNode<double>*)list, count, dp);
+  else
+    hipLaunchKernelGGL(k_wet_list<float>, grid, block, 0, s, isfh, (WetNode<float>*)list, count, dp);
+  return hipGetLastError();
+}
+
+template <int PREC>
+__global__ void __launch_bounds__(BS) k_phi_bnd(StageArgs a) {
+  typedef typename Codec<PREC>::R R;
+  typedef typename Aux<PREC>::T TA;
+  const uint32_t i = blockIdx.x * BS + threadIdx.x;
+  if (i >= a.nwet) return;
+  const DevParams& dp = a.dp;
+  const WetNode<R> w = ((const WetNode<R>*)a.wet)[i];
+  TA* ph = (TA*)a.phiS;
+  if (w.zero) {
+    ph[w.n] = (TA)0;
     return;
   }
-  const int dxw = wrapg(dx, nx), dyw = wrapg(dy, ny), dzw = wrapg(dz, nz);
-  const size_t dn = nidx(dxw, dyw, dzw, nx, ny);
-  const R pf = (R)ph[dn];
+  const R eps_norm = (R)1.0e-14, huge_cot = (R)1.0e14;
+  const R pi = (R)3.1415926535897932384626433832795028841971;
+  const size_t sx = (size_t)dp.sx, row = w.d / (uint32_t)dp.nx, col = w.d - row * (uint32_t)dp.nx;
+  const R old = (R)ph[w.n], pf = (R)ph[w.d];
   R gx, gy, gz;
   if (a.gf_from_pre) {
-    const TA* pre = (const TA*)a.pre;
-    const size_t d5 = sbase(5, dxw, dyw, dzw, sx, ny);
-    gx = (R)pre[d5]; gy = (R)pre[d5 + sx]; gz = (R)pre[d5 + 2 * sx];
+    const TA* pre = (const TA*)a.pre + row * 5 * sx + col;
+    gx = (R)pre[0]; gy = (R)pre[sx]; gz = (R)pre[2 * sx];
   } else {
-    const TA* aux = (const TA*)a.aux;
-    const size_t d7 = sbase(7, dxw, dyw, dzw, sx, ny);
-    const R mg = (R)aux[d7 + 3 * sx];
-    gx = (R)aux[d7] * mg; gy = (R)aux[d7 + sx] * mg; gz = (R)aux[d7 + 2 * sx] * mg;
+    const TA* aux = (const TA*)a.aux + row * 7 * sx + col;
+    const R mg = (R)aux[3 * sx];
+    gx = (R)aux[0] * mg; gy = (R)aux[sx] * mg; gz = (R)aux[2 * sx] * mg;
   }
-  const R gdw = gx * wnx + gy * wny + gz * wnz;
-  const R tx = gx - gdw * wnx, ty = gy - gdw * wny, tz = gz - gdw * wnz;
+  const R gdw = gx * w.wx + gy * w.wy + gz * w.wz;
+  const R tx = gx - gdw * w.wx, ty = gy - gdw * w.wy, tz = gz - gdw * w.wz;
   const R tm = sqrt(tx * tx + ty * ty + tz * tz);
   const R th = ((R)180 - dp.ph<R>().wettab) * pi / (R)180;
   const R sn = sin(th), cs = cos(th);
   const R cot = fabs(sn) < eps_norm ? copysign(huge_cot, cs) : cs / sn;
   const R dnn = -tm * cot;
-  const R bx = tx + dnn * wnx, by = ty + dnn * wny, bz = tz + dnn * wnz;
-  ghost = pf + (bx * bsx + by * bsy + bz * bsz) * ((R)4.0 * ghost * ((R)1.0 - ghost));
-  ghost = fmax((R)0, fmin((R)1, ghost));
-  ph[n] = (TA)ghost;
+  const R bx = tx + dnn * w.wx, by = ty + dnn * w.wy, bz = tz + dnn * w.wz;
+  const R ghost = pf + (bx * (R)w.sx + by * (R)w.sy + bz * (R)w.sz) * ((R)4.0 * old * ((R)1.0 - old));
+  ph[w.n] = (TA)fmax((R)0, fmin((R)1, ghost));
 }
 
 // ---------------------------------------------------------------------------
@@ -1102,7 +1133,9 @@ static hipError_t stage_t(int stage, const StageArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((n + BS - 1) / BS)), block(BS);
   switch (stage) {
     case 1: hipLaunchKernelGGL(k_norm<PREC>, grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL(k_phi_bnd<PREC>, grid, block, 0, s, a); break;
+    case 2:
+      if (a.nwet) hipLaunchKernelGGL(k_phi_bnd<PREC>, dim3((a.nwet + BS - 1) / BS), block, 0, s, a);
+      break;
     case 3: hipLaunchKernelGGL(k_div<PREC>, grid, block, 0, s, a); break;
     case 4: hipLaunchKernelGGL(k_moments<PREC>, grid, block, 0, s, a); break;
     case 6: hipLaunchKernelGGL(k_update_phi<PREC>, grid, block, 0, s, a); break;
