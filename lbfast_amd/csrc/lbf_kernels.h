@@ -52,10 +52,11 @@ struct StageArgs {
   void* frc;         // 3-field set
   void* pre;         // 5-field set of the fast path (phase-field prep output)
   int gf_from_pre;   // PHI_int_boundary: donor gradient from pre instead of aux
-  int div_only;      // phase prep: store div theta only (fused_grad_inline)
+  int grad_inline;   // the fused kernel forms grad phi and lap phi itself (fused_grad_inline)
   void* rep;         // REPULSIVE_FLUX: 6-field set, locaux 3..8 (partner index, flux)
   int8_t* rep_mask;  // REPULSIVE_FLUX: nx*ny*nz
   const int8_t* isfh;
+  const uint32_t* words;  // obstacles: see FusedArgs
   const void* wet;   // WetNode<R> list of PHI_int_boundary
   uint32_t nwet;
   DevParams dp;

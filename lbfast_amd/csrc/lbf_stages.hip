@@ -9,11 +9,11 @@
 //   k_moments     moments_LB_kernel             (lb_cuda_moments_module.f90:19-341)
 //   k_update_phi  update_phifields_kernel       (lb_cuda_update_phi_module.f90:19-104)
 //   k_lb_int_bnd  LB_int_boundary_kernel        (lb_cuda_boundary_module.f90:19-216)
-//   k_phase_prep  compute_norm + compute_div_theta_n of the fast path in one
+//   k_phase_prep(_z)  compute_norm + compute_div_theta_n of the fast path in one
 //                 z-marching pass: phi planes and theta planes live in LDS,
-//                 the output per fluid node is grad phi (as n*|g|), lap phi
-//                 and div(theta n) -- what the fused kernel's inline moments
-//                 and phase update consume.
+//                 the output per node is div(theta n) and, where the fused
+//                 kernel does not form them itself, grad phi (as n*|g|) and
+//                 lap phi -- what its inline moments and phase update consume.
 // The fused stage is the z-marching kernel of lbf_fused.hip.
 #include <mutex>
 
@@ -265,51 +265,79 @@ __global__ void __launch_bounds__(PNT) k_phase_prep(StageArgs a, int tz) {
 // Streaming fast-path phase-field prep (float phase-field storage).
 //
 // The stencils of k_norm / k_div (lb_cuda_auxfields_module.f90:72-130,
-// 1110-1160) in their separable form (part3 / grad_lap in lbf_common.h):
-// each plane contributes three 9-point partial sums per node, and every
-// thread keeps the partials of the last planes of its own nodes in
-// registers as it marches z.  That reads 9 phi values per node from LDS (27
-// direct) and 21 theta values (54 direct).  The sums run in a different
-// order than the direct stencils, so results agree with them to rounding,
-// not bit for bit.
+// 1110-1160) in separable form (lbf_common.h): a plane's x pass (difference d,
+// second difference q, centre c) is taken once per row and shared by the rows
+// above and below, the y pass of three rows gives the plane's partial sums,
+// and the z direction combines three planes in running sums.  The sums run in
+// a different order than the direct stencils, so results agree with them to
+// rounding, not bit for bit.
 //
 // A block owns a 64-column tile (outputs x0 .. x0+63, aligned with the field
 // rows, so every store is a whole-row segment) by QY rows and marches z.
-// Its QW row waves hold two theta rows each; one more wave computes theta on
-// the two edge columns x0-1 and x0+64 that the tile's divergence needs.
-// phi rows are kept in LDS with a 2-column halo each side (column c holds
-// x0-2+c, wrapped): the row's 64 lanes and two 2-lane transfers for the
-// halo columns stream in by LDS DMA two planes ahead, into a ring of four
-// planes; theta lives in a ring of two planes of 66 columns (x0-1 ..
-// x0+64).  Iteration k computes div theta of plane k-2, then reads phi
-// plane k+1 and computes grad/lap/theta of plane k, with one barrier per
-// plane.  isfluid is read only with internal obstacles.  With a.div_only the gradient and Laplacian are not stored
-// (the fused kernel forms them itself from phi); only div theta is.
+// Its QW row waves hold two adjacent theta rows each; one more wave computes
+// theta on the two edge columns x0-1 and x0+64 that the tile's divergence
+// needs.  phi rows stream into LDS three planes ahead (a ring of four) with a
+// 4-column halo each side (column c holds x0-4+c, wrapped), so that the tile
+// is a run of 16-byte pieces, a lane each: one transfer in five waves of a
+// block a plane.  Where a piece would straddle the wrap (x faces, nx not a
+// multiple of 4) the rows come a dword a lane.  theta lives in a ring of two
+// planes of 66 columns (x0-1 .. x0+64).  Iteration k computes div theta of
+// plane k-2, then reads phi plane k+1 and computes grad/lap/theta of plane k,
+// with one barrier per plane.
+// With obstacles (OB) the node words of the tile's theta nodes stream in beside
+// phi: theta is 0 at non-fluid nodes (the reference never writes aux there and
+// reads the zero-initialised allocation).
+// MODE: PREP_DIV stores div theta only (the fused kernel forms grad phi and lap
+// phi itself), PREP_WALL also grad phi at near-wall nodes (the donors of the
+// wetting update), PREP_ALL grad phi and lap phi everywhere.
+//
+// What bounds it: instruction issue (it moves 8 bytes a node).  Two adjacent
+// rows a wave, the shared x passes, the running sums (no register moves of
+// whole partials), transfers and stores through scalar offsets: 352 -> 205
+// vector instructions a wave and plane; 0.70 -> 0.53 ms at 512^3, 106 -> 84 us at
+// 256^3, and with obstacles, where isfluid was gathered byte by byte and every
+// gather waited for the transfers in flight, 86 -> 55 us at 256x128x128 (with the
+// wetting update).
+enum PrepMode { PREP_DIV = 0, PREP_WALL = 1, PREP_ALL = 2 };
 constexpr int QY = 12, QW = 7;
 constexpr int QR = QY + 4;                 // phi rows of a tile (2-row halo)
 constexpr int QT = QY + 2;                 // theta rows (1-row halo)
-constexpr int QC = 64 + 4;                 // phi columns x0-2 .. x0+65
+constexpr int QH = 4;                      // halo columns each side
+constexpr int QC = 64 + 2 * QH;            // phi columns x0-4 .. x0+67
+constexpr int QP = QC / 4;                 // 16-byte pieces of a row
 constexpr int TC = 64 + 2;                 // theta columns x0-1 .. x0+64
-constexpr int QDMA = (QR + QW - 1) / QW;   // phi rows each row wave streams per plane
+constexpr int WC = 68, WP = WC / 4;        // node words of a theta row (x0-1 .. x0+66) and their pieces
+constexpr int QDMA = (QR + QW - 1) / QW;   // phi rows each row wave streams per plane, a dword a lane
 constexpr int QNT = (QW + 1) * 64;         // threads: row waves + the edge-column wave
+static_assert(QT == 2 * QW, "two theta rows per wave");
+static_assert(QR * QP <= QNT && QT * WP <= QNT, "one 16-byte piece a thread");
 
 __host__ __device__ inline int prep_tiles_z(const DevParams& dp, int tz) {
   return ((dp.nx + 63) / 64) * ((dp.ny + QY - 1) / QY) * ((dp.nz + tz - 1) / tz);
 }
 
-// DO: div theta only (a.div_only); the gradient outputs and the registers
-// that hold them are compiled out
-template <int PREC, bool DO>
+// vmcnt wait with a wave-uniform count of at most 5
+__device__ __forceinline__ void dma_wait_n(int n) {
+  if (n >= 4) { if (n >= 5) dma_wait<5>(); else dma_wait<4>(); }
+  else if (n >= 2) { if (n == 3) dma_wait<3>(); else dma_wait<2>(); }
+  else { if (n == 1) dma_wait<1>(); else dma_wait_all(); }
+}
+
+// the x pass of one row at one column: difference, second difference, centre
+template <class R>
+struct RowX { R d, q, c; };
+
+template <int PREC, int MODE, bool OB>
 __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile) {
   typedef typename Codec<PREC>::R R;
   typedef typename Aux<PREC>::T TA;
   static_assert(sizeof(TA) == 4, "float phase-field storage");
-  __shared__ float sphi[4][QR + 1][QC];  // row QR absorbs the padding transfers
+  __shared__ float sphi[4][QR][QC];
   __shared__ R sth[2][3][QT][TC];
+  __shared__ uint32_t swd[OB ? 2 : 1][OB ? QT : 1][OB ? WC : 1];
 
   const DevParams& dp = a.dp;
   const int nx = dp.nx, ny = dp.ny, nz = dp.nz;
-  const size_t nxny = (size_t)nx * ny;
   const int sx = dp.sx;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const bool edge_wave = wave == QW;
@@ -317,225 +345,228 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
   const int x0 = (tile % ntx) * 64, y0 = ((tile / ntx) % nty) * QY;
   const int z0 = (tile / (ntx * nty)) * tz, zend = min(z0 + tz, nz);
   const int XW = min(64, nx - x0);
-  const uint32_t pb = (uint32_t)(nxny * sizeof(TA));
-  const TA* phi = (const TA*)a.phiS;
-  TA* pre = (TA*)a.pre;
-  const R FOUR = 4, ONE = 1, HALF = 0.5, G3 = (R)(3.0 / 216.0);
+  const uint32_t pb = (uint32_t)nx * (uint32_t)ny * 4u;          // bytes of a phi plane
+  const uint32_t pbg = 5u * (uint32_t)sx * (uint32_t)ny * 4u;    // of a plane of the output set
+  const uint32_t pbw = (uint32_t)(nx + 2) * (uint32_t)(ny + 2) * 4u;
+  const float* phi = (const float*)a.phiS;
+  const R FOUR = 4, SIX = 6, ONE = 1, HALF = 0.5, G3 = (R)(3.0 / 216.0), L6 = (R)(6.0 / 216.0);
   const R eps = (R)1.0e-9;
-  constexpr bool store_g = !DO;
-  auto wrapx = [&](int x) { return ((x % nx) + nx) % nx; };
+  auto modn = [](int i, int n) { return ((i % n) + n) % n; };
 
-  // theta column of this lane: row waves j = lane + 1 (x = x0 + lane); the
-  // edge wave's lane 2t + s computes theta row t at j = 0 (s = 0) or 65
-  int tj = lane + 1, trow0 = 0;
-  bool edge_active = true;
-  if (edge_wave) {
-    edge_active = lane < 2 * QT;
-    tj = (lane & 1) ? TC - 1 : 0;
-    trow0 = edge_active ? (lane >> 1) : 0;
-  }
-  const int xt = x0 - 1 + tj;            // x of this lane's theta column (unwrapped)
-  const int xo = x0 + lane;              // output column of a row-wave lane
-  const bool out_lane = !edge_wave && lane < XW;
-
-  // DMA: row wave w streams phi rows w + QW*i: its 64 lanes to columns
-  // 2..65, lanes 0-1 to columns 0-1 (x0-2, x0-1) and to 66-67 (x0+64,
-  // x0+65); rows past the tile go to the padding row
-  // row byte offsets are wave-uniform (scalar); the lane's column offsets
-  // are added when a transfer is issued
-  uint32_t rowbyte[QDMA], rowlds[QDMA];
-  const uint32_t xm = (uint32_t)wrapx(x0 + lane) * 4u;
-  const uint32_t xlh = (uint32_t)wrapx(x0 - 2 + (lane & 1)) * 4u, xrh = (uint32_t)wrapx(x0 + 64 + (lane & 1)) * 4u;
-#pragma unroll
-  for (int i = 0; i < QDMA; ++i) {
-    const int r = wave + QW * i;
-    const int yw = (((y0 - 2 + (r < QR ? r : 0)) % ny) + ny) % ny;
-    rowbyte[i] = __builtin_amdgcn_readfirstlane((uint32_t)yw * (uint32_t)nx * (uint32_t)sizeof(TA));
-    rowlds[i] = __builtin_amdgcn_readfirstlane((uint32_t)(r < QR ? r : QR) * (uint32_t)QC * 4u);
-  }
+  // ---- transfers ------------------------------------------------------------------
+  const bool quad = nx % 4 == 0 || (x0 >= QH && x0 + 64 + QH <= nx);
   const uint32_t lds_phi = lds_addr(&sphi[0][0][0]);
+  uint32_t pq = 0, xh = 0, wq = 0;
+  uint32_t rowbyte[QDMA];
+  if (quad) {
+    const int L = min((int)threadIdx.x, QR * QP - 1);
+    pq = ((uint32_t)modn(y0 - 2 + L / QP, ny) * (uint32_t)nx + (uint32_t)modn(x0 - QH + 4 * (L % QP), nx)) * 4u;
+  } else {
+    // row waves stream rows wave + QW*i: 64 lanes to columns 4..67, and two
+    // lanes each to columns 2-3 (lanes 0-1) and 68-69 (lanes 2-3)
+    pq = (uint32_t)modn(x0 + lane, nx) * 4u;
+    xh = (uint32_t)modn((lane & 2) ? x0 + 62 + (lane & 3) : x0 - 2 + (lane & 1), nx) * 4u;
+#pragma unroll
+    for (int i = 0; i < QDMA; ++i) {
+      const int r = wave + QW * i;
+      rowbyte[i] = __builtin_amdgcn_readfirstlane((uint32_t)modn(y0 - 2 + (r < QR ? r : 0), ny) * (uint32_t)nx * 4u);
+    }
+  }
+  if constexpr (OB) {
+    const int L = min((int)threadIdx.x, QT * WP - 1);
+    wq = ((uint32_t)(clampi(y0 - 1 + L / WP, -1, ny) + 1) * (uint32_t)(nx + 2) + (uint32_t)(x0 + 4 * (L % WP))) * 4u;
+  }
+  // transfers of one phi plane that this wave issues
+  const int nd = quad ? (wave * 64 < QR * QP ? 1 : 0) : (edge_wave ? 0 : 3 * ((QR - wave + QW - 1) / QW));
+  static_assert(QDMA == 3, "6 or 9 transfers a wave");
   auto dma_plane = [&](int z) {
+    const Rsrc rs = mkrsrc(plane_at(phi, pb, modn(z, nz)), pb);
+    const uint32_t base = lds_phi + (uint32_t)(z & 3) * (uint32_t)(QR * QC * 4);
+    if (quad) {
+      if ((int)threadIdx.x < QR * QP) dma_quad<0u>(rs, pq, 0u, base + (uint32_t)wave * 1024u);
+      return;
+    }
     if (edge_wave) return;
-    const int zw = ((z % nz) + nz) % nz;
-    const Rsrc rs = mkrsrc(phi + (size_t)zw * nxny, pb);
-    const uint32_t base = lds_phi + (uint32_t)(z & 3) * (QR + 1) * QC * 4u;
 #pragma unroll
-    for (int i = 0; i < QDMA; ++i) dma_dword<8u>(rs, rowbyte[i] + xm, base + rowlds[i]);
-    // the halo columns: two lanes each (the transfers of the other lanes are
-    // masked off); three transfers per row in all
-    if (lane < 2) {
-#pragma unroll
-      for (int i = 0; i < QDMA; ++i) {
-        dma_dword<0u>(rs, rowbyte[i] + xlh, base + rowlds[i]);
-        dma_dword<66u * 4u>(rs, rowbyte[i] + xrh, base + rowlds[i]);
-      }
+    for (int i = 0; i < QDMA; ++i) {
+      const int r = wave + QW * i;
+      if (r >= QR) continue;
+      const uint32_t l = base + (uint32_t)r * (uint32_t)(QC * 4);
+      dma_dword<16u>(rs, rowbyte[i] + pq, l);
+      if (lane < 2) dma_dword<8u>(rs, rowbyte[i] + xh, l);
+      if ((lane & ~1) == 2) dma_dword<66u * 4u>(rs, rowbyte[i] + xh, l);
     }
   };
-  auto fluid = [&](int x, int y, int z) -> bool {
-    if (!dp.obst) return true;
-    const int8_t v = isf_at(a.isfh, x, y, z, nx, ny, nz);
-    return v == 1 || v == -1;
+  const uint32_t lds_wd = OB ? lds_addr((float*)&swd[0][0][0]) : 0u;
+  auto dma_words = [&](int z) {
+    if ((int)threadIdx.x < QT * WP)
+      dma_quad<0u>(mkrsrc(plane_at(a.words, pbw, clampi(z, -1, nz) + 1), 0xFFFFFFFFu), wq, 0u,
+                   lds_wd + (uint32_t)(z & 1) * (uint32_t)(QT * WC * 4) + (uint32_t)wave * 1024u);
   };
 
-  // per theta row h of this lane: phi partials of planes k-1 and k (pm, p0;
-  // p0.c is phi at the node in plane k); per div row: theta partials of
-  // planes k-3 and k-2 (em, e0)
-  Part3<R> pm[2], p0[2], em[2], e0[2];
-  // outputs held for one iteration (see below)
-  R hg[2][4], hd[2];
-  size_t og[2] = {0, 0}, od[2] = {0, 0};
-  bool st_g[2] = {false, false}, st_d[2] = {false, false};
+  // ---- this lane's nodes ------------------------------------------------------------
+  // theta column tj (x = x0 - 1 + tj): row waves lane + 1, rows 2 wave + h; the
+  // edge wave's lane 2t + s computes theta row t at column 0 (s = 0) or 65
+  const int tj = edge_wave ? ((lane & 1) ? TC - 1 : 0) : lane + 1;
+  const int t0 = edge_wave ? min(lane >> 1, QT - 1) : 2 * wave;
+  const bool edge_active = !edge_wave || lane < 2 * QT;
+  const bool out_lane = !edge_wave && lane < XW;
+  // output rows (theta rows 1 .. QY inside the domain), uniform over the wave
+  bool orow[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int t = 2 * wave + h;
+    orow[h] = !edge_wave && t >= 1 && t <= QY && y0 - 1 + t < ny;
+  }
+  const uint32_t go = ((uint32_t)(5 * (y0 - 1 + t0)) * (uint32_t)sx + (uint32_t)(x0 + lane)) * 4u;  // row h adds 20 sx
+  const uint32_t fb = (uint32_t)sx * 4u;
+  const float* phi_at = &sphi[0][t0][tj + QH - 2];
+  const uint32_t* word_at = OB ? &swd[0][t0][tj] : nullptr;
 
+  // per theta row h: phi sums in flight -- (Px, dx1) give d/dx of the last
+  // plane once its upper neighbour arrives, s0, s1, c0, c1 the smoothings and
+  // centre values of the last two planes; per div row: (D, M) the running sum of
+  // div theta, e0, e1 the centre values of theta_z of the last two planes
+  R Px[2] = {0, 0}, dx1[2] = {0, 0}, Py[2] = {0, 0}, dy1[2] = {0, 0}, s0[2] = {0, 0}, s1[2] = {0, 0}, c0[2] = {0, 0},
+    c1[2] = {0, 0};
+  R D[2] = {0, 0}, M[2] = {0, 0}, e0[2] = {0, 0}, e1[2] = {0, 0};
   dma_plane(z0 - 2);
   dma_plane(z0 - 1);
-  // Iteration k: div theta of plane k-2 from the theta of planes k-3 .. k-1,
-  // then phi partials of plane k+1 and theta of plane k.  One barrier per
-  // plane: theta(k-1), written before it, is read after it; theta(k) goes to
-  // the other slot of the two-plane ring.  Iterations z0-3 and z0-2 only fill
-  // the partials of planes z0-2, z0-1; iteration zend+1 only finishes the div.
+  // operations issued after the transfers that the next iteration needs (the
+  // newest phi plane, then the stores that every wave of their rows issues);
+  // they may stay outstanding, as a wave's operations retire in issue order
+  int late = nd;
   for (int k = z0 - 3; k <= zend + 1; ++k) {
-    // phi(k+1) has landed once only the newest plane's 3*QDMA transfers are outstanding
-    if (k + 2 <= zend + 1)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * QDMA) : "memory");
-    else
-      dma_wait_all();
+    // phi(k+1) and the node words of plane k have landed
+    if (nd <= 1) dma_wait_n(late);
+    else if (late >= 9) dma_wait<9>();
+    else if (late >= 6) dma_wait<6>();
+    else dma_wait_all();
     __syncthreads();
-
-    // ---- the previous iteration's outputs ---------------------------------------
-    // Stores are issued here, a full plane before the next wait on the
-    // load/store counter, instead of just ahead of it.
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (st_g[h]) {
-        pre[og[h]] = (TA)hg[h][0];
-        pre[og[h] + sx] = (TA)hg[h][1];
-        pre[og[h] + 2 * sx] = (TA)hg[h][2];
-        pre[og[h] + 3 * sx] = (TA)hg[h][3];
-      }
-      if (st_d[h]) pre[od[h] + 4 * sx] = (TA)hd[h];
-      st_g[h] = false;
-      st_d[h] = false;
+    late = 0;
+    // the slots of phi(k-1) and words(k-1) were last read before this barrier
+    if constexpr (OB) {
+      if (k >= z0 - 2 && k < zend) dma_words(k + 1);
+    }
+    if (k + 3 <= zend + 1) {
+      dma_plane(k + 3);
+      late = nd;
     }
 
-    // ---- theta partials of plane k-1; div theta of plane k-2 on theta rows
-    // 1 + wave, 1 + wave + QW -----------------------------------------------------------
+    // ---- theta partials of plane k-1; div theta of plane k-2 -------------------------
     const int zo = k - 2;
     if (!edge_wave && k - 1 >= z0 - 1 && k - 1 <= zend) {
       const int tk = (k - 1) & 1;
+      RowX<R> X[4], Y[4], Z[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        // theta rows 2 wave - 1 .. 2 wave + 2 (clamped rows feed no output)
+        const int t = min(max(2 * wave - 1 + r, 0), QT - 1);
+        const R x_ = sth[tk][0][t][lane], xp = sth[tk][0][t][lane + 2];
+        X[r].d = xp - x_;
+        const R y_ = sth[tk][1][t][lane], yc = sth[tk][1][t][lane + 1], yp = sth[tk][1][t][lane + 2];
+        Y[r].c = (y_ + yp) + FOUR * yc;
+        const R z_ = sth[tk][2][t][lane], zc = sth[tk][2][t][lane + 1], zp = sth[tk][2][t][lane + 2];
+        Z[r].q = (z_ - zc) + (zp - zc);
+        Z[r].c = zc;
+      }
+      const Rsrc rg = mkrsrc(plane_at((float*)a.pre, pbg, zo < 0 ? 0 : zo), pbg);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int t = 1 + wave + QW * h;
-        if (t > QY) continue;
-        R w[3][3];
-        Part3<R> ep;
-#pragma unroll
-        for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-          for (int aa = 0; aa < 3; ++aa) w[bb][aa] = sth[tk][0][t - 1 + bb][tj - 1 + aa];
-        ep.dx = (w[0][2] - w[0][0]) + FOUR * (w[1][2] - w[1][0]) + (w[2][2] - w[2][0]);
-#pragma unroll
-        for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-          for (int aa = 0; aa < 3; ++aa) w[bb][aa] = sth[tk][1][t - 1 + bb][tj - 1 + aa];
-        ep.dy = (w[2][0] - w[0][0]) + FOUR * (w[2][1] - w[0][1]) + (w[2][2] - w[0][2]);
-#pragma unroll
-        for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-          for (int aa = 0; aa < 3; ++aa) w[bb][aa] = sth[tk][2][t - 1 + bb][tj - 1 + aa];
-        {
-          // smoothing of (theta_z - centre), as part3
-          const R ct = w[1][1];
-          ep.s = ((w[0][0] - ct) + FOUR * (w[0][1] - ct) + (w[0][2] - ct)) +
-                 FOUR * ((w[1][0] - ct) + (w[1][2] - ct)) + ((w[2][0] - ct) + FOUR * (w[2][1] - ct) + (w[2][2] - ct));
-          ep.c = ct;
+        const R A = G3 * ((X[h].d + FOUR * X[h + 1].d + X[h + 2].d) + (Y[h + 2].c - Y[h].c));
+        const R cm = Z[h].c, cc = Z[h + 1].c, cp = Z[h + 2].c;
+        const R b = G3 * ((Z[h].q + FOUR * Z[h + 1].q + Z[h + 2].q) + SIX * ((cm - cc) + (cp - cc)));
+        const R d = (D[h] + (A + b)) + HALF * (cc - e0[h]);
+        D[h] = M[h] + FOUR * A;
+        M[h] = A - b;
+        e0[h] = e1[h];
+        e1[h] = cc;
+        if (orow[h] && zo >= z0 && zo < zend) {
+          // obstacles: a solid node's value is never read
+          if (out_lane) bsts(rg, go + (uint32_t)h * 5u * fb, 4u * fb, (float)d);
+          ++late;
         }
-        if (zo >= z0 && zo < zend) {
-          const R d = G3 * ((em[h].dx + FOUR * e0[h].dx + ep.dx) + (em[h].dy + FOUR * e0[h].dy + ep.dy) +
-                            (ep.s - em[h].s)) + HALF * (ep.c - em[h].c);
-          const int y = y0 - 1 + t;
-          if (out_lane && y < ny && fluid(xo, y, zo)) {
-            hd[h] = d;
-            od[h] = sbase(5, xo, y, zo, sx, ny);
-            st_d[h] = true;
-          }
-        }
-        em[h] = e0[h];
-        e0[h] = ep;
       }
     }
 
     // ---- phi partials of plane k+1; grad / lap / theta of plane k -----------------
-    // row waves: theta rows wave, wave + QW (columns 1..64); edge wave: rows
-    // lane >> 1 at columns 0 and 65
-    static_assert(QT == 2 * QW, "two theta rows per wave");
     if (k + 1 <= zend + 1) {
       const int sp = (k + 1) & 3, tk = k & 1;
       const bool have_theta = k >= z0 - 1;
       const bool own = k >= z0 && k < zend;
+      RowX<R> V[4];
+      const float* pv = phi_at + sp * (QR * QC);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (edge_wave && r == 3) break;  // one row per lane
+        const R vm = (R)pv[r * QC], vc = (R)pv[r * QC + 1], vp = (R)pv[r * QC + 2];
+        V[r].d = vp - vm;
+        V[r].q = (vm - vc) + (vp - vc);
+        V[r].c = vc;
+      }
+      const Rsrc rg = mkrsrc(plane_at((float*)a.pre, pbg, own ? k : 0), pbg);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        if (edge_wave && h == 1) break;  // wave-uniform: the edge wave has one row per lane
-        const int t = edge_wave ? trow0 : wave + QW * h;
-        R v[3][3];
-#pragma unroll
-        for (int bb = 0; bb < 3; ++bb)
-#pragma unroll
-          for (int aa = 0; aa < 3; ++aa) v[bb][aa] = (R)sphi[sp][t + bb][tj + aa];
-        const Part3<R> pp = part3(v);
+        if (edge_wave && h == 1) break;  // wave-uniform
+        const R dxp = V[h].d + FOUR * V[h + 1].d + V[h + 2].d;
+        const R cc = V[h + 1].c;
+        const R dyp = (V[h + 2].q - V[h].q) + SIX * (V[h + 2].c - V[h].c);
+        const R sp_ = (V[h].q + FOUR * V[h + 1].q + V[h + 2].q) + SIX * ((V[h].c - cc) + (V[h + 2].c - cc));
         if (have_theta) {
-          const R c = p0[h].c;
-          R gx, gy, gz, lap;
-          grad_lap(pm[h], p0[h], pp, gx, gy, gz, lap);
-          const int y = y0 - 1 + t;
-          R thx = 0, thy = 0, thz = 0;
-          if (fluid(xt, y, k)) {
-            const R mg = sqrt(gx * gx + gy * gy + gz * gz);
-            const R im = rcp(mg + eps);
-            const R nxv = gx * im, nyv = gy * im, nzv = gz * im;
-            thx = c * (ONE - c) * nxv; thy = c * (ONE - c) * nyv; thz = c * (ONE - c) * nzv;
-            if (store_g && own && out_lane && t >= 1 && t <= QY && y < ny) {
-              // the reference re-reads n and |g| from storage precision
-              const R mgs = (R)(TA)mg;
-              hg[h][0] = (R)(TA)nxv * mgs;
-              hg[h][1] = (R)(TA)nyv * mgs;
-              hg[h][2] = (R)(TA)nzv * mgs;
-              hg[h][3] = lap;
-              og[h] = sbase(5, xo, y, k, sx, ny);
-              st_g[h] = true;
-            }
+          const R c = c1[h];
+          const R gx = G3 * (Px[h] + dxp), gy = G3 * (Py[h] + dyp);
+          const R gz = G3 * (sp_ - s0[h]) + HALF * (cc - c0[h]);
+          const R mg = sqrt(gx * gx + gy * gy + gz * gz);
+          const R im = rcp(mg + eps);
+          const R nxv = gx * im, nyv = gy * im, nzv = gz * im;
+          R th = c * (ONE - c);
+          uint32_t word = NODE_FLUID;
+          if constexpr (OB) {
+            word = word_at[tk * (QT * WC) + h * WC];
+            th = word & NODE_FLUID ? th : (R)0;
           }
           if (edge_active) {
-            sth[tk][0][t][tj] = (R)(TA)thx;
-            sth[tk][1][t][tj] = (R)(TA)thy;
-            sth[tk][2][t][tj] = (R)(TA)thz;
+            const int t = t0 + h;
+            sth[tk][0][t][tj] = (R)(TA)(th * nxv);
+            sth[tk][1][t][tj] = (R)(TA)(th * nyv);
+            sth[tk][2][t][tj] = (R)(TA)(th * nzv);
+          }
+          if constexpr (MODE != PREP_DIV) {
+            if (orow[h] && own) {
+              // the reference re-reads n and |g| from storage precision
+              const R mgs = (R)(TA)mg;
+              const bool st = out_lane && (MODE == PREP_ALL ? (word & NODE_FLUID) != 0 : (word & NODE_WALL) != 0);
+              if (st) {
+                const uint32_t o = go + (uint32_t)h * 5u * fb;
+                bsts(rg, o, 0u, (float)((R)(TA)nxv * mgs));
+                bsts(rg, o, fb, (float)((R)(TA)nyv * mgs));
+                bsts(rg, o, 2u * fb, (float)((R)(TA)nzv * mgs));
+                if constexpr (MODE == PREP_ALL)
+                  bsts(rg, o, 3u * fb, (float)(L6 * (s0[h] + FOUR * s1[h] + sp_) + ((c0[h] - c) + (cc - c))));
+              }
+            }
           }
         }
-        pm[h] = p0[h];
-        p0[h] = pp;
+        Px[h] = dx1[h] + FOUR * dxp;
+        dx1[h] = dxp;
+        Py[h] = dy1[h] + FOUR * dyp;
+        dy1[h] = dyp;
+        s0[h] = s1[h];
+        s1[h] = sp_;
+        c0[h] = c1[h];
+        c1[h] = cc;
       }
     }
-    // slot (k+3)&3 held plane k-1, last read in iteration k-2
-    if (k + 3 <= zend + 1) dma_plane(k + 3);
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (st_g[h]) {
-      pre[og[h]] = (TA)hg[h][0];
-      pre[og[h] + sx] = (TA)hg[h][1];
-      pre[og[h] + 2 * sx] = (TA)hg[h][2];
-      pre[og[h] + 3 * sx] = (TA)hg[h][3];
-    }
-    if (st_d[h]) pre[od[h] + 4 * sx] = (TA)hd[h];
   }
 }
 
-template <int PREC, bool DO>
+template <int PREC, int MODE, bool OB>
 __global__ void __launch_bounds__(QNT) k_phase_prep_z(StageArgs a, int tz) {
-  prep_body_z<PREC, DO>(a, tz, xcd_tile(blockIdx.x, prep_tiles_z(a.dp, tz)));
+  prep_body_z<PREC, MODE, OB>(a, tz, xcd_tile(blockIdx.x, prep_tiles_z(a.dp, tz)));
 }
 
-// many domains per launch (see fused_kernel_batch)
-template <int PREC, bool DO>
+// many domains per launch (see fused_kernel_batch); batches hold no obstacles
+template <int PREC, int MODE>
 __global__ void __launch_bounds__(QNT)
     k_phase_prep_z_batch(const PrepBatchEntry* __restrict__ tab, int ndom, int total) {
   const int g = xcd_tile(blockIdx.x, total);
@@ -544,7 +575,7 @@ __global__ void __launch_bounds__(QNT)
     const int mid = (lo + hi + 1) >> 1;
     if (tab[mid].tile0 <= g) lo = mid; else hi = mid - 1;
   }
-  prep_body_z<PREC, DO>(tab[lo].a, tab[lo].tz, g - tab[lo].tile0);
+  prep_body_z<PREC, MODE, false>(tab[lo].a, tab[lo].tz, g - tab[lo].tile0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1167,11 +1198,22 @@ hipError_t launch_stage(int stage, const StageArgs& a, int prec, hipStream_t s) 
   return hipErrorInvalidValue;
 }
 
+template <int PREC, int MODE, bool OB>
+static hipError_t prep_z(const StageArgs& a, int tz, hipStream_t s) {
+  hipLaunchKernelGGL((k_phase_prep_z<PREC, MODE, OB>), dim3(prep_tiles_z(a.dp, tz)), dim3(QNT), 0, s, a, tz);
+  return hipGetLastError();
+}
+
 template <int PREC>
 static hipError_t prep_t(const StageArgs& a, int tz, hipStream_t s) {
   if constexpr (sizeof(typename Aux<PREC>::T) == 4) {
-    if (a.div_only) hipLaunchKernelGGL((k_phase_prep_z<PREC, true>), dim3(prep_tiles_z(a.dp, tz)), dim3(QNT), 0, s, a, tz);
-    else hipLaunchKernelGGL((k_phase_prep_z<PREC, false>), dim3(prep_tiles_z(a.dp, tz)), dim3(QNT), 0, s, a, tz);
+    if constexpr (PREC == PREC_MIXED) {
+      return a.dp.obst ? prep_z<PREC, PREP_ALL, true>(a, tz, s) : prep_z<PREC, PREP_ALL, false>(a, tz, s);
+    } else {
+      // without obstacles the fused kernel always forms its gradients itself
+      if (!a.dp.obst) return prep_z<PREC, PREP_DIV, false>(a, tz, s);
+      return a.grad_inline ? prep_z<PREC, PREP_WALL, true>(a, tz, s) : prep_z<PREC, PREP_ALL, true>(a, tz, s);
+    }
   } else {
     const dim3 grid(((a.dp.nx + PTX - 1) / PTX) * ((a.dp.ny + PTY - 1) / PTY) * ((a.dp.nz + tz - 1) / tz));
     hipLaunchKernelGGL(k_phase_prep<PREC>, grid, dim3(PNT), 0, s, a, tz);
@@ -1189,10 +1231,10 @@ hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int 
   // batches hold two-component domains without obstacles: div theta only
   // exactly where fused_grad_inline() holds, i.e. for every precision but MIXED
   switch (prec) {
-    case PREC_FP32: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP32, true>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_MIXED: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_MIXED, false>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_FP16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP16S, true>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_BF16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_BF16S, true>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
+    case PREC_FP32: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP32, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
+    case PREC_MIXED: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_MIXED, PREP_ALL>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
+    case PREC_FP16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP16S, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
+    case PREC_BF16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_BF16S, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
