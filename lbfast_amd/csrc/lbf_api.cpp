@@ -263,14 +263,17 @@ static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t
 
 // One block of the fused kernel fits a CU.  A plane of an 8-row block takes
 // 0.72 of a 13-row block's time (measured 0.66 at 512^3, where HBM counts, to
-// 0.81 at 64^3); with 64-bit arithmetic the 13-row block's 128 registers a lane
-// spill and 8 rows are always the faster (160^3: FP64 311 against 560 us,
-// MIXED 219 against 404).
+// 0.81 at 64^3).  In 64-bit arithmetic the prefetching kernel needs 256 registers
+// a lane, blocks of 5 rows; with two components or obstacles they are the
+// faster (160^3 FP64 276 us against 309 with 8 rows and 560 with 13, which
+// spills; MIXED 208 against 218; FP64 channel 128x96x96 106 against 159), with
+// one component about even, a plane of 5 rows at 0.55 (256^3) to 0.75 (64^3) of
+// one of 8.
 static const double T_FUSED[1] = {1.0};
 constexpr int FUSED_EXTRA = 3;
-constexpr double T8 = 0.72;
+constexpr double T8 = 0.72, T5 = 0.72;
 static long fused_xy(const lbf_params& p, int ty) { return (long)((p.nx + 63) / 64) * ((p.ny + ty - 1) / ty); }
-static bool rows8_only(int prec) { return prec == LBF_PREC_FP64 || prec == LBF_PREC_MIXED; }
+static bool wide_arith(int prec) { return prec == LBF_PREC_FP64 || prec == LBF_PREC_MIXED; }
 // Three blocks of the 16/32-bit phase prep fit a CU (measured plane times 1.65,
 // 2.2, 2.9 us with one to three), two of the FP64 prep.
 static const double T_PREP[3] = {1.0, 1.34, 1.75};
@@ -284,18 +287,26 @@ static const double T_PREP64[2] = {1.0, 1.5};
 // 149 -> 113, 256^3 FP16S 435 -> 353, 160^3 FP64 678 -> 311.
 static void default_tiles(lbf_ctx* c) {
   int tz8 = 1, tz13 = 1;
-  const double c8 = T8 * pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
-  const double c13 = pick_chunk(fused_xy(c->p, 13), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz13);
-  const bool r8 = rows8_only(c->prec) || c8 < c13;
-  c->ty = r8 ? 8 : 13;
-  c->tz = r8 ? tz8 : tz13;
+  if (wide_arith(c->prec)) {
+    int tz5 = 1;
+    const double c5 = T5 * pick_chunk(fused_xy(c->p, 5), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz5);
+    const double c8 = pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
+    const bool r5 = c->p.twocomponent || c->p.internal_obstacles || c5 < c8;
+    c->ty = r5 ? 5 : 8;
+    c->tz = r5 ? tz5 : tz8;
+  } else {
+    const double c8 = T8 * pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
+    const double c13 = pick_chunk(fused_xy(c->p, 13), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz13);
+    c->ty = c8 < c13 ? 8 : 13;
+    c->tz = c8 < c13 ? tz8 : tz13;
+  }
   // prep blocks: 64 x 12 tiles that march 5 planes beyond their chunk (theta and
-  // phi halo planes, one step of store lag); the FP64 prep's 64 x 8 tiles 2
+  // phi halo planes, one step of store lag)
   StageArgs one{};
   one.dp = c->dp;
-  const long pt = prep_tile_count(one, c->prec, c->p.nz);
-  if (pt > 0) pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP, 3, &c->tz_prep);
-  else pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, 2, T_PREP64, 2, &c->tz_prep);
+  const long pt = prep_tile_count(one, c->p.nz);
+  if (c->prec == LBF_PREC_FP64) pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP64, 2, &c->tz_prep);
+  else pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP, 3, &c->tz_prep);
 }
 
 int lbf_create(const lbf_params* pin, lbf_ctx** out) {
@@ -630,7 +641,6 @@ static StageArgs stage_args(lbf_ctx* c) {
   a.frc = c->frc;
   a.pre = c->pre;
   a.gf_from_pre = 0;
-  a.grad_inline = fused_grad_inline(c->prec, c->dp) ? 1 : 0;
   a.rep = c->rep;
   a.rep_mask = c->rep_mask;
   a.isfh = c->isfh;
@@ -1012,7 +1022,7 @@ static int batch_tables(lbf_batch* b) {
       q[i].a.gf_from_pre = 1;
       q[i].tz = b->tz_prep[d];
       q[i].tile0 = pt;
-      if (b->two) pt += prep_tile_count(q[i].a, b->prec, b->tz_prep[d]);
+      if (b->two) pt += prep_tile_count(q[i].a, b->tz_prep[d]);
       c->cur = cur0;
       c->ucur = ucur0;
     }
@@ -1102,14 +1112,18 @@ static void batch_default_tiles(lbf_batch* b) {
     return best;
   };
   int T8b = 1, T13b = 1, Tp = 1;
-  const double c8 = T8 * search(8, FUSED_EXTRA, 1, &T8b), c13 = search(13, FUSED_EXTRA, 1, &T13b);
-  const bool r8 = rows8_only(b->prec) || c8 < c13;
-  b->ty = r8 ? 8 : 13;
+  if (wide_arith(b->prec)) {
+    b->ty = b->two ? 5 : 8;
+    search(b->ty, FUSED_EXTRA, 1, &T8b);
+  } else {
+    const double c8 = T8 * search(8, FUSED_EXTRA, 1, &T8b), c13 = search(13, FUSED_EXTRA, 1, &T13b);
+    b->ty = c8 < c13 ? 8 : 13;
+  }
   search(12, 5, 3, &Tp);
   b->tz.clear();
   b->tz_prep.clear();
   for (lbf_ctx* c : b->ctx) {
-    b->tz.push_back(chunk(c->p.nz, r8 ? T8b : T13b));
+    b->tz.push_back(chunk(c->p.nz, b->ty == 13 ? T13b : T8b));
     b->tz_prep.push_back(chunk(c->p.nz, Tp));
   }
 }

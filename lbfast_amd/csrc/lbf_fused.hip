@@ -111,18 +111,15 @@ struct RawNode {
   typename Aux<PREC>::T g[5];  // inline: grad phi (3), lap phi, div theta n; stage path: forces (3)
 };
 
-// LDS slots of the prefetched inputs (one 64-lane row of dwords each):
-// moments 0-9, phi 10, g 11-15, u_old 16-18.  GI (gradient inline): phi
-// comes from the block's phi tile instead, and g holds div theta only (slot
-// 10, u_old 11-13).
-template <bool TWO, bool INLINE, bool GI = false>
+// A wave's LDS slots of the prefetched inputs, in bytes from its base: 64
+// values of each moment, of u_old (U), of the g set (G: the prep's output or the
+// forces; with the gradient formed inside, GI, only div theta) and of phi
+// (which comes from the block's phi tile under GI).
+template <int PREC, bool TWO, bool INLINE, bool GI>
 struct Slots {
-  static constexpr int PHI = 10, G = 11, UO = 16;
-  static constexpr int N = INLINE ? (TWO ? 19 : 10) : 14;
-};
-template <>
-struct Slots<true, true, true> {
-  static constexpr int PHI = -1, G = 10, UO = 11, N = 14;
+  static constexpr int SB = 64 * sizeof(typename Codec<PREC>::T), SA = 64 * sizeof(typename Aux<PREC>::T);
+  static constexpr int NU = INLINE && TWO ? 3 : 0, NG = !INLINE ? 3 : !TWO ? 0 : GI ? 1 : 5, NP = TWO && !GI ? 1 : 0;
+  static constexpr int U = 10 * SB, G = U + NU * SB, PHI = G + NG * SA, BYTES = (PHI + NP * SA + 255) / 256 * 256;
 };
 
 // Per-lane byte offsets of one node inside a z plane of each input buffer,
@@ -133,15 +130,16 @@ struct Slots<true, true, true> {
 struct FOff {
   uint32_t m, u, g, p;
   uint32_t pm, pu, pg, pp;
-  // where the transfers of dma_raw start in the moment, u_old and g sets.  Row
-  // waves (rows != 0, wave-uniform) fetch whole field rows, 16 bytes a lane
-  // (the lane's node + row_off); the x-halo wave the aligned dword of its node.
+  // where the lane's transfers of dma_raw start in the moment, u_old and g sets
+  // and in phi.  Row waves (rows != 0, wave-uniform) fetch whole field rows, 16
+  // bytes a lane (the lane's node + row_off); the x-halo wave a dword a lane:
+  // the aligned dword of its node, or of 64-bit values one of its node's two
   int rows;
-  uint32_t lm, lu, lg;
+  uint32_t lm, lu, lg, lp;
 };
 
-// A wave's 64-node row segments of a set move four (32-bit values) or eight
-// (16-bit) fields to a transfer: lane l fetches 16 bytes of field l / G at
+// A wave's 64-node row segments of a set move two (64-bit values), four (32) or
+// eight (16) fields to a transfer: lane l fetches 16 bytes of field l / G at
 // element E (l % G), G lanes to a 64-value row.  Lanes past a short row read
 // on into the row's end and the next field; those nodes are never used, and
 // every buffer is padded past its last plane.  The transfers were bound by
@@ -154,19 +152,23 @@ __device__ __forceinline__ uint32_t row_off(int sx) {
   return ((l / G) * (uint32_t)sx + (l % G) * E - l) * (uint32_t)sizeof(V);
 }
 // the NF fields of a set at one plane into the wave's LDS from byte OFF on
-template <class V, uint32_t OFF, int NF>
+template <class V, uint32_t OFF, int NF, int W = 0>
 __device__ __forceinline__ void dma_rows(const V* plane0, uint32_t voff, int sx, uint32_t lds0) {
   constexpr int G = 64 * sizeof(V) / 16, PER = 64 / G;  // lanes per row, rows per transfer
   const Rsrc r = mkrsrc(plane0, 0xFFFFFFFFu);
-  const uint32_t step = (uint32_t)(PER * sizeof(V)) * (uint32_t)sx;
-  const int l = threadIdx.x & 63;
-  if constexpr (NF >= PER) dma_quad<OFF>(r, voff, 0u, lds0);
-  if constexpr (NF >= 2 * PER) dma_quad<OFF + 1024u>(r, voff, step, lds0);
-  constexpr int W = NF / PER, REM = NF % PER;
-  static_assert(W <= 2, "at most two full transfers");
-  if constexpr (REM != 0) {
-    if (l < REM * G) dma_quad<OFF + 1024u * W>(r, voff, (uint32_t)W * step, lds0);
+  const uint32_t soff = (uint32_t)(W * PER * sizeof(V)) * (uint32_t)sx;
+  if constexpr (NF >= (W + 1) * PER) {
+    dma_quad<OFF + 1024u * W>(r, voff, soff, lds0);
+    if constexpr (NF > (W + 1) * PER) dma_rows<V, OFF, NF, W + 1>(plane0, voff, sx, lds0);
+  } else {
+    if ((int)(threadIdx.x & 63) < (NF - W * PER) * G) dma_quad<OFF + 1024u * W>(r, voff, soff, lds0);
   }
+}
+// the x-halo wave's: at most 32 nodes, a slot of 64 values to a field
+template <class V, uint32_t OFF, int NF, int F = 0>
+__device__ __forceinline__ void dma_nodes(Rsrc r, uint32_t voff, int sx, uint32_t lds0) {
+  dma_dword<OFF + 64u * (uint32_t)sizeof(V) * F>(r, voff, lds0, (uint32_t)(F * sizeof(V)) * (uint32_t)sx);
+  if constexpr (F + 1 < NF) dma_nodes<V, OFF, NF, F + 1>(r, voff, sx, lds0);
 }
 
 // Direct loads of one plane's inputs (used when the inputs are not prefetched).
@@ -198,94 +200,65 @@ __device__ __forceinline__ void load_raw(RawNode<PREC>& r, const FusedArgs& a, i
   }
 }
 
-// LDS-DMA prefetch of one plane's inputs into this wave's slots.  Float
-// fields move their lane's dword; a 16-bit moment field moves the aligned
-// dword that holds the lane's element (the half is picked when read back:
-// byte (o.m & 2) of the slot; sx is even, so every 16-bit field row starts on
-// a dword and the u_old offsets share that parity).
+// LDS-DMA prefetch of one plane's inputs into this wave's slots.  The x-halo
+// wave moves the aligned dword that holds a 16-bit element (the half is picked
+// when read back; sx is even, so every 16-bit field row starts on a dword and
+// the u_old offsets share that parity).
 template <int PREC, bool TWO, bool INLINE, bool GI>
 __device__ __forceinline__ void dma_raw(const FusedArgs& a, int zw, const FOff& o, bool dens, uint32_t lds0) {
-  typedef Slots<TWO, INLINE, GI> SL;
+  typedef Slots<PREC, TWO, INLINE, GI> SL;
   typedef typename Codec<PREC>::T T;
-  static_assert(sizeof(typename Aux<PREC>::T) == 4, "float phase-field storage");
+  typedef typename Aux<PREC>::T TA;
   const int sx = a.dp.sx;
   const T* S = plane_at((const T*)a.min, o.pm, zw);
-  const float* g = plane_at((const float*)(INLINE ? a.pre : a.frc), o.pg, zw);
   const T* uo = plane_at((const T*)a.uin, o.pu, zw);
+  const TA* g = plane_at((const TA*)(INLINE ? a.pre : a.frc), o.pg, zw);
+  if constexpr (GI) g += 4 * (size_t)sx;
+  const TA* ph = plane_at((const TA*)a.phin, o.pp, zw);
   // slot offsets are immediates: only the wave's LDS base stays live
-  if constexpr (TWO && !GI)
-    dma_dword<256u * SL::PHI>(mkrsrc(plane_at((const float*)a.phin, o.pp, zw), o.pp), o.p, lds0);
-  if constexpr (GI) dma_dword<256u * SL::G>(mkrsrc(g, o.pg), o.g, lds0, 16u * (uint32_t)sx);
+  if constexpr (GI) dma_dword<(uint32_t)SL::G>(mkrsrc(g, o.pg), o.g, lds0);
   if (o.rows) {
     dma_rows<T, 0u, 10>(S, o.lm, sx, lds0);
-    if constexpr (!INLINE) dma_rows<float, 256u * SL::G, 3>(g, o.lg, sx, lds0);
-    else if constexpr (TWO && !GI) dma_rows<float, 256u * SL::G, 5>(g, o.lg, sx, lds0);
-    if constexpr (INLINE && TWO) {
-      if (dens) dma_rows<T, 256u * SL::UO, 3>(uo, o.lu, sx, lds0);
+    if constexpr (!GI && SL::NG > 0) dma_rows<TA, (uint32_t)SL::G, SL::NG>(g, o.lg, sx, lds0);
+    if constexpr (SL::NP > 0) dma_rows<TA, (uint32_t)SL::PHI, 1>(ph, o.lp, sx, lds0);
+    if constexpr (SL::NU > 0) {
+      if (dens) dma_rows<T, (uint32_t)SL::U, 3>(uo, o.lu, sx, lds0);
     }
-    return;
-  }
-  // x-halo wave: at most 32 nodes, a dword each.  A 16-bit field's slot is then
-  // 128 B long as in the row waves
-  const uint32_t fb = (uint32_t)sx * (uint32_t)sizeof(T), gb = (uint32_t)sx * 4u;
-  constexpr uint32_t SB = 64u * (uint32_t)sizeof(T);  // bytes of a field's slot
-  if ((threadIdx.x & 63) < 32) {
-    const Rsrc rm = mkrsrc(S, o.pm);
-    dma_dword<SB * 0>(rm, o.lm, lds0);
-    dma_dword<SB * 1>(rm, o.lm, lds0, 1 * fb);
-    dma_dword<SB * 2>(rm, o.lm, lds0, 2 * fb);
-    dma_dword<SB * 3>(rm, o.lm, lds0, 3 * fb);
-    dma_dword<SB * 4>(rm, o.lm, lds0, 4 * fb);
-    dma_dword<SB * 5>(rm, o.lm, lds0, 5 * fb);
-    dma_dword<SB * 6>(rm, o.lm, lds0, 6 * fb);
-    dma_dword<SB * 7>(rm, o.lm, lds0, 7 * fb);
-    dma_dword<SB * 8>(rm, o.lm, lds0, 8 * fb);
-    dma_dword<SB * 9>(rm, o.lm, lds0, 9 * fb);
-    if constexpr (INLINE && TWO) {
-      if (dens) {
-        const Rsrc ru = mkrsrc(uo, o.pu);
-        dma_dword<256u * SL::UO + SB * 0>(ru, o.lu, lds0);
-        dma_dword<256u * SL::UO + SB * 1>(ru, o.lu, lds0, 1 * fb);
-        dma_dword<256u * SL::UO + SB * 2>(ru, o.lu, lds0, 2 * fb);
+  } else {
+    const int l = threadIdx.x & 63;
+    if (l < (sizeof(T) == 8 ? 64 : 32)) {
+      dma_nodes<T, 0u, 10>(mkrsrc(S, o.pm), o.lm, sx, lds0);
+      if constexpr (SL::NU > 0) {
+        if (dens) dma_nodes<T, (uint32_t)SL::U, 3>(mkrsrc(uo, o.pu), o.lu, sx, lds0);
       }
     }
-  }
-  if constexpr (!INLINE || (TWO && !GI)) {
-    const Rsrc rg = mkrsrc(g, o.pg);
-    dma_dword<256u * (SL::G + 0)>(rg, o.lg, lds0);
-    dma_dword<256u * (SL::G + 1)>(rg, o.lg, lds0, 1 * gb);
-    dma_dword<256u * (SL::G + 2)>(rg, o.lg, lds0, 2 * gb);
-    if constexpr (INLINE) {
-      dma_dword<256u * (SL::G + 3)>(rg, o.lg, lds0, 3 * gb);
-      dma_dword<256u * (SL::G + 4)>(rg, o.lg, lds0, 4 * gb);
+    if (l < (sizeof(TA) == 8 ? 64 : 32)) {
+      if constexpr (!GI && SL::NG > 0) dma_nodes<TA, (uint32_t)SL::G, SL::NG>(mkrsrc(g, o.pg), o.lg, sx, lds0);
+      if constexpr (SL::NP > 0) dma_nodes<TA, (uint32_t)SL::PHI, 1>(mkrsrc(ph, o.pp), o.lp, sx, lds0);
     }
   }
 }
 
 template <int PREC, bool TWO, bool INLINE, bool GI>
-__device__ __forceinline__ void lds_raw(RawNode<PREC>& r, const float (*slot)[64], int lane, bool dens, uint32_t bT,
-                                        bool rows) {
-  typedef Slots<TWO, INLINE, GI> SL;
+__device__ __forceinline__ void lds_raw(RawNode<PREC>& r, const char* slot, int lane, bool dens, uint32_t bT, bool rows) {
+  typedef Slots<PREC, TWO, INLINE, GI> SL;
   typedef typename Codec<PREC>::T T;
-  // field f's slot holds 64 values (64 sizeof(T) bytes); a 16-bit element of the
-  // x-halo wave is half (bT & 2) of its lane's dword
-  const char* at = (const char*)&slot[0][0] +
-                   (sizeof(T) == 2 && !rows ? (uint32_t)lane * 4u + (bT & 2u) : (uint32_t)lane * (uint32_t)sizeof(T));
+  typedef typename Aux<PREC>::T TA;
+  // a 16-bit element of the x-halo wave is half (bT & 2) of its lane's dword
+  const char* at = slot + (sizeof(T) == 2 && !rows ? (uint32_t)lane * 4u + (bT & 2u) : (uint32_t)lane * (uint32_t)sizeof(T));
+  const char* aa = slot + (uint32_t)lane * (uint32_t)sizeof(TA);
 #pragma unroll
-  for (int f = 0; f < 10; ++f) r.m[f] = *(const T*)(at + f * 64 * sizeof(T));
-  if (INLINE && TWO && dens) {
+  for (int f = 0; f < 10; ++f) r.m[f] = *(const T*)(at + f * SL::SB);
+  if (SL::NU > 0 && dens) {
 #pragma unroll
-    for (int f = 0; f < 3; ++f) r.uo[f] = *(const T*)(at + SL::UO * 256 + f * 64 * sizeof(T));
+    for (int f = 0; f < 3; ++f) r.uo[f] = *(const T*)(at + SL::U + f * SL::SB);
   }
-  if constexpr (TWO && !GI) r.phi = slot[SL::PHI][lane];
-  if constexpr (!INLINE) {
+  if constexpr (SL::NP > 0) r.phi = *(const TA*)(aa + SL::PHI);
+  if constexpr (GI) {
+    r.g[4] = *(const TA*)(aa + SL::G);
+  } else {
 #pragma unroll
-    for (int f = 0; f < 3; ++f) r.g[f] = slot[SL::G + f][lane];
-  } else if constexpr (GI) {
-    r.g[4] = slot[SL::G][lane];
-  } else if constexpr (TWO) {
-#pragma unroll
-    for (int f = 0; f < 5; ++f) r.g[f] = slot[SL::G + f][lane];
+    for (int f = 0; f < SL::NG; ++f) r.g[f] = *(const TA*)(aa + SL::G + f * SL::SA);
   }
 }
 
@@ -296,6 +269,12 @@ __device__ __forceinline__ void lds_raw(RawNode<PREC>& r, const float (*slot)[64
 // shared load/store counter makes a wait for everything) finds the older
 // stores long done.  The completed output plane is therefore stored at the
 // top of the following iteration.
+// Prefetching instances.  In 64-bit arithmetic the completed plane, held for one
+// iteration, spills beside the rest unless a lane has 256 registers: blocks of 5
+// rows (8 waves), whose slots also fit the 160 KB beside the y exchange.
+template <int PREC, int TY>
+constexpr bool fused_prefetch() { return sizeof(typename Codec<PREC>::R) == 4 || TY == 5; }
+
 // One block: tile `tile` (x fastest, then y, then z chunks) of the domain `a`.
 // OB: the domain has internal obstacles (node words, solid nodes, the
 // near-wall closures); without them that code is compiled out.
@@ -361,10 +340,10 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   typedef typename Aux<PREC>::T TA;
   constexpr int NW = TY + 2;  // row waves (TY output rows + 2 halo rows)
   constexpr int PB = prec_base(PREC);
-  constexpr bool PF = PB == PREC_FP32 || PB == PREC_FP16S || PB == PREC_BF16S;
   // GI: grad phi and lap phi formed here from a phi tile (fused_grad_inline)
-  constexpr bool GI = PF && TWO && INLINE && !OB;
-  typedef Slots<TWO, INLINE, GI> SL;
+  constexpr bool GI = (PB == PREC_FP32 || PB == PREC_FP16S || PB == PREC_BF16S) && TWO && INLINE && !OB;
+  typedef Slots<PREC, TWO, INLINE, GI> SL;
+  constexpr bool PF = fused_prefetch<PREC, TY>();
   // GI phi tile: rows y0-2 .. y0+TY+1 (tile row r holds y0-2+r), columns
   // x0-2 .. x0+65 (column c holds x0-2+c), both wrapped; a ring of four z
   // planes streamed by LDS DMA three planes ahead of the plane collided
@@ -373,7 +352,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   __shared__ R sUP[NW][9][64];
   __shared__ R sDN[NW][9][64];
   __shared__ R sHX[NW][2][9];
-  __shared__ float sPF[PF ? NW + 1 : 1][PF ? SL::N : 1][64];
+  __shared__ __align__(16) char sPF[PF ? NW + 1 : 1][PF ? SL::BYTES : 16];
   __shared__ float sPH[GI ? 4 : 1][GI ? GR : 1][GI ? GC : 1];
 
   const DevParams& dp = a.dp;
@@ -419,10 +398,15 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   off.u = ((uint32_t)xw + 3u * srow) * (uint32_t)sizeof(T);
   off.rows = halo_wave ? 0 : 1;
   off.g = ((uint32_t)xw + (uint32_t)GF * srow) * (uint32_t)sizeof(TA);
-  off.lm = off.rows ? off.m + row_off<T>(sx) : off.m & ~3u;
-  off.lu = off.rows ? off.u + row_off<T>(sx) : off.u & ~3u;
-  off.lg = off.rows ? off.g + row_off<float>(sx) : off.g;
   off.p = ((uint32_t)xw + (uint32_t)nx * (uint32_t)yw) * (uint32_t)sizeof(TA);
+  // (a dword of 64-bit values in the x-halo wave: lane l serves node l / 2)
+  auto node_at = [&](uint32_t o, size_t size) -> uint32_t {
+    return size == 8 ? (uint32_t)__shfl((int)o, lane >> 1) + 4u * (lane & 1) : o & ~3u;
+  };
+  off.lm = off.rows ? off.m + row_off<T>(sx) : node_at(off.m, sizeof(T));
+  off.lu = off.rows ? off.u + row_off<T>(sx) : node_at(off.u, sizeof(T));
+  off.lg = off.rows ? off.g + row_off<TA>(sx) : node_at(off.g, sizeof(TA));
+  off.lp = off.rows ? off.p + row_off<TA>(0) : node_at(off.p, sizeof(TA));
   const uint32_t splane = (uint32_t)sx * (uint32_t)ny;
   off.pm = ((10u * splane * (uint32_t)sizeof(T)) + 3u) & ~3u;
   off.pu = ((3u * splane * (uint32_t)sizeof(T)) + 3u) & ~3u;
@@ -470,7 +454,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   uint32_t lds0 = 0;
   uint32_t word_next = NODE_FLUID;
   if constexpr (PF) {
-    lds0 = lds_addr(&sPF[wave][0][0]);
+    lds0 = lds_addr((float*)&sPF[wave][0]);
     dma_raw<PREC, TWO, INLINE, GI>(a, wrapg(z0 - 1, nz), off, dens, lds0);
     if constexpr (OB) word_next = word_load(z0 - 1);
   }
@@ -994,6 +978,9 @@ static hipError_t launch_two(const FusedArgs& a, hipStream_t s) {
 template <int PREC, bool INLINE>
 static hipError_t launch_ty(const FusedArgs& a, hipStream_t s) {
   switch (a.ty) {
+    case 5:
+      if constexpr (PREC == PREC_FP64 || PREC == PREC_MIXED) return launch_two<PREC, INLINE, 5>(a, s);
+      else return hipErrorInvalidValue;
     case 8: return launch_two<PREC, INLINE, 8>(a, s);
     case 13: return launch_two<PREC, INLINE, 13>(a, s);
     default: return hipErrorInvalidValue;
@@ -1018,6 +1005,9 @@ static hipError_t batch_std(const FusedBatchEntry* tab, int ndom, int total, int
 template <int PREC>
 hipError_t fused_batch_prec(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool two, bool std, int ty,
                             hipStream_t s) {
+  if constexpr (PREC == PREC_FP64 || PREC == PREC_MIXED) {
+    if (ty == 5) return two ? batch_std<PREC, true, 5>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 5>(tab, ndom, total, lat, ho, std, s);
+  }
   if (ty == 8) return two ? batch_std<PREC, true, 8>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 8>(tab, ndom, total, lat, ho, std, s);
   if (ty == 13) return two ? batch_std<PREC, true, 13>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 13>(tab, ndom, total, lat, ho, std, s);
   return hipErrorInvalidValue;
@@ -1039,6 +1029,7 @@ template hipError_t fused_batch_prec<LBF_FUSED_PREC>(const FusedBatchEntry*, int
 
 int fused_tile_count(const FusedArgs& a) {
   switch (a.ty) {
+    case 5: return fused_tiles<5>(a);
     case 8: return fused_tiles<8>(a);
     case 13: return fused_tiles<13>(a);
   }

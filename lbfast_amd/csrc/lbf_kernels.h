@@ -52,7 +52,6 @@ struct StageArgs {
   void* frc;         // 3-field set
   void* pre;         // 5-field set of the fast path (phase-field prep output)
   int gf_from_pre;   // PHI_int_boundary: donor gradient from pre instead of aux
-  int grad_inline;   // the fused kernel forms grad phi and lap phi itself (fused_grad_inline)
   void* rep;         // REPULSIVE_FLUX: 6-field set, locaux 3..8 (partner index, flux)
   int8_t* rep_mask;  // REPULSIVE_FLUX: nx*ny*nz
   const int8_t* isfh;
@@ -106,7 +105,7 @@ int fused_tile_count(const FusedArgs& a);
 // std: std_switches() holds for every domain
 hipError_t launch_fused_batch(const FusedBatchEntry* dev_tab, int ndom, int total_tiles, int prec, int lattice,
                               bool highorder, bool two, bool std, int ty, hipStream_t s);
-int prep_tile_count(const StageArgs& a, int prec, int tz);
+int prep_tile_count(const StageArgs& a, int tz);
 hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int total_tiles, int prec, hipStream_t s);
 // the WetNode list from the haloed isfluid: counts the nodes into *count (list
 // null) or writes them

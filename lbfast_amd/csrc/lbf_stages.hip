@@ -9,7 +9,7 @@
 //   k_moments     moments_LB_kernel             (lb_cuda_moments_module.f90:19-341)
 //   k_update_phi  update_phifields_kernel       (lb_cuda_update_phi_module.f90:19-104)
 //   k_lb_int_bnd  LB_int_boundary_kernel        (lb_cuda_boundary_module.f90:19-216)
-//   k_phase_prep(_z)  compute_norm + compute_div_theta_n of the fast path in one
+//   k_phase_prep_z  compute_norm + compute_div_theta_n of the fast path in one
 //                 z-marching pass: phi planes and theta planes live in LDS,
 //                 the output per node is div(theta n) and, where the fused
 //                 kernel does not form them itself, grad phi (as n*|g|) and
@@ -138,131 +138,7 @@ __global__ void __launch_bounds__(BS) k_div(StageArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Fast-path phase-field prep: z-marching over a 64 x PTY tile.  Iteration k
-// loads phi(k+1), computes theta(k) on tile+1 (and grad/lap for the tile),
-// then div theta at plane k-1 from the theta ring.  Outputs (fluid nodes):
-// pre = {n_x |g|, n_y |g|, n_z |g|, lap phi, div(phi(1-phi) n)}.  theta is 0 at
-// non-fluid nodes: the reference never writes aux there and reads the
-// zero-initialised allocation.
-constexpr int PTX = 64, PTY = 8, PNT = PTX * PTY;
-
-template <int PREC>
-__global__ void __launch_bounds__(PNT) k_phase_prep(StageArgs a, int tz) {
-  typedef typename Codec<PREC>::R R;
-  typedef typename Aux<PREC>::T TA;
-  constexpr int SX = PTX + 4, SY = PTY + 4;   // phi plane with a 2-node halo
-  constexpr int TX = PTX + 2, TYY = PTY + 2;  // theta plane with a 1-node halo
-  constexpr int NRING = TX * TYY - PTX * PTY; // theta halo-ring nodes per plane
-  static_assert(NRING <= PNT, "one ring node per thread at most");
-  __shared__ R sphi[3][SY][SX];
-  __shared__ R sth[3][3][TYY][TX];
-
-  const DevParams& dp = a.dp;
-  const int nx = dp.nx, ny = dp.ny, nz = dp.nz;
-  const size_t nxny = (size_t)nx * ny;
-  const int sx = dp.sx;
-  const int tid = threadIdx.x;
-  const int ntx = (nx + PTX - 1) / PTX, nty = (ny + PTY - 1) / PTY, ntz = (nz + tz - 1) / tz;
-  const int tile = xcd_tile(blockIdx.x, ntx * nty * ntz);
-  const int x0 = (tile % ntx) * PTX, y0 = ((tile / ntx) % nty) * PTY;
-  const int z0 = (tile / (ntx * nty)) * tz, zend = min(z0 + tz, nz);
-  const TA* phi = (const TA*)a.phiS;
-  const R p1 = (R)(2.0 / 27.0), p2 = (R)(1.0 / 54.0), p3 = (R)(1.0 / 216.0), p0 = (R)(8.0 / 27.0);
-  const R THREE = 3, ONE = 1, TWO = 2;
-  const R eps = (R)1.0e-9;
-
-  auto slot3 = [](int k) { return ((k % 3) + 3) % 3; };
-  auto load_plane = [&](int z) {
-    const int zw = ((z % nz) + nz) % nz;
-    const int sl = slot3(z);
-    const TA* pz = phi + (size_t)zw * nxny;
-    for (int t = tid; t < SX * SY; t += PNT) {
-      const int ix = t % SX, iy = t / SX;
-      const int gx = (((x0 - 2 + ix) % nx) + nx) % nx, gy = (((y0 - 2 + iy) % ny) + ny) % ny;
-      sphi[sl][iy][ix] = (R)pz[(size_t)gx + (size_t)nx * gy];
-    }
-  };
-  // theta (and, for an interior node, grad/lap) of theta-plane node (jx,jy)
-  // at plane k from the phi slots; returns true if the node is fluid
-  auto theta_node = [&](int jx, int jy, int k, bool interior, R& gfx, R& gfy, R& gfz, R& lap) {
-    const int sm = slot3(k - 1), s0 = slot3(k), sp = slot3(k + 1);
-    const int8_t isf = isf_at(a.isfh, x0 - 1 + jx, y0 - 1 + jy, k, nx, ny, nz);
-    R thx = 0, thy = 0, thz = 0;
-    if (isf == 1 || isf == -1) {
-#define F(a_, b_, c_) sphi[(c_) < 0 ? sm : ((c_) > 0 ? sp : s0)][jy + 1 + (b_)][jx + 1 + (a_)]
-      const R gx = GRAD_X(F), gy = GRAD_Y(F), gz = GRAD_Z(F);
-      const R mg = sqrt(gx * gx + gy * gy + gz * gz);
-      const R im = rcp(mg + eps);
-      const R c = F(0, 0, 0);
-      const R nxv = gx * im, nyv = gy * im, nzv = gz * im;
-      thx = c * (ONE - c) * nxv; thy = c * (ONE - c) * nyv; thz = c * (ONE - c) * nzv;
-      if (interior) {
-        // the reference re-reads n and |g| from storage precision
-        const R mgs = (R)(TA)mg;
-        gfx = (R)(TA)nxv * mgs; gfy = (R)(TA)nyv * mgs; gfz = (R)(TA)nzv * mgs;
-        lap = LAPL(F, c);
-      }
-#undef F
-    }
-    sth[s0][0][jy][jx] = (R)(TA)thx;
-    sth[s0][1][jy][jx] = (R)(TA)thy;
-    sth[s0][2][jy][jx] = (R)(TA)thz;
-  };
-
-  load_plane(z0 - 2);
-  load_plane(z0 - 1);
-
-  // my interior node (tx,ty) is theta node (tx+1, ty+1); ring node `tid` if tid < NRING
-  const int tx = tid % PTX, ty = tid / PTX;
-  const int xg = x0 + tx, yg = y0 + ty;
-  const bool mine = xg < nx && yg < ny;
-  int rjx = 0, rjy = 0;
-  if (tid < NRING) {
-    if (tid < TX) { rjx = tid; rjy = 0; }
-    else if (tid < 2 * TX) { rjx = tid - TX; rjy = TYY - 1; }
-    else if (tid < 2 * TX + PTY) { rjx = 0; rjy = tid - 2 * TX + 1; }
-    else { rjx = TX - 1; rjy = tid - 2 * TX - PTY + 1; }
-  }
-  R gfx_c = 0, gfy_c = 0, gfz_c = 0, lap_c = 0;  // my node at plane k-1
-  for (int k = z0 - 1; k <= zend; ++k) {
-    load_plane(k + 1);
-    __syncthreads();
-    R gfx_n = 0, gfy_n = 0, gfz_n = 0, lap_n = 0;
-    theta_node(tx + 1, ty + 1, k, true, gfx_n, gfy_n, gfz_n, lap_n);
-    if (tid < NRING) {
-      R d0, d1, d2, d3;
-      theta_node(rjx, rjy, k, false, d0, d1, d2, d3);
-    }
-    __syncthreads();
-    // div theta at plane k-1 for my node
-    const int zo = k - 1;
-    if (mine && zo >= z0 && zo < zend) {
-      const int8_t isf = isf_at(a.isfh, xg, yg, zo, nx, ny, nz);
-      if (isf == 1 || isf == -1) {
-        const int tm = slot3(zo - 1), t0 = slot3(zo), tp = slot3(zo + 1);
-        const int jx = tx + 1, jy = ty + 1;
-#define X(a_, b_, c_) sth[(c_) < 0 ? tm : ((c_) > 0 ? tp : t0)][0][jy + (b_)][jx + (a_)]
-#define Y(a_, b_, c_) sth[(c_) < 0 ? tm : ((c_) > 0 ? tp : t0)][1][jy + (b_)][jx + (a_)]
-#define Z(a_, b_, c_) sth[(c_) < 0 ? tm : ((c_) > 0 ? tp : t0)][2][jy + (b_)][jx + (a_)]
-        const R d = (DX(X) + DY(Y) + DZ(Z)) * THREE;
-#undef X
-#undef Y
-#undef Z
-        const size_t o = sbase(5, xg, yg, zo, sx, ny);
-        TA* pre = (TA*)a.pre;
-        pre[o] = (TA)gfx_c;
-        pre[o + sx] = (TA)gfy_c;
-        pre[o + 2 * sx] = (TA)gfz_c;
-        pre[o + 3 * sx] = (TA)lap_c;
-        pre[o + 4 * sx] = (TA)d;
-      }
-    }
-    gfx_c = gfx_n; gfy_c = gfy_n; gfz_c = gfz_n; lap_c = lap_n;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Streaming fast-path phase-field prep (float phase-field storage).
+// Streaming fast-path phase-field prep.
 //
 // The stencils of k_norm / k_div (lb_cuda_auxfields_module.f90:72-130,
 // 1110-1160) in separable form (lbf_common.h): a plane's x pass (difference d,
@@ -288,8 +164,7 @@ __global__ void __launch_bounds__(PNT) k_phase_prep(StageArgs a, int tz) {
 // phi: theta is 0 at non-fluid nodes (the reference never writes aux there and
 // reads the zero-initialised allocation).
 // MODE: PREP_DIV stores div theta only (the fused kernel forms grad phi and lap
-// phi itself), PREP_WALL also grad phi at near-wall nodes (the donors of the
-// wetting update), PREP_ALL grad phi and lap phi everywhere.
+// phi itself, fused_grad_inline), PREP_ALL also grad phi and lap phi.
 //
 // What bounds it: instruction issue (it moves 8 bytes a node).  Two adjacent
 // rows a wave, the shared x passes, the running sums (no register moves of
@@ -297,20 +172,24 @@ __global__ void __launch_bounds__(PNT) k_phase_prep(StageArgs a, int tz) {
 // vector instructions a wave and plane; 0.70 -> 0.53 ms at 512^3, 106 -> 84 us at
 // 256^3, and with obstacles, where isfluid was gathered byte by byte and every
 // gather waited for the transfers in flight, 86 -> 55 us at 256x128x128 (with the
-// wetting update).
-enum PrepMode { PREP_DIV = 0, PREP_WALL = 1, PREP_ALL = 2 };
+// wetting update).  FP64 (two blocks a CU by LDS) ran the direct 27-point
+// stencils from LDS before: 129 -> 63 us at 160^3.
+enum PrepMode { PREP_DIV = 0, PREP_ALL = 1 };
 constexpr int QY = 12, QW = 7;
 constexpr int QR = QY + 4;                 // phi rows of a tile (2-row halo)
 constexpr int QT = QY + 2;                 // theta rows (1-row halo)
-constexpr int QH = 4;                      // halo columns each side
-constexpr int QC = 64 + 2 * QH;            // phi columns x0-4 .. x0+67
-constexpr int QP = QC / 4;                 // 16-byte pieces of a row
+// E values to a 16-byte piece: halo columns each side (2 at least), phi columns
+// x0 - H .. x0 + 63 + H, pieces of a row
+template <class TA>
+struct PrepTile {
+  static constexpr int E = 16 / sizeof(TA), H = E < 2 ? 2 : E, C = 64 + 2 * H, P = C / E;
+};
 constexpr int TC = 64 + 2;                 // theta columns x0-1 .. x0+64
 constexpr int WC = 68, WP = WC / 4;        // node words of a theta row (x0-1 .. x0+66) and their pieces
 constexpr int QDMA = (QR + QW - 1) / QW;   // phi rows each row wave streams per plane, a dword a lane
 constexpr int QNT = (QW + 1) * 64;         // threads: row waves + the edge-column wave
 static_assert(QT == 2 * QW, "two theta rows per wave");
-static_assert(QR * QP <= QNT && QT * WP <= QNT, "one 16-byte piece a thread");
+static_assert(QT * WP <= QNT, "one 16-byte piece a thread");
 
 __host__ __device__ inline int prep_tiles_z(const DevParams& dp, int tz) {
   return ((dp.nx + 63) / 64) * ((dp.ny + QY - 1) / QY) * ((dp.nz + tz - 1) / tz);
@@ -331,8 +210,10 @@ template <int PREC, int MODE, bool OB>
 __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile) {
   typedef typename Codec<PREC>::R R;
   typedef typename Aux<PREC>::T TA;
-  static_assert(sizeof(TA) == 4, "float phase-field storage");
-  __shared__ float sphi[4][QR][QC];
+  typedef PrepTile<TA> PT;
+  constexpr int QH = PT::H, QC = PT::C, QP = PT::P, QE = PT::E, NPASS = (QR * QP + QNT - 1) / QNT;
+  constexpr uint32_t SZ = (uint32_t)sizeof(TA);
+  __shared__ __align__(16) TA sphi[4][QR][QC];
   __shared__ R sth[2][3][QT][TC];
   __shared__ uint32_t swd[OB ? 2 : 1][OB ? QT : 1][OB ? WC : 1];
 
@@ -345,31 +226,38 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
   const int x0 = (tile % ntx) * 64, y0 = ((tile / ntx) % nty) * QY;
   const int z0 = (tile / (ntx * nty)) * tz, zend = min(z0 + tz, nz);
   const int XW = min(64, nx - x0);
-  const uint32_t pb = (uint32_t)nx * (uint32_t)ny * 4u;          // bytes of a phi plane
-  const uint32_t pbg = 5u * (uint32_t)sx * (uint32_t)ny * 4u;    // of a plane of the output set
+  const uint32_t pb = (uint32_t)nx * (uint32_t)ny * SZ;          // bytes of a phi plane
+  const uint32_t pbg = 5u * (uint32_t)sx * (uint32_t)ny * SZ;    // of a plane of the output set
   const uint32_t pbw = (uint32_t)(nx + 2) * (uint32_t)(ny + 2) * 4u;
-  const float* phi = (const float*)a.phiS;
+  const TA* phi = (const TA*)a.phiS;
   const R FOUR = 4, SIX = 6, ONE = 1, HALF = 0.5, G3 = (R)(3.0 / 216.0), L6 = (R)(6.0 / 216.0);
   const R eps = (R)1.0e-9;
   auto modn = [](int i, int n) { return ((i % n) + n) % n; };
 
   // ---- transfers ------------------------------------------------------------------
-  const bool quad = nx % 4 == 0 || (x0 >= QH && x0 + 64 + QH <= nx);
-  const uint32_t lds_phi = lds_addr(&sphi[0][0][0]);
-  uint32_t pq = 0, xh = 0, wq = 0;
+  const bool quad = nx % QE == 0 || (x0 >= QH && x0 + 64 + QH <= nx);
+  const uint32_t lds_phi = lds_addr((float*)&sphi[0][0][0]);
+  uint32_t pq[NPASS] = {}, xh = 0, wq = 0;
   uint32_t rowbyte[QDMA];
   if (quad) {
-    const int L = min((int)threadIdx.x, QR * QP - 1);
-    pq = ((uint32_t)modn(y0 - 2 + L / QP, ny) * (uint32_t)nx + (uint32_t)modn(x0 - QH + 4 * (L % QP), nx)) * 4u;
+#pragma unroll
+    for (int i = 0; i < NPASS; ++i) {
+      const int L = min((int)threadIdx.x + i * QNT, QR * QP - 1);
+      pq[i] = ((uint32_t)modn(y0 - 2 + L / QP, ny) * (uint32_t)nx + (uint32_t)modn(x0 - QH + QE * (L % QP), nx)) * SZ;
+    }
   } else {
-    // row waves stream rows wave + QW*i: 64 lanes to columns 4..67, and two
-    // lanes each to columns 2-3 (lanes 0-1) and 68-69 (lanes 2-3)
-    pq = (uint32_t)modn(x0 + lane, nx) * 4u;
-    xh = (uint32_t)modn((lane & 2) ? x0 + 62 + (lane & 3) : x0 - 2 + (lane & 1), nx) * 4u;
+    // row waves stream rows wave + QW*i: 64 lanes to the tile's own columns, and
+    // the lanes of two values each to the two columns left (low lanes) and
+    // right of them; a dword a lane, W dwords to a value
+    constexpr int W = SZ / 4;
+    pq[0] = (uint32_t)modn(x0 + lane / W, nx) * SZ + 4u * (uint32_t)(lane % W);
+    if constexpr (W == 2) pq[NPASS - 1] = (uint32_t)modn(x0 + 32 + lane / W, nx) * SZ + 4u * (uint32_t)(lane % W);
+    const int hl = lane & (4 * W - 1), hv = hl / W;
+    xh = (uint32_t)modn(hv < 2 ? x0 - 2 + hv : x0 + 62 + hv, nx) * SZ + 4u * (uint32_t)(hl % W);
 #pragma unroll
     for (int i = 0; i < QDMA; ++i) {
       const int r = wave + QW * i;
-      rowbyte[i] = __builtin_amdgcn_readfirstlane((uint32_t)modn(y0 - 2 + (r < QR ? r : 0), ny) * (uint32_t)nx * 4u);
+      rowbyte[i] = __builtin_amdgcn_readfirstlane((uint32_t)modn(y0 - 2 + (r < QR ? r : 0), ny) * (uint32_t)nx * SZ);
     }
   }
   if constexpr (OB) {
@@ -377,24 +265,35 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
     wq = ((uint32_t)(clampi(y0 - 1 + L / WP, -1, ny) + 1) * (uint32_t)(nx + 2) + (uint32_t)(x0 + 4 * (L % WP))) * 4u;
   }
   // transfers of one phi plane that this wave issues
-  const int nd = quad ? (wave * 64 < QR * QP ? 1 : 0) : (edge_wave ? 0 : 3 * ((QR - wave + QW - 1) / QW));
-  static_assert(QDMA == 3, "6 or 9 transfers a wave");
+  int nd = 0;
+  if (quad) {
+#pragma unroll
+    for (int i = 0; i < NPASS; ++i) nd += wave * 64 + i * QNT < QR * QP ? 1 : 0;
+  } else if (!edge_wave) {
+    nd = (SZ == 8 ? 4 : 3) * ((QR - wave + QW - 1) / QW);
+  }
+  static_assert(QDMA == 3 && (SZ == 4 || NPASS == 2), "6, 8, 9 or 12 transfers a wave");
   auto dma_plane = [&](int z) {
     const Rsrc rs = mkrsrc(plane_at(phi, pb, modn(z, nz)), pb);
-    const uint32_t base = lds_phi + (uint32_t)(z & 3) * (uint32_t)(QR * QC * 4);
+    const uint32_t base = lds_phi + (uint32_t)(z & 3) * (uint32_t)(QR * QC * SZ);
     if (quad) {
-      if ((int)threadIdx.x < QR * QP) dma_quad<0u>(rs, pq, 0u, base + (uint32_t)wave * 1024u);
+#pragma unroll
+      for (int i = 0; i < NPASS; ++i)
+        if ((int)threadIdx.x + i * QNT < QR * QP)
+          dma_quad<0u>(rs, pq[i], 0u, base + (uint32_t)(wave + i * (QNT / 64)) * 1024u);
       return;
     }
     if (edge_wave) return;
+    constexpr uint32_t W = SZ / 4;
 #pragma unroll
     for (int i = 0; i < QDMA; ++i) {
       const int r = wave + QW * i;
       if (r >= QR) continue;
-      const uint32_t l = base + (uint32_t)r * (uint32_t)(QC * 4);
-      dma_dword<16u>(rs, rowbyte[i] + pq, l);
-      if (lane < 2) dma_dword<8u>(rs, rowbyte[i] + xh, l);
-      if ((lane & ~1) == 2) dma_dword<66u * 4u>(rs, rowbyte[i] + xh, l);
+      const uint32_t l = base + (uint32_t)r * (uint32_t)(QC * SZ);
+      dma_dword<(uint32_t)QH * SZ>(rs, rowbyte[i] + pq[0], l);
+      if constexpr (W == 2) dma_dword<(uint32_t)QH * SZ + 256u>(rs, rowbyte[i] + pq[NPASS - 1], l);
+      if (lane < 2 * (int)W) dma_dword<(uint32_t)(QH - 2) * SZ>(rs, rowbyte[i] + xh, l);
+      if (lane >= 2 * (int)W && lane < 4 * (int)W) dma_dword<(uint32_t)(QH + 62) * SZ>(rs, rowbyte[i] + xh, l);
     }
   };
   const uint32_t lds_wd = OB ? lds_addr((float*)&swd[0][0][0]) : 0u;
@@ -418,9 +317,9 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
     const int t = 2 * wave + h;
     orow[h] = !edge_wave && t >= 1 && t <= QY && y0 - 1 + t < ny;
   }
-  const uint32_t go = ((uint32_t)(5 * (y0 - 1 + t0)) * (uint32_t)sx + (uint32_t)(x0 + lane)) * 4u;  // row h adds 20 sx
-  const uint32_t fb = (uint32_t)sx * 4u;
-  const float* phi_at = &sphi[0][t0][tj + QH - 2];
+  const uint32_t go = ((uint32_t)(5 * (y0 - 1 + t0)) * (uint32_t)sx + (uint32_t)(x0 + lane)) * SZ;  // row h adds 5 sx values
+  const uint32_t fb = (uint32_t)sx * SZ;
+  const TA* phi_at = &sphi[0][t0][tj + QH - 2];
   const uint32_t* word_at = OB ? &swd[0][t0][tj] : nullptr;
 
   // per theta row h: phi sums in flight -- (Px, dx1) give d/dx of the last
@@ -438,10 +337,14 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
   int late = nd;
   for (int k = z0 - 3; k <= zend + 1; ++k) {
     // phi(k+1) and the node words of plane k have landed
-    if (nd <= 1) dma_wait_n(late);
-    else if (late >= 9) dma_wait<9>();
-    else if (late >= 6) dma_wait<6>();
-    else dma_wait_all();
+    if (late >= 6) {
+      if (late >= 12) dma_wait<12>();
+      else if (late >= 9) dma_wait<9>();
+      else if (late >= 8) dma_wait<8>();
+      else dma_wait<6>();
+    } else {
+      dma_wait_n(late);
+    }
     __syncthreads();
     late = 0;
     // the slots of phi(k-1) and words(k-1) were last read before this barrier
@@ -470,7 +373,7 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
         Z[r].q = (z_ - zc) + (zp - zc);
         Z[r].c = zc;
       }
-      const Rsrc rg = mkrsrc(plane_at((float*)a.pre, pbg, zo < 0 ? 0 : zo), pbg);
+      const Rsrc rg = mkrsrc(plane_at((TA*)a.pre, pbg, zo < 0 ? 0 : zo), pbg);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const R A = G3 * ((X[h].d + FOUR * X[h + 1].d + X[h + 2].d) + (Y[h + 2].c - Y[h].c));
@@ -483,7 +386,7 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
         e1[h] = cc;
         if (orow[h] && zo >= z0 && zo < zend) {
           // obstacles: a solid node's value is never read
-          if (out_lane) bsts(rg, go + (uint32_t)h * 5u * fb, 4u * fb, (float)d);
+          if (out_lane) bsts(rg, go + (uint32_t)h * 5u * fb, 4u * fb, (TA)d);
           ++late;
         }
       }
@@ -495,7 +398,7 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
       const bool have_theta = k >= z0 - 1;
       const bool own = k >= z0 && k < zend;
       RowX<R> V[4];
-      const float* pv = phi_at + sp * (QR * QC);
+      const TA* pv = phi_at + sp * (QR * QC);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (edge_wave && r == 3) break;  // one row per lane
@@ -504,7 +407,7 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
         V[r].q = (vm - vc) + (vp - vc);
         V[r].c = vc;
       }
-      const Rsrc rg = mkrsrc(plane_at((float*)a.pre, pbg, own ? k : 0), pbg);
+      const Rsrc rg = mkrsrc(plane_at((TA*)a.pre, pbg, own ? k : 0), pbg);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (edge_wave && h == 1) break;  // wave-uniform
@@ -535,14 +438,13 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
             if (orow[h] && own) {
               // the reference re-reads n and |g| from storage precision
               const R mgs = (R)(TA)mg;
-              const bool st = out_lane && (MODE == PREP_ALL ? (word & NODE_FLUID) != 0 : (word & NODE_WALL) != 0);
+              const bool st = out_lane && (word & NODE_FLUID) != 0;
               if (st) {
                 const uint32_t o = go + (uint32_t)h * 5u * fb;
-                bsts(rg, o, 0u, (float)((R)(TA)nxv * mgs));
-                bsts(rg, o, fb, (float)((R)(TA)nyv * mgs));
-                bsts(rg, o, 2u * fb, (float)((R)(TA)nzv * mgs));
-                if constexpr (MODE == PREP_ALL)
-                  bsts(rg, o, 3u * fb, (float)(L6 * (s0[h] + FOUR * s1[h] + sp_) + ((c0[h] - c) + (cc - c))));
+                bsts(rg, o, 0u, (TA)((R)(TA)nxv * mgs));
+                bsts(rg, o, fb, (TA)((R)(TA)nyv * mgs));
+                bsts(rg, o, 2u * fb, (TA)((R)(TA)nzv * mgs));
+                bsts(rg, o, 3u * fb, (TA)(L6 * (s0[h] + FOUR * s1[h] + sp_) + ((c0[h] - c) + (cc - c))));
               }
             }
           }
@@ -1206,25 +1108,13 @@ static hipError_t prep_z(const StageArgs& a, int tz, hipStream_t s) {
 
 template <int PREC>
 static hipError_t prep_t(const StageArgs& a, int tz, hipStream_t s) {
-  if constexpr (sizeof(typename Aux<PREC>::T) == 4) {
-    if constexpr (PREC == PREC_MIXED) {
-      return a.dp.obst ? prep_z<PREC, PREP_ALL, true>(a, tz, s) : prep_z<PREC, PREP_ALL, false>(a, tz, s);
-    } else {
-      // without obstacles the fused kernel always forms its gradients itself
-      if (!a.dp.obst) return prep_z<PREC, PREP_DIV, false>(a, tz, s);
-      return a.grad_inline ? prep_z<PREC, PREP_WALL, true>(a, tz, s) : prep_z<PREC, PREP_ALL, true>(a, tz, s);
-    }
-  } else {
-    const dim3 grid(((a.dp.nx + PTX - 1) / PTX) * ((a.dp.ny + PTY - 1) / PTY) * ((a.dp.nz + tz - 1) / tz));
-    hipLaunchKernelGGL(k_phase_prep<PREC>, grid, dim3(PNT), 0, s, a, tz);
-  }
-  return hipGetLastError();
+  if (a.dp.obst) return prep_z<PREC, PREP_ALL, true>(a, tz, s);
+  // without obstacles the 32-bit fused kernels form their gradients themselves
+  constexpr int M = PREC == PREC_FP64 || PREC == PREC_MIXED ? PREP_ALL : PREP_DIV;
+  return prep_z<PREC, M, false>(a, tz, s);
 }
 
-int prep_tile_count(const StageArgs& a, int prec, int tz) {
-  if (prec == PREC_FP64) return -1;  // the FP64 prep is not batched
-  return prep_tiles_z(a.dp, tz);
-}
+int prep_tile_count(const StageArgs& a, int tz) { return prep_tiles_z(a.dp, tz); }
 
 hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int total_tiles, int prec, hipStream_t s) {
   const dim3 grid(total_tiles), block(QNT);
