@@ -554,8 +554,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
         const Part3<R> gpp = phi_part(zsrc + 1);
         R gx, gy, gz, lap;
         grad_lap(gpm, gp0, gpp, gx, gy, gz, lap);
-        const R mg = sqrt(gx * gx + gy * gy + gz * gz);
-        const R im = rcp(mg + (R)1.0e-9);
+        R mg, im;
+        grad_norm(gx * gx + gy * gy + gz * gz, mg, im);
         const R mgs = (R)(TA)mg;
         cur.g[0] = (TA)((R)(TA)(gx * im) * mgs);
         cur.g[1] = (TA)((R)(TA)(gy * im) * mgs);

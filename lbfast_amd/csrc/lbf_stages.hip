@@ -231,7 +231,6 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
   const uint32_t pbw = (uint32_t)(nx + 2) * (uint32_t)(ny + 2) * 4u;
   const TA* phi = (const TA*)a.phiS;
   const R FOUR = 4, SIX = 6, ONE = 1, HALF = 0.5, G3 = (R)(3.0 / 216.0), L6 = (R)(6.0 / 216.0);
-  const R eps = (R)1.0e-9;
   auto modn = [](int i, int n) { return ((i % n) + n) % n; };
 
   // ---- transfers ------------------------------------------------------------------
@@ -419,8 +418,8 @@ __device__ __forceinline__ void prep_body_z(const StageArgs& a, int tz, int tile
           const R c = c1[h];
           const R gx = G3 * (Px[h] + dxp), gy = G3 * (Py[h] + dyp);
           const R gz = G3 * (sp_ - s0[h]) + HALF * (cc - c0[h]);
-          const R mg = sqrt(gx * gx + gy * gy + gz * gz);
-          const R im = rcp(mg + eps);
+          R mg, im;
+          grad_norm(gx * gx + gy * gy + gz * gz, mg, im);
           const R nxv = gx * im, nyv = gy * im, nzv = gz * im;
           R th = c * (ONE - c);
           uint32_t word = NODE_FLUID;
