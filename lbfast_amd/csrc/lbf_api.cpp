@@ -659,6 +659,11 @@ static StageArgs stage_args(lbf_ctx* c) {
   return a;
 }
 
+// bytes of the state a step reads and writes
+static size_t state_bytes(const lbf_ctx* c) {
+  return 2 * ((c->p.twocomponent ? 13 : 10) * c->NS * c->tsz + (c->p.twocomponent ? c->N * c->asz : 0));
+}
+
 static FusedArgs fused_args(lbf_ctx* c) {
   FusedArgs a{};
   a.min = c->h[c->cur];
@@ -673,6 +678,7 @@ static FusedArgs fused_args(lbf_ctx* c) {
   a.dp = c->dp;
   a.ty = c->ty;
   a.tz = c->tz;
+  a.nt = stream_stores(state_bytes(c), c->dp.sx, c->tsz);
   a.seed = (uint32_t)c->step;
   a.seedp = nullptr;
   a.sopen = c->sopen;
@@ -994,6 +1000,8 @@ static int batch_tables(lbf_batch* b) {
   std::vector<int> order = b->order;
   b->nstd = (int)(std::stable_partition(order.begin(), order.end(),
                                         [&](int d) { return std_switches(b->ctx[d]->dp); }) - order.begin());
+  size_t all_bytes = 0;
+  for (lbf_ctx* c : b->ctx) all_bytes += state_bytes(c);
   for (int par = 0; par < 2; ++par) {
     std::vector<FusedBatchEntry> f(nd);
     std::vector<PrepBatchEntry> q(nd);
@@ -1011,6 +1019,7 @@ static int batch_tables(lbf_batch* b) {
       c->ucur ^= par;
       f[i].a = fused_args(c);
       f[i].a.ty = b->ty;
+      f[i].a.nt = stream_stores(all_bytes, c->dp.sx, c->tsz);
       f[i].a.tz = b->tz[d];
       // the seed of a step is the domain's step number, as in lbf_step:
       // 1 + the counter, which the step's tick advances afterwards

@@ -99,44 +99,43 @@ template <> __device__ __forceinline__ __hip_bfloat16 bld<__hip_bfloat16>(Rsrc r
 template <> __device__ __forceinline__ int8_t bld<int8_t>(Rsrc r, uint32_t boff) {
   return (int8_t)__builtin_amdgcn_raw_buffer_load_b8(r, boff, 0, 0);
 }
-__device__ __forceinline__ void bst(Rsrc r, uint32_t boff, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, boff, 0, 0);
-}
-__device__ __forceinline__ void bst(Rsrc r, uint32_t boff, double v) {
-  typedef decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0)) V2;
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, boff, 0, 0);
-}
-__device__ __forceinline__ void bst(Rsrc r, uint32_t boff, __half v) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, 0, 0);
-}
-__device__ __forceinline__ void bst(Rsrc r, uint32_t boff, __hip_bfloat16 v) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, 0, 0);
-}
-// ... with a wave-uniform byte offset added to every lane's (a scalar operand:
-// the fields of a set share one resource)
+// Stores, with a wave-uniform byte offset added to every lane's (a scalar operand:
+// the fields of a set share one resource).  AUX 2: streaming (non-temporal).
+template <int AUX = 0>
 __device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, float v) {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, boff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, boff, soff, AUX);
 }
+template <int AUX = 0>
 __device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, double v) {
   typedef decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0)) V2;
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, boff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V2, v), r, boff, soff, AUX);
 }
+template <int AUX = 0>
 __device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, __half v) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, AUX);
 }
+template <int AUX = 0>
 __device__ __forceinline__ void bsts(Rsrc r, uint32_t boff, uint32_t soff, __hip_bfloat16 v) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), r, boff, soff, AUX);
+}
+// the first NF fields (fstride bytes apart) of a set at one z plane
+template <class T, int NF>
+__device__ __forceinline__ void store_fields(T* plane0, uint32_t pbytes, uint32_t fstride, uint32_t boff, const T (&v)[NF],
+                                             bool nt) {
+  const Rsrc r = mkrsrc(plane0, pbytes);
+  if (nt) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) bsts<2>(r, boff, (uint32_t)f * fstride, v[f]);
+  } else {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) bsts<0>(r, boff, (uint32_t)f * fstride, v[f]);
+  }
 }
 // field f of a field set at one z plane
 template <class T>
 __device__ __forceinline__ T fld(const T* plane0, size_t fs, int f, uint32_t pbytes, uint32_t boff) {
   return bld<T>(mkrsrc(plane0 + (size_t)f * fs, pbytes), boff);
 }
-template <class T>
-__device__ __forceinline__ void fst(T* plane0, size_t fs, int f, uint32_t pbytes, uint32_t boff, T v) {
-  bsts(mkrsrc(plane0, pbytes), boff, (uint32_t)f * (uint32_t)(fs * sizeof(T)), v);
-}
-
 // LDS DMA.  buffer_load_dword with the lds modifier writes each lane's dword
 // to LDS at M0 + 4*lane instead of to a VGPR: a wave can stream the next
 // plane's inputs into its own LDS slots while it computes, at no register
@@ -470,39 +469,31 @@ __device__ __forceinline__ Mom<typename Codec<P>::R> load_mom_b(const typename C
   return o;
 }
 
-// Store of the ten moments; the 16-bit codecs round stochastically with the
-// per-node, per-plane seed rnd.
+// Store of the ten moments (nt: streaming); the 16-bit codecs round
+// stochastically with the per-node, per-plane seed rnd.
 template <int P>
 __device__ __forceinline__ void store_mom_b(typename Codec<P>::T* plane0, size_t fs, uint32_t pb, uint32_t boff,
-                                            const Mom<typename Codec<P>::R>& o, const DevParams& dp,
-                                            uint32_t rnd) {
+                                            const Mom<typename Codec<P>::R>& o, const DevParams& dp, uint32_t rnd,
+                                            bool nt) {
   typedef Codec<P> C; typedef typename C::R R; typedef typename C::T T;
+  const uint32_t fstride = (uint32_t)(fs * sizeof(T));
   if constexpr (C::dev) {
     // each field's random bits: the FP32 bits of the next field of the same
     // group (cyclic), XOR the seed
     const uint32_t rm = rnd & C::RBITS;
     auto sr = [&](float x, float xn) { return C::srx(x, (__float_as_uint(xn) & C::RBITS) ^ rm); };
     const float x0 = o.P * scl<P>(dp, 0), x1 = o.u * scl<P>(dp, 1), x2 = o.v * scl<P>(dp, 2), x3 = o.w * scl<P>(dp, 3);
-    fst(plane0, fs, 0, pb, boff, sr(x0, x1));
     const T tu = sr(x1, x2), tv = sr(x2, x3), tw = sr(x3, x0);
     const R ur = C::dec(tu, iscl<P>(dp, 1)), vr = C::dec(tv, iscl<P>(dp, 2)), wr = C::dec(tw, iscl<P>(dp, 3));
-    fst(plane0, fs, 1, pb, boff, tu); fst(plane0, fs, 2, pb, boff, tv); fst(plane0, fs, 3, pb, boff, tw);
     const float x4 = (o.xx - ur * ur) * scl<P>(dp, 4), x5 = (o.yy - vr * vr) * scl<P>(dp, 5);
     const float x6 = (o.zz - wr * wr) * scl<P>(dp, 6), x7 = (o.xy - ur * vr) * scl<P>(dp, 7);
     const float x8 = (o.xz - ur * wr) * scl<P>(dp, 8), x9 = (o.yz - vr * wr) * scl<P>(dp, 9);
-    fst(plane0, fs, 4, pb, boff, sr(x4, x5));
-    fst(plane0, fs, 5, pb, boff, sr(x5, x6));
-    fst(plane0, fs, 6, pb, boff, sr(x6, x7));
-    fst(plane0, fs, 7, pb, boff, sr(x7, x8));
-    fst(plane0, fs, 8, pb, boff, sr(x8, x9));
-    fst(plane0, fs, 9, pb, boff, sr(x9, x4));
+    const T v[10] = {sr(x0, x1), tu, tv, tw, sr(x4, x5), sr(x5, x6), sr(x6, x7), sr(x7, x8), sr(x8, x9), sr(x9, x4)};
+    store_fields(plane0, pb, fstride, boff, v, nt);
   } else {
-    fst(plane0, fs, 0, pb, boff, C::enc(o.P, 0.f));
-    fst(plane0, fs, 1, pb, boff, C::enc(o.u, 0.f)); fst(plane0, fs, 2, pb, boff, C::enc(o.v, 0.f));
-    fst(plane0, fs, 3, pb, boff, C::enc(o.w, 0.f));
-    fst(plane0, fs, 4, pb, boff, C::enc(o.xx, 0.f)); fst(plane0, fs, 5, pb, boff, C::enc(o.yy, 0.f));
-    fst(plane0, fs, 6, pb, boff, C::enc(o.zz, 0.f)); fst(plane0, fs, 7, pb, boff, C::enc(o.xy, 0.f));
-    fst(plane0, fs, 8, pb, boff, C::enc(o.xz, 0.f)); fst(plane0, fs, 9, pb, boff, C::enc(o.yz, 0.f));
+    const T v[10] = {C::enc(o.P, 0.f),  C::enc(o.u, 0.f),  C::enc(o.v, 0.f),  C::enc(o.w, 0.f),  C::enc(o.xx, 0.f),
+                     C::enc(o.yy, 0.f), C::enc(o.zz, 0.f), C::enc(o.xy, 0.f), C::enc(o.xz, 0.f), C::enc(o.yz, 0.f)};
+    store_fields(plane0, pb, fstride, boff, v, nt);
   }
 }
 

@@ -446,7 +446,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
     Mom<R> o;
     o.P = oc[0]; o.u = oc[1]; o.v = oc[2]; o.w = oc[3];
     o.xx = oc[4]; o.yy = oc[5]; o.zz = oc[6]; o.xy = oc[7]; o.xz = oc[8]; o.yz = oc[9];
-    store_mom_b<PREC>(plane_at(Sout, off.pm, zo), (size_t)sx, off.pm, off.m, o, dp, nseed ^ (uint32_t)zo * 0xC2B2AE35u);
+    store_mom_b<PREC>(plane_at(Sout, off.pm, zo), (size_t)sx, off.pm, off.m, o, dp, nseed ^ (uint32_t)zo * 0xC2B2AE35u, a.nt != 0);
   };
 
   const R third = (R)(1.0 / 3.0);
@@ -630,29 +630,27 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
               // open faces: the post-moments state of a first-layer node,
               // which the open-face correction reads after this launch (the
               // stage sequence reads it from S)
-              store_mom_b<PREC>(plane_at((T*)a.sopen, off.pm, zw), (size_t)sx, off.pm, off.m, m, dp, 0u);
+              store_mom_b<PREC>(plane_at((T*)a.sopen, off.pm, zw), (size_t)sx, off.pm, off.m, m, dp, 0u, false);
             }
           }
           if constexpr (TWO) {
             if (dens) {
-              T* uo = plane_at((T*)a.uout, off.pu, zw);
-              T eu = C::enc(m.u, scl<PREC>(dp, 1)), ev = C::enc(m.v, scl<PREC>(dp, 2)), ew = C::enc(m.w, scl<PREC>(dp, 3));
+              T e[3] = {C::enc(m.u, scl<PREC>(dp, 1)), C::enc(m.v, scl<PREC>(dp, 2)), C::enc(m.w, scl<PREC>(dp, 3))};
               if constexpr (C::dev) {
                 const uint32_t st = (nseed ^ (uint32_t)zw * 0x27D4EB2Fu) & C::RBITS;
                 const float xu = m.u * scl<PREC>(dp, 1), xv = m.v * scl<PREC>(dp, 2), xw_ = m.w * scl<PREC>(dp, 3);
-                eu = C::srx(xu, (__float_as_uint(xv) & C::RBITS) ^ st);
-                ev = C::srx(xv, (__float_as_uint(xw_) & C::RBITS) ^ st);
-                ew = C::srx(xw_, (__float_as_uint(xu) & C::RBITS) ^ st);
+                e[0] = C::srx(xu, (__float_as_uint(xv) & C::RBITS) ^ st);
+                e[1] = C::srx(xv, (__float_as_uint(xw_) & C::RBITS) ^ st);
+                e[2] = C::srx(xw_, (__float_as_uint(xu) & C::RBITS) ^ st);
               }
-              fst(uo, (size_t)sx, 0, off.pu, off.u, eu);
-              fst(uo, (size_t)sx, 1, off.pu, off.u, ev);
-              fst(uo, (size_t)sx, 2, off.pu, off.u, ew);
+              store_fields(plane_at((T*)a.uout, off.pu, zw), off.pu, (uint32_t)(sx * sizeof(T)), off.u, e, a.nt != 0);
             }
             // update_phi (update_phi:88-93), u after the moments stage
             const R t = -ph.sharp_c * dvt;
             const R po = phl - m.u * (R)0.5 * (gfx) - m.v * (R)0.5 * (gfy) - m.w * (R)0.5 * (gfz) +
                          ph.tau_diff * lap + t;
-            fst(plane_at((TA*)a.phiout, off.pp, zw), (size_t)sx, 0, off.pp, off.p, (TA)po);
+            const TA pv[1] = {(TA)po};
+            store_fields(plane_at((TA*)a.phiout, off.pp, zw), off.pp, 0u, off.p, pv, a.nt != 0);
           }
           if (OB && !bb && wall) {
             // LB_int_boundary (boundary:117-212) on the post-moments state: the

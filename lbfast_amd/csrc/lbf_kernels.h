@@ -18,6 +18,7 @@ struct FusedArgs {
   const uint32_t* words;  // obstacles: a word per node of the haloed isfluid (NODE_FLUID, lbf_physics.h)
   DevParams dp;
   int ty, tz;        // tile rows, z-chunk length
+  int nt;            // streaming stores of the new state (stream_stores)
   // 16-bit storage: the step's stochastic-rounding seed is seed (+ *seedp
   // when seedp is set: a device counter that captured graphs advance)
   uint32_t seed;
@@ -83,6 +84,18 @@ inline bool fused_grad_inline(int prec, const DevParams& dp) {
 // take the kernels that read the switches.
 inline bool std_switches(const DevParams& dp) {
   return !dp.smag && (!dp.twocomp || (dp.dens && dp.incomp && !dp.buoy));
+}
+
+// Streaming stores of the new state pay where it does not come back from the
+// 256 MB of memory-side cache in the next step, and cost where it would, or
+// where a row ends inside a 128-byte line.  Fused kernel without and with:
+// 512^3 two steps of three domains in turn 8.5 -> 7.8 ms (two components), 4.85
+// -> 4.5 (one); 256x128x128 channel 154 -> 149 us; 160^3 FP64 281 -> 268; but 128^3
+// 61 -> 65 us and 150x97x75 32 -> 37, 201x130x117 111 -> 113 (odd rows).  16-bit
+// values are bound by instruction issue and gain nothing (384x192x192 channel
+// 463 -> 474 us, 512^3 2.62 ms either way).
+inline bool stream_stores(size_t state_bytes, int sx, size_t value_bytes) {
+  return value_bytes >= 4 && state_bytes > ((size_t)256 << 20) && (size_t)sx * value_bytes % 128 == 0;
 }
 
 // Batched launches: one grid over many domains (same lattice, precision,
