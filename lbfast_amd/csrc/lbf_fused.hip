@@ -52,12 +52,12 @@
 // What bounds it: arithmetic and scalar issue, and HBM where the domain is
 // large.  Measured at 512^3 before and after the axis-by-axis order (27% fewer
 // vector instructions a launch), the 16-byte row transfers, the compiled-in
-// switches (std_switches) and one buffer resource per set (scalar instructions
-// of the plane loop 661 -> 367): two components FP32 3.81 -> 3.25 ms (15.0 GB of
-// compulsory state at 4.6 TB/s, the rate of a plain copy on the same card),
-// FP16S 3.15 -> 2.57 ms, one component FP32 2.76 -> 2.34 ms.  Registers decide
-// the variants: a spill inside the plane loop makes the compiler wait for every
-// transfer in flight (FP16S 2.57 -> 3.70 ms with 32 bytes of spills).
+// switches (std_switches), one buffer resource per set (scalar instructions
+// of the plane loop 661 -> 367) and streaming stores (stream_stores): two
+// components FP32 3.81 -> 3.18 ms (15.0 GB of compulsory state at 4.7 TB/s, the
+// rate of a plain copy), FP16S 3.15 -> 2.57 ms, one component 2.76 -> 2.20 ms.
+// Registers decide the variants: a spill inside the plane loop makes the compiler
+// wait for every transfer in flight (FP16S 2.57 -> 3.70 ms, 32 bytes of spills).
 //
 // Periodicity: indices wrap in-kernel (the reference's intpbc halo copies,
 // mpi_module.f90:2820-2918).  isfluid and the solid neighbours of near-wall
