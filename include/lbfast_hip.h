@@ -259,7 +259,8 @@ int lbf_last_step_timing(lbf_ctx* ctx, double* total_ms, double* fused_ms);
  * call.  Profilers and benchmarks turn it on; long production runs leave it off. */
 int lbf_set_timing(lbf_ctx* ctx, int32_t on);
 
-/* Fused-kernel tile shape override (0 = default/autotuned). */
+/* Fused-kernel tile shape override (0 = default): tile_y 8 or 13 rows, with
+ * 64-bit arithmetic (FP64, MIXED) also 5. */
 int lbf_set_tile(lbf_ctx* ctx, int32_t tile_y, int32_t tile_z);
 
 int32_t lbf_abi_version(void);
@@ -285,8 +286,8 @@ int lbf_batch_step(lbf_batch* b, int32_t nsteps);
 /* Capture nsteps (even, >= 2) steps into a hipGraph that later
  * lbf_batch_step calls replay; set_tile and autotune discard it. */
 int lbf_batch_capture(lbf_batch* b, int32_t nsteps);
-/* Row tile (8 or 13) of the fused kernel and z chunks of the fused and
- * phase-field kernels, for every domain (chunks clipped to each nz). */
+/* Row tile (as lbf_set_tile) of the fused kernel and z chunks of the fused
+ * and phase-field kernels, for every domain (chunks clipped to each nz). */
 int lbf_batch_set_tile(lbf_batch* b, int32_t tile_y, int32_t tile_z, int32_t tile_z_prep);
 /* The table order: order[i] is the domain whose tiles come i-th in the
  * grid of every launch (each XCD takes a contiguous eighth of it); a
@@ -294,10 +295,11 @@ int lbf_batch_set_tile(lbf_batch* b, int32_t tile_y, int32_t tile_z, int32_t til
 int lbf_batch_set_order(lbf_batch* b, const int32_t* order);
 /* Time trial_steps (even) steps of each candidate on the batch itself, keep
  * the fastest and restore every domain's state.  Searched in turn: the tiles
- * as they are and the row tiles with one z chunk for all domains (tile_y: the row
- * tile kept, tile_z: the fastest of the common chunks); the z
- * chunk of each size class (domains of one nz); the table order (as given,
- * largest first, largest and smallest alternating). */
+ * as they are and the row tiles with one z chunk for all domains; the z chunk
+ * of each size class (domains of one nz); the table order (as given, largest
+ * first, largest and smallest alternating).  tile_y: the row tile kept; tile_z:
+ * the common chunk that was the fastest with it, so that lbf_batch_set_tile
+ * takes the pair (lbf_batch_tiles tells what is kept). */
 int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* tile_y, int32_t* tile_z);
 /* The batch's current choices: row tile, and per domain (arrays of
  * ndomains) the fused and phase-field z chunks and the table order. */

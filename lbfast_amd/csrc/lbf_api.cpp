@@ -274,6 +274,16 @@ constexpr int FUSED_EXTRA = 3;
 constexpr double T8 = 0.72, T5 = 0.72;
 static long fused_xy(const lbf_params& p, int ty) { return (long)((p.nx + 63) / 64) * ((p.ny + ty - 1) / ty); }
 static bool wide_arith(int prec) { return prec == LBF_PREC_FP64 || prec == LBF_PREC_MIXED; }
+// row tiles that the fused kernel is compiled for, in 32 and in 64 bits
+static const std::vector<int>& row_tiles(int prec) {
+  static const std::vector<int> narrow = {8, 13}, wide = {5, 8, 13};
+  return wide_arith(prec) ? wide : narrow;
+}
+static bool row_tile_ok(int prec, int ty) {
+  const std::vector<int>& t = row_tiles(prec);
+  return std::find(t.begin(), t.end(), ty) != t.end();
+}
+static const char* row_tile_text(int prec) { return wide_arith(prec) ? "5, 8 or 13" : "8 or 13"; }
 // Three blocks of the 16/32-bit phase prep fit a CU (measured plane times 1.65,
 // 2.2, 2.9 us with one to three), two of the FP64 prep.
 static const double T_PREP[3] = {1.0, 1.34, 1.75};
@@ -438,7 +448,7 @@ int lbf_create(const lbf_params* pin, lbf_ctx** out) {
 int lbf_set_tile(lbf_ctx* c, int32_t ty, int32_t tz) {
   if (!c) return LBF_EINVAL;
   if (ty == 0 && tz == 0) { default_tiles(c); return LBF_OK; }
-  if (ty != 0 && ty != 8 && ty != 13) return fail(c, LBF_EINVAL, "tile_y must be 8 or 13");
+  if (ty != 0 && !row_tile_ok(c->prec, ty)) return fail(c, LBF_EINVAL, "tile_y must be %s", row_tile_text(c->prec));
   if (ty) c->ty = ty;
   if (tz) {
     if (tz < 1) return fail(c, LBF_EINVAL, "tile_z must be >= 1");
@@ -1206,7 +1216,7 @@ const char* lbf_batch_last_error(const lbf_batch* b) { return b ? b->err.c_str()
 
 int lbf_batch_set_tile(lbf_batch* b, int32_t ty, int32_t tz, int32_t tz_prep) {
   if (!b) return LBF_EINVAL;
-  if (ty != 8 && ty != 13) return bfail(b, LBF_EINVAL, "tile_y must be 8 or 13");
+  if (!row_tile_ok(b->prec, ty)) return bfail(b, LBF_EINVAL, "tile_y must be %s", row_tile_text(b->prec));
   if (tz < 1 || tz_prep < 1) return bfail(b, LBF_EINVAL, "z chunks must be >= 1");
   BHIPCHK(b, hipStreamSynchronize(b->stream));
   b->ty = ty;
@@ -1316,9 +1326,11 @@ int lbf_batch_timing(lbf_batch* b, double* ms) {
 // The project's autotuner: times `trial_steps` (even) steps of each candidate
 // on the batch itself, keeps the fastest, and restores every domain's state
 // afterwards.  Candidates, searched in turn: the tiles as they are, or a row tile
-// (8 or 13) with one z chunk (16..128) for every domain; then the z chunk of each size class
-// (domains of one nz) with the others held; then the table order (as given,
-// largest first, or largest and smallest alternating).
+// (row_tiles) with one z chunk (16..128) for every domain; then the z chunk of
+// each size class (domains of one nz) with the others held; then the table order
+// (as given, largest first, or largest and smallest alternating).  Reported: the
+// row tile kept and the common chunk that was the fastest with that row tile, a
+// pair that was timed.
 int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int32_t* best_tz) {
   if (!b) return LBF_EINVAL;
   if (trial_steps < 2 || (trial_steps & 1)) return bfail(b, LBF_EINVAL, "trial_steps must be even and >= 2");
@@ -1370,24 +1382,28 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
   };
   batch_drop_graph(b);
   // 1. the current tiles, or a row tile and one z chunk for every domain
-  const int tys[2] = {8, 13}, tzs[4] = {16, 32, 64, 128};
+  const int tzs[4] = {16, 32, 64, 128};
   const std::vector<int> tz0 = b->tz, tzp0 = b->tz_prep;
-  double best = 1e300, ubest = 1e300;
-  int bty = b->ty, btz = 0, utz = tzs[0];  // utz: the fastest uniform chunk, reported
+  double best = 1e300;
+  int bty = b->ty, btz = 0;
+  std::vector<std::pair<int, int>> common;  // each row tile's fastest common chunk
   {
     int rc = trial(&best);
     if (rc) { release(); return rc; }
   }
-  for (int ty : tys)
+  for (int ty : row_tiles(b->prec)) {
+    double ubest = 1e300;
+    common.emplace_back(ty, tzs[0]);
     for (int tz : tzs) {
       b->ty = ty;
       set_uniform(tz);
       double m = 0;
       int rc = trial(&m);
       if (rc) { release(); return rc; }
-      if (m < ubest) { ubest = m; utz = tz; }
+      if (m < ubest) { ubest = m; common.back().second = tz; }
       if (m < best) { best = m; bty = ty; btz = tz; }
     }
+  }
   b->ty = bty;
   if (btz) {
     set_uniform(btz);
@@ -1458,7 +1474,9 @@ int lbf_batch_autotune(lbf_batch* b, int32_t trial_steps, int32_t* best_ty, int3
   int rc = batch_tables(b);
   if (rc) return rc;
   if (best_ty) *best_ty = b->ty;
-  if (best_tz) *best_tz = utz;
+  if (best_tz)
+    for (const auto& t : common)
+      if (t.first == b->ty) *best_tz = t.second;
   b->timing_valid = false;
   return LBF_OK;
 }
