@@ -57,7 +57,6 @@ struct lbf_ctx {
   int cur = 0, ucur = 0;
   int step = 0;
   bool initialized = false;
-  bool isf_set = false;
   bool raw_pending = false;
   int ty = 8, tz = 0, tz_prep = 64;
   std::vector<hipEvent_t> evs;  // per-launch event pairs (lbf_set_timing)
@@ -611,29 +610,38 @@ int lbf_upload_isfluid(lbf_ctx* c, const int8_t* host) {
         h[(size_t)i + (size_t)hx * ((size_t)j + (size_t)hy * k)] =
             one ? 1 : host[(size_t)c3[0] + (size_t)nx * ((size_t)c3[1] + (size_t)ny * c3[2])];
       }
-  HIPCHK(c, hipMemcpy(c->isfh, h.data(), h.size(), hipMemcpyHostToDevice));
-  if (c->words) HIPCHK(c, launch_node_words(c->isfh, c->words, c->dp, c->stream));
-  if (c->wet_count) {
-    // the wetting list: count, allocate, write (an empty one for no solid node)
-    c->nwet = 0;
-    uint32_t n = 0;
-    if (any_solid) {
-      HIPCHK(c, launch_fill_zero(c->wet_count, sizeof n, c->stream));
-      HIPCHK(c, launch_wet_list(c->isfh, nullptr, c->wet_count, c->dp, c->prec, c->stream));
-      HIPCHK(c, hipMemcpyAsync(&n, c->wet_count, sizeof n, hipMemcpyDeviceToHost, c->stream));
-    }
+  // What can fail for want of memory comes before the first change: after an
+  // error the domain keeps the isfluid, the words and the wetting list it had.
+  // The new isfluid waits in the staging buffer, whose 8 bytes a node hold the
+  // halo too (at least two nodes an axis).
+  const int8_t* isf = (const int8_t*)c->staging;
+  HIPCHK(c, hipMemcpyAsync(c->staging, h.data(), h.size(), hipMemcpyHostToDevice, c->stream));
+  void* wet = nullptr;
+  uint32_t n = 0;
+  if (c->wet_count && any_solid) {
+    // the wetting list: count, allocate, write
+    HIPCHK(c, launch_fill_zero(c->wet_count, sizeof n, c->stream));
+    HIPCHK(c, launch_wet_list(isf, nullptr, c->wet_count, c->dp, c->prec, c->stream));
+    HIPCHK(c, hipMemcpyAsync(&n, c->wet_count, sizeof n, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (c->wet) HIPCHK(c, hipFree(c->wet));
-    c->wet = nullptr;
     if (n) {
-      HIPCHK(c, hipMalloc(&c->wet, (size_t)n * wet_node_size(c->prec)));
-      HIPCHK(c, launch_fill_zero(c->wet_count, sizeof n, c->stream));
-      HIPCHK(c, launch_wet_list(c->isfh, c->wet, c->wet_count, c->dp, c->prec, c->stream));
+      hipError_t e = hipMalloc(&wet, (size_t)n * wet_node_size(c->prec));
+      if (e == hipSuccess) e = launch_fill_zero(c->wet_count, sizeof n, c->stream);
+      if (e == hipSuccess) e = launch_wet_list(isf, wet, c->wet_count, c->dp, c->prec, c->stream);
+      if (e != hipSuccess) {
+        if (wet) hipFree(wet);
+        hipGetLastError();  // not to be met by the next launch's check
+        return fail(c, LBF_EHIP, "wetting list of %u nodes: %s", n, hipGetErrorString(e));
+      }
     }
-    c->nwet = n;
   }
+  void* old = c->wet;
+  c->wet = wet;
+  c->nwet = n;
+  HIPCHK(c, launch_copy(c->isfh, isf, h.size(), c->stream));
+  if (c->words) HIPCHK(c, launch_node_words(c->isfh, c->words, c->dp, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->isf_set = true;
+  if (old) HIPCHK(c, hipFree(old));
   return LBF_OK;
 }
 
