@@ -260,19 +260,14 @@ static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t
   return best;
 }
 
-// One block of the fused kernel fits a CU.  A plane of an 8-row block takes
-// 0.72 of a 13-row block's time (measured 0.66 at 512^3, where HBM counts, to
-// 0.81 at 64^3).  In 64-bit arithmetic the prefetching kernel needs 256 registers
-// a lane, blocks of 5 rows; with two components or obstacles they are the
-// faster (160^3 FP64 276 us against 309 with 8 rows and 560 with 13, which
-// spills; MIXED 208 against 218; FP64 channel 128x96x96 106 against 159), with
-// one component about even, a plane of 5 rows at 0.55 (256^3) to 0.75 (64^3) of
-// one of 8.
 static const double T_FUSED[1] = {1.0};
 constexpr int FUSED_EXTRA = 3;
-constexpr double T8 = 0.72, T5 = 0.72;
 static long fused_xy(const lbf_params& p, int ty) { return (long)((p.nx + 63) / 64) * ((p.ny + ty - 1) / ty); }
 static bool wide_arith(int prec) { return prec == LBF_PREC_FP64 || prec == LBF_PREC_MIXED; }
+// bytes of the state a step reads and writes
+static size_t state_bytes(const lbf_ctx* c) {
+  return 2 * ((c->p.twocomponent ? 13 : 10) * c->NS * c->tsz + (c->p.twocomponent ? c->N * c->asz : 0));
+}
 // row tiles that the fused kernel is compiled for, in 32 and in 64 bits
 static const std::vector<int>& row_tiles(int prec) {
   static const std::vector<int> narrow = {8, 13}, wide = {5, 8, 13};
@@ -283,6 +278,30 @@ static bool row_tile_ok(int prec, int ty) {
   return std::find(t.begin(), t.end(), ty) != t.end();
 }
 static const char* row_tile_text(int prec) { return wide_arith(prec) ? "5, 8 or 13" : "8 or 13"; }
+// The row tiles that a domain's default is chosen from, each with the time of a
+// block's plane (in units of one of them); of equal makespans the first.
+struct RowTile { int rows; double plane; };
+static std::vector<RowTile> row_choices(const lbf_ctx* c) {
+  // 32 and 16 bits: a plane of 8 rows takes 0.72 of one of 13 (measured 0.66 at
+  // 512^3, where HBM counts, to 0.81 at 64^3)
+  if (!wide_arith(c->prec)) return {{13, 1.0}, {8, 0.72}};
+  // 64-bit arithmetic.  The prefetching kernel needs up to 256 registers a lane,
+  // blocks of 5 rows; with two components or obstacles they are the faster
+  // (160^3 FP64 276 us against 309 with 8 rows and 560 with 13, which spills;
+  // MIXED 208 against 218; FP64 channel 128x96x96 106 against 159)
+  if (c->p.twocomponent || c->p.internal_obstacles) return {{5, 1.0}};
+  // One component: the other tiles do not prefetch, which costs most where the
+  // state does not stay in the 256 MB of memory-side cache.  A plane of 5 rows
+  // against one of 8: FP64 0.64-0.73 (D3Q19), 0.66-0.77 (D3Q27) in the cache and
+  // 0.49-0.58 beyond, MIXED 0.73-0.80 and 0.60-0.62.
+  const bool beyond = state_bytes(c) > ((size_t)256 << 20), d19 = c->p.lattice == 19;
+  const double t5 = c->prec == LBF_PREC_FP64 ? (beyond ? 0.52 : d19 ? 0.67 : 0.72) : (beyond ? 0.61 : 0.76);
+  // D3Q19 does not spill with 13 rows: 1.37-1.5 (D3Q27 1.6 and more).  176x268x32
+  // 56.7 us with 5 rows, 60.3 with 8, 52.4 with 13 (MIXED 54.9, 49.0, 42.7); 192^3
+  // 226, 288, 270 (MIXED 182, 191, 178); 150x97x75 45.9, 50.4, 47.5
+  if (d19) return {{8, 1.0}, {5, t5}, {13, 1.4}};
+  return {{8, 1.0}, {5, t5}};
+}
 // Three blocks of the 16/32-bit phase prep fit a CU (measured plane times 1.65,
 // 2.2, 2.9 us with one to three), two of the FP64 prep.
 static const double T_PREP[3] = {1.0, 1.34, 1.75};
@@ -295,19 +314,15 @@ static const double T_PREP64[2] = {1.0, 1.5};
 // 32^3 36.8 -> 17.9 us, 64^3 46.8 -> 22.2, 128^3 92.5 -> 62.2, 201x130x117
 // 149 -> 113, 256^3 FP16S 435 -> 353, 160^3 FP64 678 -> 311.
 static void default_tiles(lbf_ctx* c) {
-  int tz8 = 1, tz13 = 1;
-  if (wide_arith(c->prec)) {
-    int tz5 = 1;
-    const double c5 = T5 * pick_chunk(fused_xy(c->p, 5), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz5);
-    const double c8 = pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
-    const bool r5 = c->p.twocomponent || c->p.internal_obstacles || c5 < c8;
-    c->ty = r5 ? 5 : 8;
-    c->tz = r5 ? tz5 : tz8;
-  } else {
-    const double c8 = T8 * pick_chunk(fused_xy(c->p, 8), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz8);
-    const double c13 = pick_chunk(fused_xy(c->p, 13), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz13);
-    c->ty = c8 < c13 ? 8 : 13;
-    c->tz = c8 < c13 ? tz8 : tz13;
+  double best = 1e300;
+  for (const RowTile& t : row_choices(c)) {
+    int tz = 1;
+    const double cost = t.plane * pick_chunk(fused_xy(c->p, t.rows), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz);
+    if (cost < best) {
+      best = cost;
+      c->ty = t.rows;
+      c->tz = tz;
+    }
   }
   // prep blocks: 64 x 12 tiles that march 5 planes beyond their chunk (theta and
   // phi halo planes, one step of store lag)
@@ -675,11 +690,6 @@ static StageArgs stage_args(lbf_ctx* c) {
     a.obc_val[f][3] = c->p.openbc_w[f];
   }
   return a;
-}
-
-// bytes of the state a step reads and writes
-static size_t state_bytes(const lbf_ctx* c) {
-  return 2 * ((c->p.twocomponent ? 13 : 10) * c->NS * c->tsz + (c->p.twocomponent ? c->N * c->asz : 0));
 }
 
 static FusedArgs fused_args(lbf_ctx* c) {
@@ -1138,19 +1148,27 @@ static void batch_default_tiles(lbf_batch* b) {
     }
     return best;
   };
-  int T8b = 1, T13b = 1, Tp = 1;
-  if (wide_arith(b->prec)) {
-    b->ty = b->two ? 5 : 8;
-    search(b->ty, FUSED_EXTRA, 1, &T8b);
-  } else {
-    const double c8 = T8 * search(8, FUSED_EXTRA, 1, &T8b), c13 = search(13, FUSED_EXTRA, 1, &T13b);
-    b->ty = c8 < c13 ? 8 : 13;
+  double best = 1e300;
+  int Tf = 1, Tp = 1;
+  std::vector<RowTile> rows = row_choices(b->ctx[0]);
+  // One component in 64 bits: this estimate does not tell 5 rows from 8 (20 domains
+  // of 64^3 205 us against 244 in FP64 D3Q19, but 209 against 181 in MIXED D3Q27;
+  // 6 of 32^3 33 against 24), the autotuner does.
+  if (wide_arith(b->prec) && !b->two) rows = {{8, 1.0}};
+  for (const RowTile& t : rows) {
+    int T = 1;
+    const double cost = t.plane * search(t.rows, FUSED_EXTRA, 1, &T);
+    if (cost < best) {
+      best = cost;
+      b->ty = t.rows;
+      Tf = T;
+    }
   }
   search(12, 5, 3, &Tp);
   b->tz.clear();
   b->tz_prep.clear();
   for (lbf_ctx* c : b->ctx) {
-    b->tz.push_back(chunk(c->p.nz, b->ty == 13 ? T13b : T8b));
+    b->tz.push_back(chunk(c->p.nz, Tf));
     b->tz_prep.push_back(chunk(c->p.nz, Tp));
   }
 }

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from lbfast_amd import build, hip
-from lbfast_amd.params import make_params, PREC_FP32
+from lbfast_amd.params import make_params, PREC_FP32, PREC_FP64, PREC_MIXED
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -62,4 +62,22 @@ def test_failed_upload_of_isfluid_changes_nothing(stub):
     d.upload_isfluid(np.ones_like(a))
     d.step(1)
     assert _wetting(stub)[0] == _wetting(stub)[2] == 0
+    d.close()
+
+
+@pytest.mark.parametrize("n,prec,lattice,rows", [
+    # one component in 64-bit arithmetic: the rows that were the fastest of 5, 8 and
+    # 13, each with its best chunk (D3Q27 has 13 rows spill)
+    ((176, 268, 32), PREC_FP64, 19, 13), ((50, 275, 85), PREC_FP64, 19, 13), ((100, 100, 100), PREC_FP64, 19, 5),
+    ((192, 192, 192), PREC_FP64, 19, 5), ((176, 268, 32), PREC_MIXED, 19, 13), ((64, 64, 64), PREC_MIXED, 19, 8),
+    ((192, 192, 192), PREC_MIXED, 19, 13), ((192, 192, 192), PREC_FP64, 27, 5), ((176, 268, 32), PREC_MIXED, 27, 8),
+    ((192, 192, 192), PREC_MIXED, 27, 5)])
+def test_rows_of_64_bit_domains(stub, n, prec, lattice, rows):
+    p = make_params(n, lattice=lattice, highorder=lattice == 27, precision=prec)
+    d = hip.Domain(p)
+    d.init_state()
+    d.step(1)
+    ty, tz = ctypes.c_int(), ctypes.c_int()
+    stub.stub_fused_tile(ctypes.byref(ty), ctypes.byref(tz))
+    assert ty.value == rows
     d.close()
