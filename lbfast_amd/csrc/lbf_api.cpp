@@ -260,6 +260,11 @@ static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t
   return best;
 }
 
+// The fused kernel's blocks are counted one to a CU.  Only the 8-row blocks of
+// one-component D3Q19 in 32 and 16 bits leave room for a second (76 registers, 75 KB
+// of LDS); counting on it would change little: the best 8-row chunks with two on a
+// CU against 13 rows 26.2 and 26.4 us at 100^3, 30.6 and 29.7 at 176x268x32, 122 and
+// 119 at 192^3, 27.4 and 28.4 at 150x97x75 (FP32).
 static const double T_FUSED[1] = {1.0};
 constexpr int FUSED_EXTRA = 3;
 static long fused_xy(const lbf_params& p, int ty) { return (long)((p.nx + 63) / 64) * ((p.ny + ty - 1) / ty); }
@@ -302,10 +307,15 @@ static std::vector<RowTile> row_choices(const lbf_ctx* c) {
   if (d19) return {{8, 1.0}, {5, t5}, {13, 1.4}};
   return {{8, 1.0}, {5, t5}};
 }
-// Three blocks of the 16/32-bit phase prep fit a CU (measured plane times 1.65,
-// 2.2, 2.9 us with one to three), two of the FP64 prep.
+// Blocks of the phase prep on a CU: three of the 16/32-bit prep (measured plane
+// times 1.65, 2.2, 2.9 us with one to three); in 64-bit arithmetic its 118 to 124
+// registers leave two, in FP64 with obstacles its 87 KB of LDS one.
 static const double T_PREP[3] = {1.0, 1.34, 1.75};
 static const double T_PREP64[2] = {1.0, 1.5};
+static int prep_slots(const lbf_ctx* c, const double** t) {
+  *t = wide_arith(c->prec) ? T_PREP64 : T_PREP;
+  return !wide_arith(c->prec) ? 3 : c->prec == LBF_PREC_FP64 && c->p.internal_obstacles ? 1 : 2;
+}
 
 // Chunks that fill the CUs in whole rounds.  The rule before aimed at 1024
 // blocks and at least 8 planes a chunk, which left small domains a serial march
@@ -329,8 +339,9 @@ static void default_tiles(lbf_ctx* c) {
   StageArgs one{};
   one.dp = c->dp;
   const long pt = prep_tile_count(one, c->p.nz);
-  if (c->prec == LBF_PREC_FP64) pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP64, 2, &c->tz_prep);
-  else pick_chunk(pt, c->p.nz, c->ncu, 5, T_PREP, 3, &c->tz_prep);
+  const double* t;
+  const int slots = prep_slots(c, &t);
+  pick_chunk(pt, c->p.nz, c->ncu, 5, t, slots, &c->tz_prep);
 }
 
 int lbf_create(const lbf_params* pin, lbf_ctx** out) {
@@ -1164,6 +1175,8 @@ static void batch_default_tiles(lbf_batch* b) {
       Tf = T;
     }
   }
+  // (three slots also in MIXED, where two fit: in this estimate of throughput that
+  // is the better: 20 domains of 64^3 350 us against 357, 32 and 2 x 128 279 against 287)
   search(12, 5, 3, &Tp);
   b->tz.clear();
   b->tz_prep.clear();

@@ -9,10 +9,12 @@
 static long g_left = -1;  // allocations until hipMalloc fails; -1: never
 static lbf::FusedArgs g_fused;
 static lbf::StageArgs g_wetting;
+static int g_prep_tz;
 
 extern "C" {
 void stub_fail_after(long n) { g_left = n; }
 void stub_fused_tile(int* ty, int* tz) { *ty = g_fused.ty; *tz = g_fused.tz; }
+int stub_prep_chunk() { return g_prep_tz; }
 // of the last wetting update: the list's length, and the haloed isfluid's sum and
 // number of wall words
 void stub_wetting(long* out) {
@@ -83,7 +85,7 @@ hipError_t launch_node_words(const int8_t* isfh, uint32_t* words, const DevParam
 hipError_t launch_fill_zero(void* p, size_t n, hipStream_t) { if (n < 64) memset(p, 0, n); return hipSuccess; }
 hipError_t launch_copy(void* d, const void* s, size_t n, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
 hipError_t launch_fused_batch(const FusedBatchEntry*, int, int, int, int, bool, bool, bool, int, hipStream_t) { return hipSuccess; }
-hipError_t launch_phase_prep(const StageArgs&, int, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_phase_prep(const StageArgs&, int, int tz, hipStream_t) { g_prep_tz = tz; return hipSuccess; }
 hipError_t launch_phase_prep_batch(const PrepBatchEntry*, int, int, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_encode_moments(void*, const float*, const DevParams&, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_decode_field(const void*, int, void*, int, const DevParams&, int, hipStream_t) { return hipSuccess; }

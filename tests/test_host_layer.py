@@ -81,3 +81,19 @@ def test_rows_of_64_bit_domains(stub, n, prec, lattice, rows):
     stub.stub_fused_tile(ctypes.byref(ty), ctypes.byref(tz))
     assert ty.value == rows
     d.close()
+
+
+@pytest.mark.parametrize("prec,obstacles,n,fit", [
+    # (measured 258 -> 250, 193 -> 188, 84.5 -> 82.8 and 72.8 -> 71.3 us a step)
+    (PREC_FP64, 1, (131, 233, 48), 1), (PREC_FP64, 1, (171, 114, 67), 1), (PREC_MIXED, 0, (94, 245, 34), 2),
+    (PREC_MIXED, 0, (58, 91, 169), 2), (PREC_FP64, 0, (94, 245, 34), 2), (PREC_FP32, 0, (94, 245, 34), 3)])
+def test_prep_blocks_fit_one_round(stub, prec, obstacles, n, fit):
+    """A domain small enough for it has the phase prep's blocks on the 256 CUs all at
+    once: registers and LDS leave `fit` of them on each."""
+    p = make_params(n, lattice=27, twocomponent=True, densratio=True, internal_obstacles=obstacles, precision=prec)
+    d = hip.Domain(p)
+    d.init_state()
+    d.step(1)
+    tiles = -(-n[0] // 64) * -(-n[1] // 12)
+    assert tiles * -(-n[2] // stub.stub_prep_chunk()) <= 256 * fit
+    d.close()
