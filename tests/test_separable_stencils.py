@@ -187,3 +187,36 @@ def test_float32_at_least_as_accurate_as_reference_order():
         es = np.sqrt(np.mean((s_.astype(np.float64) - t)[band] ** 2))
         er = np.sqrt(np.mean((r_.astype(np.float64) - t)[band] ** 2))
         assert es <= 1.25 * er, (name, es, er)
+
+
+def _fma(a, b, c):
+    # the product of two float32 is exact in float64; one more rounding in the sum
+    return np.float32(np.float64(a) * np.float64(b) + np.float64(c))
+
+
+@pytest.mark.parametrize("off", [(0, 0), (1, 1), (-1, -1), (1, -1), (-1, 1)])
+def test_gradient_norm_in_fp32(off):
+    """grad_norm of lbf_common.h restated: from a reciprocal square root and a
+    reciprocal that are a unit in the last place off, either way, the root of the
+    squared gradient is the correctly rounded one (0.5 ulp, and the second-order
+    remainder of the correction: 1e-3) and 1 / (root + 1e-9) is within 1 ulp of the
+    float32 sum's (0.5 and the same), for |g| of 1e-16 to 1."""
+    f32 = np.float32
+    rng = np.random.default_rng(3)
+    g2 = (10.0 ** rng.uniform(-32, 0, 200000)).astype(f32)
+
+    def est(x, o):
+        r = x.astype(f32)
+        return r if o == 0 else np.nextafter(r, f32(np.inf if o > 0 else 0), dtype=f32)
+
+    y = est(1 / np.sqrt(np.maximum(g2, f32(1e-36)).astype(np.float64)), off[0])
+    s = g2 * y
+    mg = _fma(_fma(-s, s, g2), f32(0.5) * y, s)
+    d = mg + f32(1e-9)
+    i0 = est(1 / d.astype(np.float64), off[1])
+    im = _fma(i0, _fma(-i0, d, f32(1)), i0)
+    root, rec = np.sqrt(g2.astype(np.float64)), 1 / d.astype(np.float64)
+    assert np.abs((mg - root) / np.spacing(root.astype(f32))).max() < 0.501
+    assert np.abs((im - rec) / np.spacing(rec.astype(f32))).max() < 1.0
+    zero = f32(0)
+    assert _fma(_fma(-zero, zero, zero), f32(0.5) * f32(1e18), zero) == 0
