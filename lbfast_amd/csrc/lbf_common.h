@@ -258,8 +258,8 @@ __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
 // float64 on 2^20 gradients a decade, 1e-16 to 1: the root 0.29 ulp rms and 0.50 at
 // most, as the correctly rounded one; the reciprocal and the product n |g| 0.44 to
 // 0.59 and 0.52 to 0.70 ulp rms, at or below those of a plain rcp of that root (0.45
-// to 0.61, 0.53 to 0.72).  Below 1e-18, where n |g| is under 1e-9 g, the root is only
-// an upper bound's order (the squares leave the normal range); 0 gives 0.
+// to 0.61, 0.53 to 0.72).  Below 1e-18 the square leaves the normal range and the
+// root loses its digits, where n |g| is under 1e-9 of g; 0 gives 0.
 __device__ __forceinline__ void grad_norm(float g2, float& mg, float& im) {
   const float y = __builtin_amdgcn_rsqf(fmaxf(g2, 1.0e-36f)), s = g2 * y;
   mg = __builtin_fmaf(__builtin_fmaf(-s, s, g2), 0.5f * y, s);

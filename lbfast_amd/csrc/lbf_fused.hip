@@ -339,9 +339,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, int tile) {
   typedef typename C::T T;
   typedef typename Aux<PREC>::T TA;
   constexpr int NW = TY + 2;  // row waves (TY output rows + 2 halo rows)
-  constexpr int PB = prec_base(PREC);
-  // GI: grad phi and lap phi formed here from a phi tile (fused_grad_inline)
-  constexpr bool GI = (PB == PREC_FP32 || PB == PREC_FP16S || PB == PREC_BF16S) && TWO && INLINE && !OB;
+  // GI: grad phi and lap phi formed here from a phi tile
+  constexpr bool GI = TWO && INLINE && fused_grad_inline(PREC, OB);
   typedef Slots<PREC, TWO, INLINE, GI> SL;
   constexpr bool PF = fused_prefetch<PREC, TY>();
   // GI phi tile: rows y0-2 .. y0+TY+1 (tile row r holds y0-2+r), columns
@@ -1000,15 +999,23 @@ static hipError_t batch_std(const FusedBatchEntry* tab, int ndom, int total, int
              : batch_lat<PREC, TWO, TY, false>(tab, ndom, total, lat, ho, s);
 }
 
+template <int PREC, bool TWO>
+static hipError_t batch_ty(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool std, int ty, hipStream_t s) {
+  if constexpr (PREC == PREC_FP64 || PREC == PREC_MIXED) {
+    if (ty == 5) return batch_std<PREC, TWO, 5>(tab, ndom, total, lat, ho, std, s);
+  }
+  if (ty == 8) return batch_std<PREC, TWO, 8>(tab, ndom, total, lat, ho, std, s);
+  if (ty == 13) return batch_std<PREC, TWO, 13>(tab, ndom, total, lat, ho, std, s);
+  return hipErrorInvalidValue;
+}
+
 template <int PREC>
 hipError_t fused_batch_prec(const FusedBatchEntry* tab, int ndom, int total, int lat, bool ho, bool two, bool std, int ty,
                             hipStream_t s) {
-  if constexpr (PREC == PREC_FP64 || PREC == PREC_MIXED) {
-    if (ty == 5) return two ? batch_std<PREC, true, 5>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 5>(tab, ndom, total, lat, ho, std, s);
-  }
-  if (ty == 8) return two ? batch_std<PREC, true, 8>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 8>(tab, ndom, total, lat, ho, std, s);
-  if (ty == 13) return two ? batch_std<PREC, true, 13>(tab, ndom, total, lat, ho, std, s) : batch_std<PREC, false, 13>(tab, ndom, total, lat, ho, std, s);
-  return hipErrorInvalidValue;
+  if (!two) return batch_ty<PREC, false>(tab, ndom, total, lat, ho, std, ty, s);
+  // two components in FP64 are not batched (lbf_batch_create)
+  if constexpr (PREC != PREC_FP64) return batch_ty<PREC, true>(tab, ndom, total, lat, ho, std, ty, s);
+  else return hipErrorInvalidValue;
 }
 
 template <int PREC>

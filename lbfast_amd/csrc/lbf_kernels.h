@@ -68,13 +68,13 @@ struct StageArgs {
   double obc_val[6][4];
 };
 
-// The fused kernel forms grad phi and lap phi itself from phi (the prep
-// then stores only div theta) for the prefetching precisions without
-// internal obstacles: with obstacles, PHI_int_boundary rewrites phi on solid
-// nodes between the prep and the fused kernel, and the reference's gradients
-// are those of the phi before it.
-inline bool fused_grad_inline(int prec, const DevParams& dp) {
-  return (prec == PREC_FP32 || prec == PREC_FP16S || prec == PREC_BF16S) && dp.twocomp && !dp.obst;
+// Where the two-component fused kernel forms grad phi and lap phi itself from phi
+// and the prep stores only div theta (both sides follow this one rule): in 32-bit
+// arithmetic without internal obstacles.  With obstacles, PHI_int_boundary rewrites
+// phi on solid nodes between the prep and the fused kernel, and the reference's
+// gradients are those of the phi before it.
+constexpr bool fused_grad_inline(int prec, bool obst) {
+  return (prec_base(prec) == PREC_FP32 || prec_base(prec) == PREC_FP16S || prec_base(prec) == PREC_BF16S) && !obst;
 }
 
 // The switches of every two-component configuration as the reference's

@@ -163,8 +163,8 @@ __global__ void __launch_bounds__(BS) k_div(StageArgs a) {
 // With obstacles (OB) the node words of the tile's theta nodes stream in beside
 // phi: theta is 0 at non-fluid nodes (the reference never writes aux there and
 // reads the zero-initialised allocation).
-// MODE: PREP_DIV stores div theta only (the fused kernel forms grad phi and lap
-// phi itself, fused_grad_inline), PREP_ALL also grad phi and lap phi.
+// MODE: PREP_DIV stores div theta only (where fused_grad_inline() says that the
+// fused kernel forms grad phi and lap phi itself), PREP_ALL also those.
 //
 // What bounds it: instruction issue (it moves 8 bytes a node).  Two adjacent
 // rows a wave, the shared x passes, the running sums (no register moves of
@@ -1105,28 +1105,33 @@ static hipError_t prep_z(const StageArgs& a, int tz, hipStream_t s) {
   return hipGetLastError();
 }
 
+// what the fused kernel leaves to the prep
+template <int PREC, bool OB>
+constexpr int prep_mode() { return fused_grad_inline(PREC, OB) ? PREP_DIV : PREP_ALL; }
+
 template <int PREC>
 static hipError_t prep_t(const StageArgs& a, int tz, hipStream_t s) {
-  if (a.dp.obst) return prep_z<PREC, PREP_ALL, true>(a, tz, s);
-  // without obstacles the 32-bit fused kernels form their gradients themselves
-  constexpr int M = PREC == PREC_FP64 || PREC == PREC_MIXED ? PREP_ALL : PREP_DIV;
-  return prep_z<PREC, M, false>(a, tz, s);
+  if (a.dp.obst) return prep_z<PREC, prep_mode<PREC, true>(), true>(a, tz, s);
+  return prep_z<PREC, prep_mode<PREC, false>(), false>(a, tz, s);
+}
+
+template <int PREC>
+static hipError_t prep_batch(const PrepBatchEntry* tab, int ndom, int total, hipStream_t s) {
+  hipLaunchKernelGGL((k_phase_prep_z_batch<PREC, prep_mode<PREC, false>()>), dim3(total), dim3(QNT), 0, s, tab, ndom, total);
+  return hipGetLastError();
 }
 
 int prep_tile_count(const StageArgs& a, int tz) { return prep_tiles_z(a.dp, tz); }
 
 hipError_t launch_phase_prep_batch(const PrepBatchEntry* dev_tab, int ndom, int total_tiles, int prec, hipStream_t s) {
-  const dim3 grid(total_tiles), block(QNT);
-  // batches hold two-component domains without obstacles: div theta only
-  // exactly where fused_grad_inline() holds, i.e. for every precision but MIXED
+  // batches hold no obstacles, and two components not in FP64
   switch (prec) {
-    case PREC_FP32: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP32, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_MIXED: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_MIXED, PREP_ALL>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_FP16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_FP16S, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    case PREC_BF16S: hipLaunchKernelGGL((k_phase_prep_z_batch<PREC_BF16S, PREP_DIV>), grid, block, 0, s, dev_tab, ndom, total_tiles); break;
-    default: return hipErrorInvalidValue;
+    case PREC_FP32: return prep_batch<PREC_FP32>(dev_tab, ndom, total_tiles, s);
+    case PREC_MIXED: return prep_batch<PREC_MIXED>(dev_tab, ndom, total_tiles, s);
+    case PREC_FP16S: return prep_batch<PREC_FP16S>(dev_tab, ndom, total_tiles, s);
+    case PREC_BF16S: return prep_batch<PREC_BF16S>(dev_tab, ndom, total_tiles, s);
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_phase_prep(const StageArgs& a, int prec, int tz, hipStream_t s) {
