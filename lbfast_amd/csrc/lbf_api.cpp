@@ -284,8 +284,13 @@ static bool row_tile_ok(int prec, int ty) {
 }
 static const char* row_tile_text(int prec) { return wide_arith(prec) ? "5, 8 or 13" : "8 or 13"; }
 // The row tiles that a domain's default is chosen from, each with the time of a
-// block's plane (in units of one of them); of equal makespans the first.
-struct RowTile { int rows; double plane; };
+// block's plane (in units of one of them) and the planes that a block marches
+// beyond its chunk; of equal makespans the first.
+struct RowTile {
+  int rows;
+  double plane;
+  int extra = FUSED_EXTRA;
+};
 static std::vector<RowTile> row_choices(const lbf_ctx* c) {
   // 32 and 16 bits: a plane of 8 rows takes 0.72 of one of 13 (measured 0.66 at
   // 512^3, where HBM counts, to 0.81 at 64^3)
@@ -296,16 +301,19 @@ static std::vector<RowTile> row_choices(const lbf_ctx* c) {
   // MIXED 208 against 218; FP64 channel 128x96x96 106 against 159)
   if (c->p.twocomponent || c->p.internal_obstacles) return {{5, 1.0}};
   // One component: the other tiles do not prefetch, which costs most where the
-  // state does not stay in the 256 MB of memory-side cache.  A plane of 5 rows
-  // against one of 8: FP64 0.64-0.73 (D3Q19), 0.66-0.77 (D3Q27) in the cache and
-  // 0.49-0.58 beyond, MIXED 0.73-0.80 and 0.60-0.62.
-  const bool beyond = state_bytes(c) > ((size_t)256 << 20), d19 = c->p.lattice == 19;
-  const double t5 = c->prec == LBF_PREC_FP64 ? (beyond ? 0.52 : d19 ? 0.67 : 0.72) : (beyond ? 0.61 : 0.76);
+  // state does not stay in the 256 MB of memory-side cache.  The weight of a plane of
+  // 5 rows against one of 8 (and, with it, one plane more for the first transfers)
+  // chose, over 40 random sizes of 24 to 512 of each lattice and precision, within
+  // 0.6% of the fastest of 5, 8 and 13 rows on the mean, 6.2% at most; one weight of
+  // 0.72 for all had been 1.1 to 5.1% and up to 25% away.
+  const bool beyond = state_bytes(c) > ((size_t)256 << 20), f64 = c->prec == LBF_PREC_FP64, ho = c->dp.highorder != 0;
+  const double t5 = f64 ? (beyond ? 0.52 : ho ? 0.68 : 0.64) : (beyond ? 0.62 : ho ? 0.70 : 0.75);
+  const RowTile five = {5, t5, FUSED_EXTRA + 1};
   // D3Q19 does not spill with 13 rows: 1.37-1.5 (D3Q27 1.6 and more).  176x268x32
   // 56.7 us with 5 rows, 60.3 with 8, 52.4 with 13 (MIXED 54.9, 49.0, 42.7); 192^3
   // 226, 288, 270 (MIXED 182, 191, 178); 150x97x75 45.9, 50.4, 47.5
-  if (d19) return {{8, 1.0}, {5, t5}, {13, 1.4}};
-  return {{8, 1.0}, {5, t5}};
+  if (c->p.lattice == 19) return {{8, 1.0}, five, {13, 1.4}};
+  return {{8, 1.0}, five};
 }
 // Blocks of the phase prep on a CU: three of the 16/32-bit prep (measured plane
 // times 1.65, 2.2, 2.9 us with one to three); in 64-bit arithmetic its 118 to 124
@@ -327,7 +335,7 @@ static void default_tiles(lbf_ctx* c) {
   double best = 1e300;
   for (const RowTile& t : row_choices(c)) {
     int tz = 1;
-    const double cost = t.plane * pick_chunk(fused_xy(c->p, t.rows), c->p.nz, c->ncu, FUSED_EXTRA, T_FUSED, 1, &tz);
+    const double cost = t.plane * pick_chunk(fused_xy(c->p, t.rows), c->p.nz, c->ncu, t.extra, T_FUSED, 1, &tz);
     if (cost < best) {
       best = cost;
       c->ty = t.rows;
@@ -1168,7 +1176,7 @@ static void batch_default_tiles(lbf_batch* b) {
   if (wide_arith(b->prec) && !b->two) rows = {{8, 1.0}};
   for (const RowTile& t : rows) {
     int T = 1;
-    const double cost = t.plane * search(t.rows, FUSED_EXTRA, 1, &T);
+    const double cost = t.plane * search(t.rows, t.extra, 1, &T);
     if (cost < best) {
       best = cost;
       b->ty = t.rows;

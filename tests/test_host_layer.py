@@ -69,9 +69,10 @@ def test_failed_upload_of_isfluid_changes_nothing(stub):
     # one component in 64-bit arithmetic: the rows that were the fastest of 5, 8 and
     # 13, each with its best chunk (D3Q27 has 13 rows spill)
     ((176, 268, 32), PREC_FP64, 19, 13), ((50, 275, 85), PREC_FP64, 19, 13), ((100, 100, 100), PREC_FP64, 19, 5),
-    ((192, 192, 192), PREC_FP64, 19, 5), ((176, 268, 32), PREC_MIXED, 19, 13), ((64, 64, 64), PREC_MIXED, 19, 8),
+    ((192, 192, 192), PREC_FP64, 19, 5), ((64, 64, 64), PREC_FP64, 19, 8), ((36, 295, 114), PREC_FP64, 27, 8),
+    ((150, 97, 75), PREC_FP64, 27, 5), ((176, 268, 32), PREC_MIXED, 19, 13), ((64, 64, 64), PREC_MIXED, 19, 8),
     ((192, 192, 192), PREC_MIXED, 19, 13), ((192, 192, 192), PREC_FP64, 27, 5), ((176, 268, 32), PREC_MIXED, 27, 8),
-    ((192, 192, 192), PREC_MIXED, 27, 5)])
+    ((335, 50, 237), PREC_MIXED, 27, 5)])
 def test_rows_of_64_bit_domains(stub, n, prec, lattice, rows):
     p = make_params(n, lattice=lattice, highorder=lattice == 27, precision=prec)
     d = hip.Domain(p)
