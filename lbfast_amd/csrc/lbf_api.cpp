@@ -240,8 +240,13 @@ void lbf_destroy(lbf_ctx* c) {
 // makespan, counted in planes.  A block of tz planes marches tz + extra (halo
 // planes of the march and the prologue); t[k - 1] is a plane's time with k
 // blocks on every CU (nt at most), in units of t[0].  Chunks of ceil(nz / c)
-// planes; of equals the longest, which repeats fewest halo planes.
-static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t, int nt, int* tz_out) {
+// planes; of equals the longest, which repeats fewest halo planes.  cap bounds
+// turn_time() of the choice.
+static double turn_time(long blocks, int planes, int ncu, double makespan) {
+  return std::max(makespan / 3, (double)blocks * planes / ncu);
+}
+static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t, int nt, int* tz_out,
+                         double cap = 1e300) {
   double best = 1e300;
   int last = 0;
   for (int c = 1; c <= nz; ++c) {
@@ -252,7 +257,7 @@ static double pick_chunk(long tiles, int nz, int ncu, int extra, const double* t
     const long rest = n % slots;
     const double rounds = (double)(n / slots) * t[nt - 1] + (rest ? t[(rest + ncu - 1) / ncu - 1] : 0.0);
     const double cost = rounds * (tz + extra);
-    if (cost < best * 0.999) {
+    if (cost < best * 0.999 && turn_time(n, tz + extra, ncu, cost) <= cap) {
       best = cost;
       *tz_out = tz;
     }
@@ -315,6 +320,32 @@ static std::vector<RowTile> row_choices(const lbf_ctx* c) {
   if (c->p.lattice == 19) return {{8, 1.0}, five, {13, 1.4}};
   return {{8, 1.0}, five};
 }
+// Domains that step in turn on streams of their own share the CUs: with three of
+// them a step takes a third of the makespan or, the CUs full, all planes marched
+// over all CUs (turn_time), and short chunks march more halo planes.  Where the
+// kernels gained little over the time when chunks had 8 planes at least (some 1024
+// blocks), short chunks cost there what they gain alone, so the turn_time of a
+// one-component domain is bounded by that of such chunks and what the kernel gained
+// (64-bit D3Q19, the same loads as then, 6% to spare; 32 and 16 bits 15%).
+// 64-bit D3Q19, 60 random sizes up to 2 million nodes against those chunks: alone
+// 1.63x FP64, 1.42x MIXED, three in turn 1.20x and 1.19x, none slower in either;
+// unbounded 1.80x, 1.64x and 1.17x, 1.12x, but down to 0.87x in turn (30x49x295 FP64
+// 26.7 -> 30.8 us).  FP32 unbounded down to 0.96x in turn (37x50x228).  D3Q27 in 64
+// bits and two components gained more than short chunks can cost.
+static double fused_cap(const lbf_ctx* c) {
+  const lbf_params& p = c->p;
+  if (p.twocomponent || p.internal_obstacles || (wide_arith(c->prec) && p.lattice != 19)) return 1e300;
+  const long w8 = (long)((p.ny + 7) / 8) * 11, w13 = (long)((p.ny + 12) / 13) * 16;  // waves of the y extent
+  const int rows = w13 < w8 ? 13 : 8;
+  const long xy = fused_xy(p, rows), chunks = std::max(1L, (1024 + xy - 1) / xy);
+  const int tz = std::min(p.nz, std::max(8, (int)((p.nz + chunks - 1) / chunks)));
+  const long n = xy * ((p.nz + tz - 1) / tz);
+  const double makespan = (double)((n + c->ncu - 1) / c->ncu) * (tz + FUSED_EXTRA);
+  double cap = (wide_arith(c->prec) ? 1.06 : 1.15) * turn_time(n, tz + FUSED_EXTRA, c->ncu, makespan);
+  for (const RowTile& t : row_choices(c))
+    if (t.rows == rows) cap *= t.plane;
+  return cap;
+}
 // Blocks of the phase prep on a CU: three of the 16/32-bit prep (measured plane
 // times 1.65, 2.2, 2.9 us with one to three); in 64-bit arithmetic its 118 to 124
 // registers leave two, in FP64 with obstacles its 87 KB of LDS one.
@@ -333,9 +364,11 @@ static int prep_slots(const lbf_ctx* c, const double** t) {
 // 149 -> 113, 256^3 FP16S 435 -> 353, 160^3 FP64 678 -> 311.
 static void default_tiles(lbf_ctx* c) {
   double best = 1e300;
+  const double cap = fused_cap(c);
   for (const RowTile& t : row_choices(c)) {
     int tz = 1;
-    const double cost = t.plane * pick_chunk(fused_xy(c->p, t.rows), c->p.nz, c->ncu, t.extra, T_FUSED, 1, &tz);
+    const double cost =
+        t.plane * pick_chunk(fused_xy(c->p, t.rows), c->p.nz, c->ncu, t.extra, T_FUSED, 1, &tz, cap / t.plane);
     if (cost < best) {
       best = cost;
       c->ty = t.rows;

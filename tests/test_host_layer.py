@@ -98,3 +98,28 @@ def test_prep_blocks_fit_one_round(stub, prec, obstacles, n, fit):
     tiles = -(-n[0] // 64) * -(-n[1] // 12)
     assert tiles * -(-n[2] // stub.stub_prep_chunk()) <= 256 * fit
     d.close()
+
+
+@pytest.mark.parametrize("n,prec,lattice,before", [
+    # the tile before, and in turn with two others of its size: us a step with chunks
+    # of 8 planes at least, with it, and now
+    ((30, 49, 295), PREC_FP64, 19, (5, 12)),    # 26.7, 30.8
+    ((39, 275, 37), PREC_FP64, 19, (5, 10)),    # 20.3, 24.0, 20.3
+    ((156, 77, 56), PREC_FP64, 19, (8, 7)),     # 33.3, 36.0, 32.2
+    ((37, 50, 228), PREC_FP32, 19, (13, 4)),    # 15.2, 15.9
+    ((62, 325, 45), PREC_FP32, 27, (8, 8))])    # 22.7, 23.4
+def test_chunks_leave_room_for_domains_in_turn(stub, n, prec, lattice, before):
+    p = make_params(n, lattice=lattice, highorder=lattice == 27, precision=prec)
+    d = hip.Domain(p)
+    d.init_state()
+    d.step(1)
+    ty, tz = ctypes.c_int(), ctypes.c_int()
+    stub.stub_fused_tile(ctypes.byref(ty), ctypes.byref(tz))
+
+    # all planes that the blocks march, halo planes included, by the time of each
+    plane = {8: 0.72, 13: 1.0} if prec == PREC_FP32 else {5: 0.64, 8: 1.0, 13: 1.4}
+
+    def marched(rows, z):
+        return -(-n[0] // 64) * -(-n[1] // rows) * -(-n[2] // z) * plane[rows] * (z + (4 if rows == 5 else 3))
+    assert marched(ty.value, tz.value) < marched(*before)
+    d.close()
