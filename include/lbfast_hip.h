@@ -270,8 +270,10 @@ int32_t lbf_abi_version(void);
  * independent domains (initialised contexts sharing lattice, HIGHORDER,
  * precision and component count; any sizes and physical parameters; no
  * obstacles or REPULSIVE_FLUX) advance together: each step is one phase-field
- * launch and one fused launch whose grids cover every domain's tiles, so that
- * small domains fill the GPU.  The batch borrows the contexts (they must
+ * launch and one fused launch (two where only some of the domains have the usual
+ * switches: no SMAGORINSKI and, with two components, DENSRATIO, INTERFACE_INCOMP
+ * and no BUOYANCY_FORCING) whose grids cover every domain's tiles, so that small
+ * domains fill the GPU.  The batch borrows the contexts (they must
  * outlive it) and keeps their step counters and buffers current, so uploads,
  * downloads and single-domain calls stay valid between batch calls; work on
  * a context's stream is ordered before and after each batch step.  Two-
@@ -290,8 +292,8 @@ int lbf_batch_capture(lbf_batch* b, int32_t nsteps);
  * and phase-field kernels, for every domain (chunks clipped to each nz). */
 int lbf_batch_set_tile(lbf_batch* b, int32_t tile_y, int32_t tile_z, int32_t tile_z_prep);
 /* The table order: order[i] is the domain whose tiles come i-th in the
- * grid of every launch (each XCD takes a contiguous eighth of it); a
- * permutation of 0..ndomains-1.  Results do not depend on it. */
+ * grid of every launch that it is in (each XCD takes a contiguous eighth of
+ * it); a permutation of 0..ndomains-1.  Results do not depend on it. */
 int lbf_batch_set_order(lbf_batch* b, const int32_t* order);
 /* Time trial_steps (even) steps of each candidate on the batch itself, keep
  * the fastest and restore every domain's state.  Searched in turn: the tiles

@@ -54,10 +54,14 @@
 // vector instructions a launch), the 16-byte row transfers, the compiled-in
 // switches (std_switches), one buffer resource per set (scalar instructions
 // of the plane loop 661 -> 367) and streaming stores (stream_stores): two
-// components FP32 3.81 -> 3.18 ms (15.0 GB of compulsory state at 4.7 TB/s, the
-// rate of a plain copy), FP16S 3.15 -> 2.57 ms, one component 2.76 -> 2.20 ms.
+// components FP32 3.81 -> 3.18 ms (15.0 GB of compulsory state at 4.7 TB/s, as
+// much as a plain copy moves; 19 GB with the excess reads), FP16S 3.15 -> 2.57
+// ms, one component 2.76 -> 2.20 ms.
 // Registers decide the variants: a spill inside the plane loop makes the compiler
 // wait for every transfer in flight (FP16S 2.57 -> 3.70 ms, 32 bytes of spills).
+// One remains, in the general D3Q27 HIGHORDER two-component variant of 32 bits
+// with 13 rows: a column offset of the phi tile, reloaded in tiles at the x faces.
+// Forming it each plane instead was 1-3% slower (scalar spills 22 -> 29 and more).
 //
 // Periodicity: indices wrap in-kernel (the reference's intpbc halo copies,
 // mpi_module.f90:2820-2918).  isfluid and the solid neighbours of near-wall

@@ -3,7 +3,8 @@ step covers every domain's tiles.
 
 Every node's arithmetic is independent of the tiling, so a domain advanced in
 a batch must equal, bit for bit, the same domain advanced on its own (which
-the parity tests hold to the oracle).  Also checked: replays of a captured
+the parity tests hold to the oracle; the one exception, SMAGORINSKI with one
+component in 32-bit arithmetic, is in test_gpu_row_segments).  Also checked: replays of a captured
 graph, interleaved with eager work, equal eager steps; odd step counts keep
 the buffer bookkeeping; the autotuner leaves every domain's state as it was.
 """
